@@ -554,6 +554,87 @@ __device__ __forceinline__ void comp_full_lean(const ssc_component& c, double x,
   }
 }
 
+// One component's gradient and Hessian in four numbers, with q = (x, y, qz):
+//   grad = f q,   H = f diag(1, 1, w) + k q q^T.
+// Spherical components have qz = z, w = 1, f = phi'/r and k = (phi'' - phi'/r) / r^2; the
+// Miyamoto-Nagai disk has qz = z S / zeta, f = G m / D^3, k = -3 f / D^2 and
+// w = S b^2 / zeta^3 + z^2 / zeta^2.  The NFW k follows from its f without forming phi'':
+// phi'' - phi'/r = -3 f + G m / (r (r + r_s)^2).  Lean forms (see parts_mn).  A component is
+// thus passed between lanes or waves in 32 bytes, and spherical components add up in (f, k)
+// before the 3 x 3 terms are formed: about half the instructions of comp_full_lean per component.
+struct CompQuad {
+  double f, k, qz, w;
+};
+
+template <int K = -1>
+__device__ __forceinline__ CompQuad comp_quad(const ssc_component& c, double x, double y,
+                                              double z) {
+  const int kind = K >= 0 ? K : c.kind;
+  const double gm = c.p[0];
+  CompQuad q{0.0, 0.0, z, 1.0};
+  switch (kind) {
+    case SSC_COMP_MIYAMOTO_NAGAI: {
+      const double a = c.p[1], b2 = c.p[2] * c.p[2];
+      const double v = fma(z, z, b2);
+      const double iz = rsq(v);  // 1 / zeta
+      const double S = fma(v, iz, a);
+      const double iD = rsq(fma(x, x, fma(y, y, S * S)));
+      const double iD2 = iD * iD, iz2 = iz * iz;
+      q.f = gm * (iD2 * iD);
+      q.k = -3.0 * q.f * iD2;
+      q.qz = z * S * iz;
+      q.w = fma(S * b2, iz2 * iz, z * z * iz2);
+      break;
+    }
+    case SSC_COMP_NFW: {
+      const double rs = c.p[1];
+      const double r2 = fma(x, x, fma(y, y, z * z));
+      const double ir = rsq(r2);
+      const double r = r2 * ir, ir2 = ir * ir;
+      const double irp = recip(r + rs);
+      const double L = log1p_nonneg(r * recip(rs));
+      q.f = gm * ir2 * fma(L, ir, -irp);
+      q.k = ir2 * fma(-3.0, q.f, gm * ir * irp * irp);
+      break;
+    }
+    case SSC_COMP_HERNQUIST: {
+      const double r2 = fma(x, x, fma(y, y, fma(z, z, c.p[2])));
+      const double ir = rsq(r2);
+      const double irc = recip(fma(r2, ir, c.p[1]));
+      const double d1 = gm * irc * irc;
+      q.f = d1 * ir;
+      q.k = -(ir * ir) * fma(2.0 * d1, irc, q.f);
+      break;
+    }
+    case SSC_COMP_PLUMMER: {
+      const double rs = c.p[1];
+      const double is = rsq(fma(x, x, fma(y, y, fma(z, z, rs * rs))));
+      const double is2 = is * is;
+      q.f = gm * (is2 * is);
+      q.k = -3.0 * q.f * is2;
+      break;
+    }
+    default:
+      break;
+  }
+  return q;
+}
+
+// Accumulate one component's gradient g[3] and Hessian upper triangle H[0, 1, 2, 4, 5, 8].
+__device__ __forceinline__ void quad_add(const CompQuad& q, double x, double y, double* g,
+                                         double* H) {
+  const double kx = q.k * x, ky = q.k * y, kz = q.k * q.qz;
+  g[0] = fma(q.f, x, g[0]);
+  g[1] = fma(q.f, y, g[1]);
+  g[2] = fma(q.f, q.qz, g[2]);
+  H[0] += fma(kx, x, q.f);
+  H[1] = fma(kx, y, H[1]);
+  H[2] = fma(kx, q.qz, H[2]);
+  H[4] += fma(ky, y, q.f);
+  H[5] = fma(ky, q.qz, H[5]);
+  H[8] += fma(kz, q.qz, q.f * q.w);
+}
+
 // comp_full with the component's kind fixed at compile time (K >= 0: the kind switch folds
 // away; K < 0: the kind is read from c as in comp_full); LEAN selects comp_full_lean.
 template <int K, bool LEAN = false>

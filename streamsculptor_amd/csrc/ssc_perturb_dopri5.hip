@@ -13,13 +13,19 @@
 // end-of-interval clipping, quartic dense output at save times).
 //
 // Layout: a particle is spread over a group of L lanes (a power of two, 8 <= L <= 256); lane l
-// owns the response vectors l, l + L, ... (G = 1, 2 or 4 of them) and, for l < 6, base
-// component l.  At each
-// stage the six base owners publish the stage row through LDS, lane c of the group forms host
-// component c's gradient and Hessian there and publishes them, and every lane sums the
-// components, so the base orbit and the host terms are formed once per group.  The stage values
-// and the error norm are block-synchronous: every lane of the block passes the same barriers,
-// and a group whose particle has finished idles until the block's last particle is done.
+// owns the response vectors l, l + L, ... (G = 1, 2 or 4 of them).  Every wave of a group carries
+// the base row on its own first six lanes (the copies stay equal bit for bit), so the stage row
+// reaches the wave's lanes without a barrier.  The host terms are the long serial chain of a
+// stage: a group of several waves deals the host components out to its waves, each wave's
+// component fixed, so that the kinds of code run side by side, and they meet in LDS after one
+// barrier (two buffers); a group of up to one wave forms all components in every lane and its
+// loop holds no barrier at all, so the waves of a block run on their own.  (Lanes of one wave
+// forming components of different kinds ran the kinds one after the other, their parameters
+// fetched through vector memory at every stage, between two barriers.)  What bounds a step now is
+// instruction latency: about 1,800 vector and 560 scalar instructions a wave and step, two waves
+// a SIMD in 256 registers.  One particle with 256 response vectors: 16.4 -> 8.2 us a step; 1,000
+// of them, their responses to 128 Hernquist subhalos with the radius block over 1,500 Myr on
+// average at rtol = atol = 1e-8: 29 -> 14.6 ms.
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -40,13 +46,18 @@ constexpr int PD_MIN_L = 8;
 constexpr int PD_GROUPS = PD_BLOCK / PD_MIN_L;
 constexpr int PD_WAVES = PD_BLOCK / 64;
 
-// Sum of v over the L lanes of a particle group, bit-identical in every lane of the group: the
-// butterfly forms each pairwise sum from the same two operands in both partner lanes; groups
-// wider than a wave add their wave partials in wave order through LDS (one barrier, taken when
-// L > 64, which is uniform over the launch).
-__device__ __forceinline__ double group_sum(double v, int L, double* part) {
-  const int w = L < 64 ? L : 64;
-  for (int o = w >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, w);
+// Sum of v over the L lanes of a particle group, bit-identical in every lane of the group:
+// within a wave each pairwise sum has the same two operands in both partner lanes (data-parallel
+// moves and lane swaps, no trip through the LDS unit); groups wider than a wave add their wave
+// partials in wave order through LDS (one barrier, taken when L > 64, which is uniform over the
+// launch).  Every lane of the wave must be active.
+__device__ __forceinline__ double part_sum(double v, int L, double* part) {
+  switch (L) {
+    case 8: return group_sum<8>(v);
+    case 16: return group_sum<16>(v);
+    case 32: return group_sum<32>(v);
+    default: v = group_sum<64>(v);
+  }
   if (L <= 64) return v;
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -90,7 +101,7 @@ __device__ __forceinline__ double err_of(double y, const double (&k)[7], double 
                                          const Dp5Ctl& ctl) {
   const double err =
       h * (E1 * k[0] + E3 * k[2] + E4 * k[3] + E5 * k[4] + E6 * k[5] + E7 * k[6]);
-  const double u = err / (ctl.atol + ctl.rtol * fmax(fabs(y), fabs(yn)));
+  const double u = err * recip(ctl.atol + ctl.rtol * fmax(fabs(y), fabs(yn)));
   return u * u;
 }
 
@@ -173,9 +184,14 @@ __device__ __forceinline__ double pos_sum(double x0, double v0, const double (&k
   }
 }
 
-// One response vector per lane fits two waves per SIMD with a few spilled registers (1.5x
-// faster than one wave per SIMD without spills); two vectors per lane need one wave per SIMD,
-// four (513 to 1024 vectors) spill about a hundred registers at one wave per SIMD.
+// Lane src's value in every lane of a group part of w <= 64 lanes (src uniform over the launch).
+__device__ __forceinline__ double part_bcast(double v, int src, int w) {
+  if (w == 64)
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), src),
+                            __builtin_amdgcn_readlane(__double2loint(v), src));
+  return __shfl(v, src, w);
+}
+
 template <int SK, int RAD, int G>
 __global__ __launch_bounds__(PD_BLOCK) __attribute__((amdgpu_waves_per_eu(G == 1 ? 2 : 1,
                                                                           G == 1 ? 2 : 1)))
@@ -186,10 +202,12 @@ void perturb_dopri5_kernel(
     double* __restrict__ w_out, double* __restrict__ dw_out, double* __restrict__ ys,
     double* __restrict__ dys, int32_t* __restrict__ stats) {
   extern __shared__ __align__(16) char lds_raw[];
-  __shared__ double xv_sh[PD_GROUPS][2][6];
   __shared__ double part_sh[2][PD_WAVES];
-  __shared__ double hg_sh[PD_GROUPS][SSC_MAX_COMPONENTS][9];  // host component partials
+  __shared__ __align__(16) CompQuad hg_sh[2][PD_WAVES / 2][SSC_MAX_COMPONENTS];  // wide groups
   constexpr int DD = RAD ? 12 : 6;
+  constexpr bool HQ = SK == SSC_SRC_LINE_HERNQUIST;
+  if (threadIdx.x < 2 * (PD_WAVES / 2) * SSC_MAX_COMPONENTS)
+    (&hg_sh[0][0][0])[threadIdx.x] = CompQuad{0.0, 0.0, 0.0, 0.0};
   SourceLDS<SK> lds;
   lds.init(pert, lds_raw);  // barrier inside
 
@@ -199,10 +217,17 @@ void perturb_dopri5_kernel(
   const int gi = threadIdx.x / L, lane = threadIdx.x - gi * L;
   const int64_t i = (int64_t)blockIdx.x * ppb + gi;
   const bool valid = i < n;
-  const int bc = lane < 6 ? lane : -1;  // owned base component
+  const bool wide = L > 64;                          // several waves per particle
+  const int WL = wide ? 64 : L;                      // lanes of the group in one wave
+  const int nw = wide ? L >> 6 : 1;
+  const int wi = __builtin_amdgcn_readfirstlane(wide ? lane >> 6 : 0);  // wave of the group
+  const int wl = lane & (WL - 1);
+  const int bc = wl < 6 ? wl : -1;                   // carried base component
+  const bool bw = lane < 6;                          // the copy that counts and is written
 
   bool vh[G];  // vector present
   int vj[G], voff[G];
+  double rad_a[G];  // Plummer radius block: the scale radius
 #pragma unroll
   for (int q = 0; q < G; ++q) {
     const int v = lane + q * L;
@@ -210,6 +235,7 @@ void perturb_dopri5_kernel(
     const bool rad = RAD && v >= m;
     vj[q] = vh[q] ? (rad ? v - m : v) : 0;
     voff[q] = rad ? 6 : 0;
+    rad_a[q] = RAD && !HQ ? pert.rs[vj[q]] : 0.0;
   }
 
   const double ta = valid ? (t_start ? t_start[i] : t0) : t1;
@@ -239,7 +265,7 @@ void perturb_dopri5_kernel(
   // saves at or before the start
   auto save_row = [&](int js, bool interp, double s, double h) {
     const int64_t row = (int64_t)i * nts + js;
-    if (bc >= 0)
+    if (bw)
       ys[row * 6 + bc] = interp ? dense_at(by, bk, byn, h, s) : by;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
@@ -261,7 +287,7 @@ void perturb_dopri5_kernel(
   };
   auto fill_row = [&](int js, double val) {
     const int64_t row = (int64_t)i * nts + js;
-    if (bc >= 0) ys[row * 6 + bc] = val;
+    if (bw) ys[row * 6 + bc] = val;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
       if (!vh[q]) continue;
@@ -277,84 +303,94 @@ void perturb_dopri5_kernel(
   }
 
   bool live = valid && tau0 < tau1;
-  int xb = 0, pb = 0;
+  int hb = 0, pb = 0;
+  const int nc = hp.n_components;
+  const ssc_component mine = hp.c[wi < nc ? wi : 0];  // this wave's host component (wide groups)
 
-  // Stage S at tau_s = tau + c_S h: publish the base stage value; lane c < n_components of the
-  // group forms host component c's gradient and Hessian at the stage position and publishes
-  // them; every lane sums the components in order, then forms its slopes.  Two barriers.
+  // Stage S at tau_s = tau + c_S h.  A wave whose particles have all finished only keeps the
+  // barriers of a wide block; lanes of finished particles of a live wave compute unused values
+  // (their slopes are not read again).
   auto stage = [&](auto S_, double tau, double h) {
     constexpr int S = decltype(S_)::value;
     constexpr int O = stage_out<S>();
     const double bval = stage_in<S>(by, bk, h);
-    if (live && bc >= 0) xv_sh[gi][xb][bc] = bval;
     if (S == 6) byn = bval;
-    __syncthreads();
-    const double* xv = xv_sh[gi][xb];
-    if (live && lane < hp.n_components) {
-      double phi = 0.0, gc[3] = {0.0, 0.0, 0.0}, Hc[9];
+    double xv[6];
 #pragma unroll
-      for (int r = 0; r < 9; ++r) Hc[r] = 0.0;
-      comp_full(hp.c[lane], xv[0], xv[1], xv[2], phi, gc, Hc);
-      double* o = hg_sh[gi][lane];
-      o[0] = gc[0]; o[1] = gc[1]; o[2] = gc[2];
-      o[3] = Hc[0]; o[4] = Hc[1]; o[5] = Hc[2]; o[6] = Hc[4]; o[7] = Hc[5]; o[8] = Hc[8];
-    }
-    __syncthreads();
-    if (live) {
-      const double px = xv[0], py = xv[1], pz = xv[2];
-      double g[3] = {0.0, 0.0, 0.0}, H[9];
+    for (int c = 0; c < 6; ++c) xv[c] = part_bcast(bval, c, WL);
+    double g[3] = {0.0, 0.0, 0.0}, H[9];
 #pragma unroll
-      for (int r = 0; r < 9; ++r) H[r] = 0.0;
-      for (int c = 0; c < hp.n_components; ++c) {
-        const double* o = hg_sh[gi][c];
-        g[0] += o[0]; g[1] += o[1]; g[2] += o[2];
-        H[0] += o[3]; H[1] += o[4]; H[2] += o[5]; H[4] += o[6]; H[5] += o[7]; H[8] += o[8];
+    for (int r = 0; r < 9; ++r) H[r] = 0.0;
+    if (wide) {
+      if (wi < nc) {
+        const CompQuad cq = comp_quad(mine, xv[0], xv[1], xv[2]);
+        if (wl == 0) hg_sh[hb][gi][wi] = cq;
       }
-      H[3] = H[1]; H[6] = H[2]; H[7] = H[5];
-      if (bc >= 0) bk[O] = bc < 3 ? dir * xv[3 + bc] : -dir * g[bc - 3];
-      const double t = dir * (tau + stage_c<S>() * h);
-#pragma unroll
-      for (int q = 0; q < G; ++q) {
-        double yt[6];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-          yt[c] = pos_sum<S>(y[q][c], y[q][3 + c], kv[q][c], h, dir);
-          yt[3 + c] = stage_in<S>(y[q][3 + c], kv[q][c], h);
-        }
-        if (S == 6)
-#pragma unroll
-          for (int c = 0; c < 6; ++c) yn[q][c] = yt[c];
-        double fx = 0.0, fy = 0.0, fz = 0.0;
-        double sx, sy, sz, gm, qs;
-        if (vh[q] && lds.get(0, t, vj[q], sx, sy, sz, gm, qs)) {
-          const double ex = px - sx, ey = py - sy, ez = pz - sz;
-          double f, fr;  // grad Phi_j = f e; grad(dPhi_j/da_j) = fr e
-          if (SK == SSC_SRC_LINE_HERNQUIST) {  // qs = a
-            const double r2 = fma(ex, ex, fma(ey, ey, ez * ez));
-            const double ir = rsq(r2);
-            const double ia = 1.0 / fma(r2, ir, qs);
-            f = gm * ir * ia * ia;
-            fr = -2.0 * f * ia;
-          } else {  // qs = a^2
-            const double is = rsq(fma(ex, ex, fma(ey, ey, fma(ez, ez, qs))));
-            f = gm * is * is * is;
-            fr = -3.0 * f * sqrt(qs) * is * is;
-          }
-          const double ff = voff[q] ? fr : f;
-          fx = ff * ex; fy = ff * ey; fz = ff * ez;
-        }
-        const double hx = H[0] * yt[0] + H[1] * yt[1] + H[2] * yt[2];
-        const double hy = H[3] * yt[0] + H[4] * yt[1] + H[5] * yt[2];
-        const double hz = H[6] * yt[0] + H[7] * yt[1] + H[8] * yt[2];
-        kv[q][0][O] = -dir * (fx + hx);
-        kv[q][1][O] = -dir * (fy + hy);
-        kv[q][2][O] = -dir * (fz + hz);
+      for (int c = wi + nw; c < nc; c += nw) {  // a host of more components than waves
+        const CompQuad cq = comp_quad(hp.c[c], xv[0], xv[1], xv[2]);
+        if (wl == 0) hg_sh[hb][gi][c] = cq;
       }
+      __syncthreads();
+      // the first three slots in one batch of reads (empty ones hold zeros; a loop with one LDS
+      // round trip per component: 8.8 against 8.2 us a step)
+      CompQuad cq[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) cq[c] = hg_sh[hb][gi][c];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) quad_add(cq[c], xv[0], xv[1], g, H);
+      for (int c = 3; c < nc; ++c) quad_add(hg_sh[hb][gi][c], xv[0], xv[1], g, H);
+      hb ^= 1;
+    } else {
+      for (int c = 0; c < nc; ++c)
+        quad_add(comp_quad(hp.c[c], xv[0], xv[1], xv[2]), xv[0], xv[1], g, H);
     }
-    xb ^= 1;
+    H[3] = H[1]; H[6] = H[2]; H[7] = H[5];
+    if (bc >= 0) {
+      const double gb = bc == 3 ? g[0] : (bc == 4 ? g[1] : g[2]);
+      const double vb = bc == 0 ? xv[3] : (bc == 1 ? xv[4] : xv[5]);
+      bk[O] = bc < 3 ? dir * vb : -dir * gb;
+    }
+    const double t = dir * (tau + stage_c<S>() * h);
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      double yt[6];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        yt[c] = pos_sum<S>(y[q][c], y[q][3 + c], kv[q][c], h, dir);
+        yt[3 + c] = stage_in<S>(y[q][3 + c], kv[q][c], h);
+      }
+      if (S == 6)
+#pragma unroll
+        for (int c = 0; c < 6; ++c) yn[q][c] = yt[c];
+      double sx, sy, sz, gm, qs;
+      const bool act = lds.get(0, t, vj[q], sx, sy, sz, gm, qs);
+      const double ex = xv[0] - sx, ey = xv[1] - sy, ez = xv[2] - sz;
+      double f, fr;  // grad Phi_j = f e; grad(dPhi_j/da_j) = fr e
+      if (HQ) {      // qs = a
+        const double r2 = fma(ex, ex, fma(ey, ey, ez * ez));
+        const double ir = rsq(r2);
+        const double ia = recip(fma(r2, ir, qs));
+        f = gm * ir * ia * ia;
+        fr = -2.0 * f * ia;
+      } else {  // qs = a^2
+        const double is = rsq(fma(ex, ex, fma(ey, ey, fma(ez, ez, qs))));
+        f = gm * is * is * is;
+        fr = -3.0 * f * rad_a[q] * is * is;
+      }
+      // an inactive source contributes nothing whatever its position
+      const double ff = vh[q] && act ? (voff[q] ? fr : f) : 0.0;
+      const bool on = vh[q] && act;
+      const double fx = on ? ff * ex : 0.0, fy = on ? ff * ey : 0.0, fz = on ? ff * ez : 0.0;
+      const double hx = H[0] * yt[0] + H[1] * yt[1] + H[2] * yt[2];
+      const double hy = H[3] * yt[0] + H[4] * yt[1] + H[5] * yt[2];
+      const double hz = H[6] * yt[0] + H[7] * yt[1] + H[8] * yt[2];
+      kv[q][0][O] = -dir * (fx + hx);
+      kv[q][1][O] = -dir * (fy + hy);
+      kv[q][2][O] = -dir * (fz + hz);
+    }
   };
   auto reduce = [&](double v) {
-    const double s = group_sum(v, L, part_sh[pb]);
+    const double s = part_sum(v, L, part_sh[pb]);
     pb ^= 1;
     return s;
   };
@@ -368,7 +404,7 @@ void perturb_dopri5_kernel(
     // starting step (Hairer, Norsett & Wanner, Solving ODEs I, sec. II.4) on the whole state
     double s0 = 0.0, s1 = 0.0;
     if (live) {
-      if (bc >= 0) {
+      if (bw) {
         const double sc = ctl.atol + fabs(by) * ctl.rtol;
         s0 = (by / sc) * (by / sc);
         s1 = (bk[0] / sc) * (bk[0] / sc);
@@ -393,7 +429,7 @@ void perturb_dopri5_kernel(
       stage(std::integral_constant<int, 7>{}, tau0, h0);  // f(tau0 + h0, y + h0 f0) -> slot 1
       double s2 = 0.0;
       if (live) {
-        if (bc >= 0) {
+        if (bw) {
           const double sc = ctl.atol + fabs(by) * ctl.rtol;
           const double u = (bk[1] - bk[0]) / sc;
           s2 = u * u;
@@ -427,7 +463,15 @@ void perturb_dopri5_kernel(
     if (tnext > tau1) tnext = tau1;
   }
 
-  while (__syncthreads_or(live ? 1 : 0)) {
+  // The loop ends for a wave when its particles have finished, or with the block where groups
+  // of several waves share its barriers; with one group per block every wave forms the same
+  // `live`.
+  auto more = [&]() -> bool {
+    if (L == PD_BLOCK) return __builtin_amdgcn_readfirstlane(live ? 1 : 0) != 0;
+    if (wide) return __syncthreads_or(live ? 1 : 0) != 0;
+    return __any(live ? 1 : 0) != 0;
+  };
+  while (more()) {
     const double h = tnext - tprev;
     stage(std::integral_constant<int, 1>{}, tprev, h);
     stage(std::integral_constant<int, 2>{}, tprev, h);
@@ -437,7 +481,7 @@ void perturb_dopri5_kernel(
     stage(std::integral_constant<int, 6>{}, tprev, h);
     double ss = 0.0;
     if (live) {
-      if (bc >= 0) ss = err_of(by, bk, byn, h, ctl);
+      if (bw) ss = err_of(by, bk, byn, h, ctl);
 #pragma unroll
       for (int q = 0; q < G; ++q)
         if (vh[q])
@@ -445,15 +489,15 @@ void perturb_dopri5_kernel(
           for (int c = 0; c < 3; ++c) {
             ss += err_of(y[q][3 + c], kv[q][c], yn[q][3 + c], h, ctl);
             const double ex = dir * h * (h * qsum<8, 5>(kv[q][c]));
-            const double u = ex / (ctl.atol + ctl.rtol * fmax(fabs(y[q][c]), fabs(yn[q][c])));
+            const double u =
+                ex * recip(ctl.atol + ctl.rtol * fmax(fabs(y[q][c]), fabs(yn[q][c])));
             ss = fma(u, u, ss);
           }
     }
     const double e = sqrt(reduce(ss) / ntot);
     if (live) {
       const bool keep = (e < 1.0) || at_dtmin;
-      double factor = 0.9 * pow(1.0 / e, 0.2);
-      factor = fmin(fmax(factor, keep ? 1.0 : 0.2), 10.0);
+      const double factor = fmin(fmax(step_factor(e), keep ? 1.0 : 0.2), 10.0);
       double dtn = h * factor;
       if (ctl.dtmax > 0.0 && dtn > ctl.dtmax) dtn = ctl.dtmax;
       if (ctl.dtmin > 0.0) {
@@ -466,7 +510,7 @@ void perturb_dopri5_kernel(
           const double tj = dir * ts[js];
           if (tj == tnext) {
             const int64_t row = (int64_t)i * nts + js;
-            if (bc >= 0) ys[row * 6 + bc] = byn;
+            if (bw) ys[row * 6 + bc] = byn;
 #pragma unroll
             for (int q = 0; q < G; ++q) {
               if (!vh[q]) continue;
@@ -511,7 +555,7 @@ void perturb_dopri5_kernel(
   if (failed) {
     const double inf = __builtin_inf();
     for (int j = 0; j < nts; ++j) fill_row(j, inf);
-    if (bc >= 0 && w_out) w_out[6 * i + bc] = inf;
+    if (bw && w_out) w_out[6 * i + bc] = inf;
 #pragma unroll
     for (int q = 0; q < G; ++q) {
       if (!vh[q] || !dw_out) continue;
@@ -522,7 +566,7 @@ void perturb_dopri5_kernel(
     return;
   }
   for (; js < nts; ++js) fill_row(js, __builtin_nan(""));
-  if (bc >= 0 && w_out) w_out[6 * i + bc] = by;
+  if (bw && w_out) w_out[6 * i + bc] = by;
 #pragma unroll
   for (int q = 0; q < G; ++q) {
     if (!vh[q] || !dw_out) continue;
