@@ -82,6 +82,10 @@ struct GroupSources {
   }
 };
 
+// Every operation keeps its correctly rounded value (div_rn, sqrt_rn where the library would
+// expand an IEEE division or square root): the step-size controller turns a last-bit change of a
+// force into another, equally valid step sequence, and rows that differ by up to the truncation
+// error.
 // dy/dtau at tau (t = dir * tau) for the orbit ODE [v, -grad Phi].
 template <int SK, bool GR, int HS>
 __device__ __forceinline__ void rhs(const ssc_host_potential& hp, const SourceLDS<SK>& lds,
@@ -169,6 +173,10 @@ __global__ __launch_bounds__(DP_BLOCK) void dopri5_kernel(
   for (; js < nts && dir * tsi[js] == tau0; ++js)
 #pragma unroll
     for (int c = 0; c < 6; ++c) yrow[6 * js + c] = y[c];
+  // the next two save times are kept in registers, so that neither a step nor a saved row waits
+  // for one to arrive from memory
+  auto save_time = [&](int j) { return j < nts ? dir * tsi[j] : __builtin_inf(); };
+  double tsave = save_time(js), tsave2 = save_time(js + 1);
 
   int nacc = 0, nrej = 0, nsteps = 0;
   double tprev = tau0;
@@ -239,7 +247,8 @@ __global__ __launch_bounds__(DP_BLOCK) void dopri5_kernel(
       for (int c = 0; c < 6; ++c) {
         const double err = h * (E1 * f0[c] + E3 * k3[c] + E4 * k4[c] + E5 * k5[c] + E6 * k6[c] +
                                 E7 * k7[c]);
-        u[c] = err / (ctl.atol + ctl.rtol * fmax(fabs(y[c]), fabs(yn[c])));
+        const double scale = ctl.atol + ctl.rtol * fmax(fabs(y[c]), fabs(yn[c]));
+        u[c] = div_rn(err, scale);
       }
       const double e = rms6(u);
       const bool keep = (e < 1.0) || at_dtmin;
@@ -265,7 +274,7 @@ __global__ __launch_bounds__(DP_BLOCK) void dopri5_kernel(
         }
       }
       if (keep) {
-        if (yrow && js < nts && dir * tsi[js] <= tnext) {
+        if (js < nts && tsave <= tnext) {
           // dense output on (tprev, tnext]
           double F0[6], a4[6], b3[6], c2[6];
 #pragma unroll
@@ -279,13 +288,15 @@ __global__ __launch_bounds__(DP_BLOCK) void dopri5_kernel(
             b3[c] = D2 - 2.0 * D1 - 2.0 * a4[c];
             c2[c] = D1 - a4[c] - b3[c];
           }
-          for (; js < nts && dir * tsi[js] <= tnext; ++js) {
-            const double tj = dir * tsi[js];
+          for (; js < nts && tsave <= tnext; ++js) {
+            const double tj = tsave;
+            tsave = tsave2;
+            tsave2 = save_time(js + 2);
             if (tj == tnext) {
 #pragma unroll
               for (int c = 0; c < 6; ++c) yrow[6 * js + c] = yn[c];
             } else {
-              const double s = (tj - tprev) / h;
+              const double s = div_rn(tj - tprev, h);
 #pragma unroll
               for (int c = 0; c < 6; ++c)
                 yrow[6 * js + c] = y[c] + s * (F0[c] + s * (c2[c] + s * (b3[c] + s * a4[c])));
