@@ -7,8 +7,8 @@
 // on the fp32 VALU (BF16-rounded weights, fp32 inputs) so the input coordinates keep fp32
 // resolution.
 //
-// Training path: batch-major activations, generic strided GEMM C = A . B (64x64 block tile,
-// four 32x32 wave tiles, split-K for the batch reductions of the weight gradients).
+// Training path: 64x64 block tiles of four 32x32 wave tiles, split-K for the batch reductions of
+// the weight gradients, several jobs per launch.
 // Inference path: weights pre-packed in MFMA fragment order; a wave evaluates 16 points per
 // tile with the activations kept in registers between layers (points on the MFMA N axis).
 #include <hip/hip_runtime.h>
@@ -24,274 +24,250 @@ namespace ssc {
 namespace mlp {
 
 // ------------------------------------------------------------------------------------------
-// generic GEMM: Cz[m][n] = sum_{k in chunk z} A(m,k) B(k,n) (+ bias[n] when bias != NULL)
-// A(m,k) = A[m*sAm + k*sAk], B(k,n) = B[k*sBk + n*sBn]  (BF16 bits)
+// Training kernels.  A minibatch's matrix products are small (8192 x 256 x 256: 1 GFLOP, 12 MB),
+// so an iteration is bound by launches, load latency and how many blocks each launch has.  One
+// launch therefore carries every job whose inputs are ready (JobList: products, column sums and
+// reductions side by side, a block range each); a product's epilogue applies the activation or
+// its derivative; and a product's tile loads its whole K range (up to TK) into LDS with every
+// load in flight at once.  Operands are kept K-contiguous for all products: activations and
+// their gradients are written in both orders by the epilogue that forms them.  Every sum keeps
+// its order (K ascending in steps of 16 within a tile, the split-K chunks, the column sums), so
+// a training run gives the same network bit for bit.  An iteration of 8,192 points (loss,
+// gradients, Adam): 31 launches and 281 us with a kernel per step and a 32-wide K stage, 11
+// launches and 131 us now; of it 21 us per backward launch (its 20 MB would take 5), 12 us per
+// forward product, 14 us the first layer's gradient (chains of 128 additions, the order's price).
+//
+// A product: C(m, n) = sum_k A(m, k) B(n, k), A(m, k) = a[m * sa + k * ka] and B likewise, in
+// 64 x 64 tiles by four waves of 32 x 32; K split into chunks of kchunk.
 // ------------------------------------------------------------------------------------------
-constexpr int GT = 64;   // block tile
-constexpr int GK = 32;   // k per LDS stage
-constexpr int GPAD = 40; // LDS row pitch (elements): 80 B keeps 16-byte fragment reads aligned
+constexpr int GT = 64;     // block tile
+constexpr int GK = 32;     // granularity of the split-K chunks
+constexpr int TK = 256;    // k's staged at once
+constexpr int TPAD = 264;  // LDS row pitch (elements): 16-byte fragments, rows 4 banks apart
+constexpr int CS_ROWS = 512;  // batch rows per partial of the column sums
 
-// Operand layouts of the tile loader.  GL_K: k contiguous (stride 1 in k, row stride a multiple
-// of 8, 16-byte aligned base): a thread moves 8 k's of one row with one 16-byte load and one
-// 16-byte LDS store.  GL_R: rows contiguous (stride 1 in m or n, k stride a multiple of 8,
-// aligned base): a thread loads 8 rows of one k with one 16-byte load and stores them across
-// the 8 LDS rows.  GL_ANY: element loads at any strides.  Every layout leaves the same values
-// (zeros past the edges) in LDS, so the products do not depend on the choice.
-enum { GL_ANY = 0, GL_K = 1, GL_R = 2 };
-
-// One operand's 64 x 32 stage of the tile in registers: 8 BF16 values per thread.
-template <int L>
-struct TileLoad {
-  uint4 v;
-  // X(r, k) = X[r * sr + k * sk]; rows r0 .. r0 + 63 of R, k's k0 .. k0 + 31 of [.., ke)
-  __device__ void load(const uint16_t* __restrict__ X, int64_t sr, int64_t sk, int r0, int R,
-                       int k0, int ke, int t) {
-    uint16_t e8[8];
-    if (L == GL_K) {
-      const int r = r0 + (t >> 2), k = k0 + (t & 3) * 8;
-      if (r < R && k + 8 <= ke) {
-        v = *reinterpret_cast<const uint4*>(X + (int64_t)r * sr + k);
-        return;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        e8[e] = (r < R && k + e < ke) ? X[(int64_t)r * sr + (k + e)] : (uint16_t)0;
-    } else if (L == GL_R) {
-      const int k = k0 + (t >> 3), r = r0 + (t & 7) * 8;
-      if (k < ke && r + 8 <= R) {
-        v = *reinterpret_cast<const uint4*>(X + (int64_t)k * sk + r);
-        return;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        e8[e] = (k < ke && r + e < R) ? X[(int64_t)k * sk + (r + e)] : (uint16_t)0;
-    } else {
-      const int r = r0 + (t >> 2), k = k0 + (t & 3) * 8;
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        e8[e] = (r < R && k + e < ke) ? X[(int64_t)r * sr + (int64_t)(k + e) * sk] : (uint16_t)0;
-    }
-    memcpy(&v, e8, 16);
-  }
-  __device__ void store(uint16_t (*Xs)[GPAD], int t) const {
-    if (L == GL_R) {
-      const int kk = t >> 3, rr = (t & 7) * 8;
-      uint16_t e8[8];
-      memcpy(e8, &v, 16);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) Xs[rr + e][kk] = e8[e];
-    } else {
-      *reinterpret_cast<uint4*>(&Xs[t >> 2][(t & 3) * 8]) = v;
-    }
-  }
+enum { EPI_PART, EPI_ACT, EPI_DACT, EPI_OUT };
+struct Operand {
+  const uint16_t* p;
+  int64_t s, k;  // strides of row and k; 16-byte loads when k == 1 and s % 8 == 0
+  int rows;
+};
+struct Product {
+  Operand a, b;
+  int K, kchunk, tm, tn;
+  int epi;
+  const float* bias;     // EPI_ACT, EPI_OUT
+  const float* Z;        // EPI_DACT: pre-activations [m][256]
+  float* out;            // PART: [z][M][N]; ACT: Z; DACT: dZ; OUT: y
+  uint16_t* out16;       // ACT: silu(Z); DACT: dZ; OUT: dY, row major (may be NULL)
+  uint16_t* out16t;      // the same transposed, row pitch ldt (may be NULL)
+  int64_t ldt;
+  // EPI_OUT with a loss (target != NULL): dY = 2 w (y - t) / sum w, block partials of the loss
+  const float *target, *weight, *wsum_dev;
+  float inv_wsum;
+  float *dY, *loss_part;
+};
+struct ColSum {  // partial column sums of D [nb][ncol]
+  const float* D;
+  float* part;
+  int64_t nb;
+  int ncol;
+};
+struct Layer1Grad {  // partials of dW1, db1
+  const float *dZ, *x;
+  float* part;
+  int64_t nb;
+};
+struct Reduce {  // out[e] = sum_z part[z][e]
+  const float* part;
+  float* out;
+  int nz, ne;
 };
 
-// The next stage's operands are loaded into registers while the current stage's MFMAs run.
-template <int LA, int LB>
-__global__ __launch_bounds__(256) void gemm_kernel(const uint16_t* __restrict__ A, int64_t sAm,
-                                                   int64_t sAk, const uint16_t* __restrict__ B,
-                                                   int64_t sBk, int64_t sBn, float* __restrict__ C,
-                                                   int64_t ldc, int64_t cz, int M, int N, int K,
-                                                   int kchunk, const float* __restrict__ bias) {
-  __shared__ __align__(16) uint16_t As[GT][GPAD];
-  __shared__ __align__(16) uint16_t Bs[GT][GPAD];
-  const int m0 = blockIdx.x * GT, n0 = blockIdx.y * GT;
-  const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
+struct alignas(16) TileLds {
+  uint16_t a[GT][TPAD], b[GT][TPAD];
+};
+
+// One operand's 64 rows x TK k's of a stage: 16-byte pieces, all eight of a thread's loads in
+// flight before its first LDS store, zeros past the edges.  Pieces need K contiguous, rows of a
+// multiple of 8 elements and a K range that ends on a piece; other operands (the four-wide output
+// gradient and weights, a ragged batch's last stage) are read element by element.
+constexpr int NPIECE = TK / 8 * GT / 256;
+__device__ __forceinline__ bool in_pieces(const Operand& o, int k0, int ke) {
+  return o.k == 1 && (o.s & 7) == 0 && (ke - k0 >= TK || ((ke - k0) & 7) == 0);
+}
+__device__ __forceinline__ void load_pieces(const Operand& o, int r0, int k0, int ke, int t,
+                                            uint4 (&v)[NPIECE]) {
+  const int kc = k0 + ((t & 31) << 3);
+#pragma unroll
+  for (int u = 0; u < NPIECE; ++u) {
+    const int r = r0 + (t >> 5) + 8 * u;
+    v[u] = make_uint4(0, 0, 0, 0);
+    if (r < o.rows && kc < ke) v[u] = *reinterpret_cast<const uint4*>(o.p + (int64_t)r * o.s + kc);
+  }
+}
+__device__ __forceinline__ void store_pieces(uint16_t (*X)[TPAD], int t,
+                                             const uint4 (&v)[NPIECE]) {
+#pragma unroll
+  for (int u = 0; u < NPIECE; ++u)
+    *reinterpret_cast<uint4*>(&X[(t >> 5) + 8 * u][(t & 31) << 3]) = v[u];
+}
+__device__ __forceinline__ void fill_elements(const Operand& o, int r0, int k0, int ke, int kw,
+                                              int t, uint16_t (*X)[TPAD]) {
+  for (int c = t; c < GT * kw; c += 256) {
+    // neighbouring threads along the contiguous direction
+    const int row = o.k == 1 ? c / kw : c % GT, kk = o.k == 1 ? c - row * kw : c / GT;
+    const int r = r0 + row, k = k0 + kk;
+    X[row][kk] = r < o.rows && k < ke ? o.p[(int64_t)r * o.s + (int64_t)k * o.k] : (uint16_t)0;
+  }
+}
+
+template <int EPI>
+__device__ __forceinline__ void product(const Product& g, int blk, TileLds& lds) {
+  const int mi = blk % g.tm, ni = (blk / g.tm) % g.tn, z = blk / (g.tm * g.tn);
+  const int m0 = mi * GT, n0 = ni * GT;
+  const int kb = z * g.kchunk, ke = min(g.K, kb + g.kchunk);
   const int t = threadIdx.x, l = t & 63, w = t >> 6;
   const int wm = w & 1, wn = w >> 1;
   f32x16 acc = {};
-  TileLoad<LA> la;
-  TileLoad<LB> lb;
-  if (kb < ke) {
-    la.load(A, sAm, sAk, m0, M, kb, ke, t);
-    lb.load(B, sBn, sBk, n0, N, kb, ke, t);
-  }
-  for (int k0 = kb; k0 < ke; k0 += GK) {
-    la.store(As, t);
-    lb.store(Bs, t);
+  for (int k0 = kb; k0 < ke; k0 += TK) {
+    const int kw = min(TK, (ke - k0 + 15) & ~15);
+    const bool pa = in_pieces(g.a, k0, ke), pb = in_pieces(g.b, k0, ke);
+    uint4 va[NPIECE], vb[NPIECE];
+    if (pa) load_pieces(g.a, m0, k0, ke, t, va);
+    if (pb) load_pieces(g.b, n0, k0, ke, t, vb);
+    if (k0 > kb) __syncthreads();  // the previous stage has been read
+    if (pa)
+      store_pieces(lds.a, t, va);
+    else
+      fill_elements(g.a, m0, k0, ke, kw, t, lds.a);
+    if (pb)
+      store_pieces(lds.b, t, vb);
+    else
+      fill_elements(g.b, n0, k0, ke, kw, t, lds.b);
     __syncthreads();
-    if (k0 + GK < ke) {
-      la.load(A, sAm, sAk, m0, M, k0 + GK, ke, t);
-      lb.load(B, sBn, sBk, n0, N, k0 + GK, ke, t);
-    }
-#pragma unroll
-    for (int ks = 0; ks < GK; ks += 16) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(&As[32 * wm + (l & 31)][ks + 8 * (l >> 5)]);
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(&Bs[32 * wn + (l & 31)][ks + 8 * (l >> 5)]);
+#pragma unroll 4
+    for (int ks = 0; ks < kw; ks += 16) {
+      const bf16x8 a =
+          *reinterpret_cast<const bf16x8*>(&lds.a[32 * wm + (l & 31)][ks + 8 * (l >> 5)]);
+      const bf16x8 b =
+          *reinterpret_cast<const bf16x8*>(&lds.b[32 * wn + (l & 31)][ks + 8 * (l >> 5)]);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
     }
-    __syncthreads();
   }
+  const int M = g.a.rows, N = g.b.rows;
   const int col = n0 + 32 * wn + (l & 31);
-  if (col >= N) return;
-  const float bv = bias ? bias[col] : 0.0f;
+  const float bv = g.bias && col < N ? g.bias[col] : 0.0f;
+  float inv = g.inv_wsum, lsum = 0.0f;
+  if (EPI == EPI_OUT && g.target && g.wsum_dev) inv = 1.0f / *g.wsum_dev;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int row = m0 + 32 * wm + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-    if (row < M) C[(int64_t)blockIdx.z * cz + (int64_t)row * ldc + col] = acc[r] + bv;
-  }
-}
-
-__global__ void splitk_reduce_kernel(const float* __restrict__ P, int nz, int64_t mn,
-                                     float* __restrict__ C) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= mn) return;
-  float s = 0.0f;
-  for (int z = 0; z < nz; ++z) s += P[(int64_t)z * mn + i];
-  C[i] = s;
-}
-
-// ------------------------------------------------------------------------------------------
-// elementwise / reduction kernels
-// ------------------------------------------------------------------------------------------
-__global__ void round_kernel(const float* __restrict__ src, uint16_t* __restrict__ dst, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = f2bf(src[i]);
-}
-
-// The three matrix-core weights W2, W3, W4 to BF16 in one launch.
-__global__ void round_weights_kernel(const float* __restrict__ p, uint16_t* __restrict__ w2,
-                                     uint16_t* __restrict__ w3, uint16_t* __restrict__ w4) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < H * H) {
-    w2[i] = f2bf(p[OW2 + i]);
-  } else if (i < 2 * H * H) {
-    w3[i - H * H] = f2bf(p[OW3 + i - H * H]);
-  } else if (i < 2 * H * H + OUT * H) {
-    w4[i - 2 * H * H] = f2bf(p[OW4 + i - 2 * H * H]);
-  }
-}
-
-// Z1[b][o] = sum_i x[b][i] bf16(W1[o][i]) + b1[o];  A1 = bf16(silu(Z1))
-__global__ void layer1_fwd_kernel(const float* __restrict__ p, const float* __restrict__ x,
-                                  int64_t nb, float* __restrict__ Z, uint16_t* __restrict__ Aout) {
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= nb * H) return;
-  const int64_t b = idx / H;
-  const int o = (int)(idx - b * H);
-  float z = p[OB1 + o];
+  for (int q = 0; q < 4; ++q) {  // rows row0 .. row0 + 3 of this lane's column
+    const int row0 = m0 + 32 * wm + 8 * q + 4 * (l >> 5);
+    uint16_t h[4];
 #pragma unroll
-  for (int i = 0; i < IN; ++i) z = fmaf(x[b * IN + i], bf2f(f2bf(p[OW1 + o * IN + i])), z);
-  Z[idx] = z;
-  Aout[idx] = f2bf(silu(z));
-}
-
-__global__ void act_fwd_kernel(const float* __restrict__ Z, uint16_t* __restrict__ Aout, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) Aout[i] = f2bf(silu(Z[i]));
-}
-
-// dZ = dA * silu'(Z): fp32 in place in dA, BF16 copy in dZb
-__global__ void act_bwd_kernel(float* __restrict__ dA, const float* __restrict__ Z,
-                               uint16_t* __restrict__ dZb, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float d = dA[i] * silu_grad(Z[i]);
-  dA[i] = d;
-  if (dZb) dZb[i] = f2bf(d);
-}
-
-// Weighted squared error of the 4 outputs: loss = sum_b w_b |Y_b - T_b|^2 / sum_b w_b;
-// dY = 2 w_b (Y_b - T_b) / sum_b w_b (fp32 and BF16); per-block partial losses.  The weight sum
-// comes as 1/sum (inv_wsum) or, when wsum_dev is set, as the sum itself in device memory.
-__global__ __launch_bounds__(256) void mse_kernel(const float* __restrict__ Y,
-                                                  const float* __restrict__ T,
-                                                  const float* __restrict__ wt, float inv_wsum,
-                                                  const float* __restrict__ wsum_dev,
-                                                  int64_t nb, float* __restrict__ dY,
-                                                  uint16_t* __restrict__ dYb,
-                                                  float* __restrict__ partial) {
-  __shared__ float red[256];
-  if (wsum_dev) inv_wsum = 1.0f / *wsum_dev;
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  float acc = 0.0f;
-  if (b < nb) {
-    const float w = wt ? wt[b] : 1.0f;
+    for (int e = 0; e < 4; ++e) {
+      const int row = row0 + e;
+      const bool in = row < M && col < N;
+      const float c = acc[4 * q + e] + bv;
+      h[e] = 0;
+      if (!in) continue;
+      if constexpr (EPI == EPI_PART) {
+        g.out[((int64_t)z * M + row) * N + col] = c;
+      } else if constexpr (EPI == EPI_ACT) {
+        g.out[(int64_t)row * H + col] = c;
+        h[e] = f2bf(silu(c));
+        g.out16[(int64_t)row * H + col] = h[e];
+      } else if constexpr (EPI == EPI_DACT) {
+        const float d = c * silu_grad(g.Z[(int64_t)row * H + col]);
+        g.out[(int64_t)row * H + col] = d;
+        h[e] = f2bf(d);
+        if (g.out16) g.out16[(int64_t)row * H + col] = h[e];
+      } else {
+        g.out[(int64_t)row * OUT + col] = c;
+        if (g.target) {
+          const float wt = g.weight ? g.weight[row] : 1.0f;
+          const float d = c - g.target[(int64_t)row * OUT + col];
+          lsum += wt * d * d;
+          const float gr = 2.0f * wt * d * inv;
+          g.dY[(int64_t)row * OUT + col] = gr;
+          h[e] = f2bf(gr);
+          g.out16[(int64_t)row * OUT + col] = h[e];
+        }
+      }
+    }
+    if (EPI != EPI_PART && g.out16t && col < N) {
+      uint16_t* o = g.out16t + (int64_t)col * g.ldt + row0;
+      if (row0 + 4 <= M) {
+        uint2 v;
+        memcpy(&v, h, 8);
+        *reinterpret_cast<uint2*>(o) = v;
+      } else {
 #pragma unroll
-    for (int j = 0; j < OUT; ++j) {
-      const float d = Y[b * OUT + j] - T[b * OUT + j];
-      acc += w * d * d;
-      const float g = 2.0f * w * d * inv_wsum;
-      dY[b * OUT + j] = g;
-      dYb[b * OUT + j] = f2bf(g);
+        for (int e = 0; e < 4; ++e)
+          if (row0 + e < M) o[e] = h[e];
+      }
     }
   }
-  red[threadIdx.x] = acc * inv_wsum;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+  if (EPI == EPI_OUT && g.target) {
+    float* red = reinterpret_cast<float*>(&lds);
+    __syncthreads();  // the tiles have been read
+    red[t] = lsum * inv;
     __syncthreads();
+    for (int s = 128; s > 0; s >>= 1) {
+      if (t < s) red[t] += red[t + s];
+      __syncthreads();
+    }
+    if (t == 0) g.loss_part[mi] = red[0];
   }
-  if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-__global__ __launch_bounds__(256) void sum_kernel(const float* __restrict__ partial, int n,
-                                                  float* __restrict__ out) {
-  __shared__ float red[256];
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < n; i += 256) s += partial[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = red[0];
 }
 
 // Column sums over the batch in two deterministic passes: blocks of (64 columns x 4 row
-// phases) over batch chunks of CS_ROWS rows write partials, a second kernel adds the chunks.
-constexpr int CS_ROWS = 512;
-
-__global__ __launch_bounds__(256) void colsum_partial_kernel(const float* __restrict__ D,
-                                                             int64_t ld, int64_t nb, int ncol,
-                                                             float* __restrict__ part) {
-  __shared__ float red[4][64];
-  const int c = blockIdx.x * 64 + (threadIdx.x & 63), ph = threadIdx.x >> 6;
-  const int64_t b0 = (int64_t)blockIdx.y * CS_ROWS, b1 = min(nb, b0 + CS_ROWS);
+// phases) over batch chunks of CS_ROWS rows write partials, a later job adds the chunks.
+__device__ void col_sum(const ColSum& g, int blk, TileLds& lds) {
+  float(*red)[64] = reinterpret_cast<float(*)[64]>(&lds);
+  const int nc = (g.ncol + 63) / 64, by = blk / nc;
+  const int c = (blk - by * nc) * 64 + (threadIdx.x & 63), ph = threadIdx.x >> 6;
+  const int64_t b0 = (int64_t)by * CS_ROWS, b1 = min(g.nb, b0 + CS_ROWS);
   float s = 0.0f;
-  if (c < ncol)
+  if (c < g.ncol)
     // rows b0 + ph, b0 + ph + 4, ... added in order; the loads of 32 of them are issued first
     for (int64_t b = b0 + ph; b < b1; b += 128) {
       float v[32];
 #pragma unroll
-      for (int u = 0; u < 32; ++u) v[u] = b + 4 * u < b1 ? D[(b + 4 * u) * ld + c] : 0.0f;
+      for (int u = 0; u < 32; ++u) v[u] = b + 4 * u < b1 ? g.D[(b + 4 * u) * g.ncol + c] : 0.0f;
 #pragma unroll
       for (int u = 0; u < 32; ++u)
         if (b + 4 * u < b1) s += v[u];
     }
   red[ph][threadIdx.x & 63] = s;
   __syncthreads();
-  if (ph == 0 && c < ncol)
-    part[(int64_t)blockIdx.y * ncol + c] =
+  if (ph == 0 && c < g.ncol)
+    g.part[(int64_t)by * g.ncol + c] =
         red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
 }
 
 // dW1[o][i] = sum_b dZ1[b][o] x[b][i] and db1[o] = sum_b dZ1[b][o], partials per batch chunk:
 // part[chunk][o][4] = (dW1[o][0..2], db1[o]).
-__global__ __launch_bounds__(256) void layer1_grad_partial_kernel(const float* __restrict__ dZ,
-                                                                  const float* __restrict__ x,
-                                                                  int64_t nb,
-                                                                  float* __restrict__ part) {
-  __shared__ float red[4][64][IN + 1];
-  const int o = blockIdx.x * 64 + (threadIdx.x & 63), ph = threadIdx.x >> 6;
-  const int64_t b0 = (int64_t)blockIdx.y * CS_ROWS, b1 = min(nb, b0 + CS_ROWS);
+__device__ void layer1_grad(const Layer1Grad& g, int blk, TileLds& lds) {
+  float(*red)[64][IN + 1] = reinterpret_cast<float(*)[64][IN + 1]>(&lds);
+  float* xs = reinterpret_cast<float*>(&red[4]);  // the chunk's inputs, read by every column
+  const int by = blk / (H / 64);
+  const int o = (blk % (H / 64)) * 64 + (threadIdx.x & 63), ph = threadIdx.x >> 6;
+  const int64_t b0 = (int64_t)by * CS_ROWS, b1 = min(g.nb, b0 + CS_ROWS);
+  for (int e = threadIdx.x; e < (int)(b1 - b0) * IN; e += 256) xs[e] = g.x[b0 * IN + e];
+  __syncthreads();
   float s[IN + 1] = {0.0f, 0.0f, 0.0f, 0.0f};
-  // rows b0 + ph, b0 + ph + 4, ... accumulated in order; the loads of 16 of them are issued first
-  for (int64_t b = b0 + ph; b < b1; b += 64) {
-    float d[16], xv[16][IN];
+  // rows b0 + ph, b0 + ph + 4, ... accumulated in order; the loads of 32 of them are issued first
+  for (int64_t b = b0 + ph; b < b1; b += 128) {
+    float d[32];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-      const bool in = b + 4 * u < b1;
-      d[u] = in ? dZ[(b + 4 * u) * H + o] : 0.0f;
+    for (int u = 0; u < 32; ++u) d[u] = b + 4 * u < b1 ? g.dZ[(b + 4 * u) * H + o] : 0.0f;
 #pragma unroll
-      for (int i = 0; i < IN; ++i) xv[u][i] = in ? x[(b + 4 * u) * IN + i] : 0.0f;
-    }
-#pragma unroll
-    for (int u = 0; u < 16; ++u) {
+    for (int u = 0; u < 32; ++u) {
       if (b + 4 * u >= b1) break;
+      const float* xv = xs + (b + 4 * u - b0) * IN;
 #pragma unroll
-      for (int i = 0; i < IN; ++i) s[i] = fmaf(d[u], xv[u][i], s[i]);
+      for (int i = 0; i < IN; ++i) s[i] = fmaf(d[u], xv[i], s[i]);
       s[IN] += d[u];
     }
   }
@@ -301,19 +277,88 @@ __global__ __launch_bounds__(256) void layer1_grad_partial_kernel(const float* _
   if (ph == 0)
 #pragma unroll
     for (int i = 0; i <= IN; ++i)
-      part[((int64_t)blockIdx.y * H + o) * (IN + 1) + i] =
+      g.part[((int64_t)by * H + o) * (IN + 1) + i] =
           red[0][threadIdx.x][i] + red[1][threadIdx.x][i] + red[2][threadIdx.x][i] +
           red[3][threadIdx.x][i];
 }
 
-// out[e] = sum_z part[z][e] (e < ne); with stride_out = IN + 1 split for the layer-1 case
-__global__ void chunk_sum_kernel(const float* __restrict__ part, int nz, int ne,
-                                 float* __restrict__ out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= ne) return;
+__device__ void reduce_parts(const Reduce& g, int blk) {
+  const int e = blk * 256 + threadIdx.x;
+  if (e >= g.ne) return;
   float s = 0.0f;
-  for (int z = 0; z < nz; ++z) s += part[(int64_t)z * ne + e];
-  out[e] = s;
+  int z = 0;
+  for (; z + 8 <= g.nz; z += 8) {  // added in order; eight loads in flight
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = g.part[(int64_t)(z + u) * g.ne + e];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += v[u];
+  }
+  for (; z < g.nz; ++z) s += g.part[(int64_t)z * g.ne + e];
+  g.out[e] = s;
+}
+
+// Jobs of one launch: a column sum first (few blocks, the longest chains), a product, and with
+// WGRAD the split-K product of a weight gradient; blocks[i] is the number of blocks of job i.
+struct ProductJobs {
+  int blocks[3];
+  ColSum cs;
+  Product p[2];
+};
+template <int EPI, bool WGRAD>
+__global__ __launch_bounds__(256) void products_kernel(ProductJobs j) {
+  __shared__ TileLds lds;
+  int blk = blockIdx.x;
+  if (WGRAD) {
+    if (blk < j.blocks[0]) {
+      col_sum(j.cs, blk, lds);
+      return;
+    }
+    blk -= j.blocks[0];
+  }
+  if (!WGRAD || blk < j.blocks[1])
+    product<EPI>(j.p[0], blk, lds);
+  else
+    product<EPI_PART>(j.p[1], blk - j.blocks[1], lds);
+}
+
+// The last jobs: first-layer gradient partials and the reductions of all earlier partials.
+constexpr int NRED = 6;
+struct FinishJobs {
+  int blocks[1 + NRED];
+  Layer1Grad l1;
+  Reduce r[NRED];
+  const float* loss_part;  // NULL: no loss
+  int n_loss;
+  float* loss;
+};
+__global__ __launch_bounds__(256) void finish_kernel(FinishJobs j) {
+  __shared__ TileLds lds;
+  int blk = blockIdx.x;
+  if (blk < j.blocks[0]) {
+    layer1_grad(j.l1, blk, lds);
+    return;
+  }
+  blk -= j.blocks[0];
+#pragma unroll
+  for (int q = 0; q < NRED; ++q) {
+    if (blk < j.blocks[1 + q]) {
+      reduce_parts(j.r[q], blk);
+      return;
+    }
+    blk -= j.blocks[1 + q];
+  }
+  if (!j.loss_part) return;
+  float* red = reinterpret_cast<float*>(&lds);
+  float s = 0.0f;
+  for (int i = threadIdx.x; i < j.n_loss; i += 256) s += j.loss_part[i];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  for (int k = 128; k > 0; k >>= 1) {
+    if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) j.loss[0] = red[0];
 }
 
 __global__ void layer1_grad_finish(const float* __restrict__ part, int nz, float* __restrict__ dW1,
@@ -321,12 +366,82 @@ __global__ void layer1_grad_finish(const float* __restrict__ part, int nz, float
   const int o = blockIdx.x * blockDim.x + threadIdx.x;
   if (o >= H) return;
   float s[IN + 1] = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int z = 0; z < nz; ++z)
-#pragma unroll
-    for (int i = 0; i <= IN; ++i) s[i] += part[((int64_t)z * H + o) * (IN + 1) + i];
+#pragma unroll 4
+  for (int z = 0; z < nz; ++z) {
+    const float4 v = *reinterpret_cast<const float4*>(part + ((int64_t)z * H + o) * (IN + 1));
+    s[0] += v.x;
+    s[1] += v.y;
+    s[2] += v.z;
+    s[3] += v.w;
+  }
 #pragma unroll
   for (int i = 0; i < IN; ++i) dW1[o * IN + i] = s[i];
   db1[o] = s[IN];
+}
+
+// The matrix-core weights W2, W3, W4 to BF16, W2 and W3 transposed as well, and the first layer:
+// Z1[b][o] = sum_i x[b][i] bf16(W1[o][i]) + b1[o], A1 = bf16(silu(Z1)) in both orders (a thread
+// takes one neuron and eight points).
+constexpr int L1_PTS = 8;
+__global__ __launch_bounds__(256) void first_kernel(const float* __restrict__ p,
+                                                    const float* __restrict__ x, int64_t nb,
+                                                    int wblocks, uint16_t* __restrict__ w2,
+                                                    uint16_t* __restrict__ w3,
+                                                    uint16_t* __restrict__ w4,
+                                                    uint16_t* __restrict__ w2t,
+                                                    uint16_t* __restrict__ w3t,
+                                                    float* __restrict__ Z,
+                                                    uint16_t* __restrict__ A,
+                                                    uint16_t* __restrict__ At, int64_t ldt) {
+  if ((int)blockIdx.x < wblocks) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 2 * H * H) {
+      const int e = i < H * H ? i : i - H * H;
+      const uint16_t h = f2bf(p[(i < H * H ? OW2 : OW3) + e]);
+      const int o = e / H, c = e % H;
+      (i < H * H ? w2 : w3)[e] = h;
+      (i < H * H ? w2t : w3t)[c * H + o] = h;
+    } else if (i < 2 * H * H + OUT * H) {
+      w4[i - 2 * H * H] = f2bf(p[OW4 + i - 2 * H * H]);
+    }
+    return;
+  }
+  const int o = threadIdx.x;
+  const int64_t b0 = (int64_t)(blockIdx.x - wblocks) * L1_PTS;
+  float w[IN];
+#pragma unroll
+  for (int i = 0; i < IN; ++i) w[i] = bf2f(f2bf(p[OW1 + o * IN + i]));
+  const float bias = p[OB1 + o];
+  uint16_t h[L1_PTS];
+#pragma unroll
+  for (int e = 0; e < L1_PTS; ++e) {
+    const int64_t b = b0 + e;
+    h[e] = 0;
+    if (b >= nb) continue;
+    float z = bias;
+#pragma unroll
+    for (int i = 0; i < IN; ++i) z = fmaf(x[b * IN + i], w[i], z);
+    h[e] = f2bf(silu(z));
+    Z[b * H + o] = z;
+    A[b * H + o] = h[e];
+  }
+  if (At) {  // ldt is nb rounded up to 8: the padding may be written
+    uint4 v;
+    memcpy(&v, h, 16);
+    *reinterpret_cast<uint4*>(At + (int64_t)o * ldt + b0) = v;
+  }
+}
+
+// A given output gradient into the workspace: fp32 copy, BF16 in both orders.
+__global__ void seed_kernel(const float* __restrict__ dy, int64_t nb, float* __restrict__ dY,
+                            uint16_t* __restrict__ dYb, uint16_t* __restrict__ dYt, int64_t ldt) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nb * OUT) return;
+  const float d = dy[i];
+  const uint16_t h = f2bf(d);
+  dY[i] = d;
+  dYb[i] = h;
+  dYt[(i % OUT) * ldt + i / OUT] = h;
 }
 
 __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g,
@@ -436,165 +551,186 @@ namespace {
 using namespace mlp;
 
 struct Workspace {
-  float *Z1, *Z2, *Z3, *dA, *dY, *part, *red;
-  uint16_t *A1, *A2, *A3, *dZb, *dYb, *W2b, *W3b, *W4b;
+  float *Z1, *Z2, *Z3, *dZ3, *dZ2, *dZ1, *dY, *ytmp, *loss_part;
+  float *pW4, *pW3, *pW2, *pb4, *pb3, *pb2, *pl1;  // partials of the gradient sums
+  uint16_t *A1, *A2, *A3, *A1t, *A2t, *A3t, *dZb, *dZ3t, *dZ2t, *dYb, *dYt;
+  uint16_t *W2b, *W3b, *W4b, *W2t, *W3t;
+  int64_t ldt;  // row pitch of the transposed arrays: the batch rounded up to 8
+  int64_t bytes;
 };
 
 int64_t splitk_for(int64_t nb) {
   int64_t z = nb / 512;
   return z < 1 ? 1 : (z > 64 ? 64 : z);
 }
+int64_t chunks_of(int64_t nb) { return (nb + CS_ROWS - 1) / CS_ROWS; }
 
-int64_t ws_bytes(int64_t nb) {
-  const int64_t nz = splitk_for(nb);
-  int64_t b = 0;
-  b += 3 * nb * H * 4;            // Z1..Z3
-  b += nb * H * 4;                // dA / dZ (fp32)
-  b += 2 * nb * OUT * 4;          // dY, (spare)
-  b += (nz * H * H + ((nb + CS_ROWS - 1) / CS_ROWS) * H * (IN + 1)) * 4;  // partials
-  b += ((nb + 255) / 256 + 64) * 4;  // loss partials
-  b += 3 * nb * H * 2;            // A1..A3
-  b += nb * H * 2;                // dZ bf16
-  b += nb * OUT * 2;              // dY bf16
-  b += (2 * H * H + OUT * H) * 2; // BF16 weights
-  return b + 16 * 64;             // alignment slack
-}
-
+// Layout of the workspace for a batch; base NULL: the size only.
 Workspace carve(void* base, int64_t nb) {
-  char* p = (char*)base;
+  Workspace w;
+  int64_t off = 0;
+  base = (void*)(((uintptr_t)base + 63) & ~(uintptr_t)63);
   auto take = [&](int64_t bytes) {
-    char* r = p;
-    p += (bytes + 63) / 64 * 64;
+    char* r = base ? (char*)base + off : nullptr;
+    off += (bytes + 63) / 64 * 64;
     return r;
   };
-  const int64_t nz = splitk_for(nb);
-  Workspace w;
-  w.Z1 = (float*)take(nb * H * 4);
-  w.Z2 = (float*)take(nb * H * 4);
-  w.Z3 = (float*)take(nb * H * 4);
-  w.dA = (float*)take(nb * H * 4);
-  w.dY = (float*)take(2 * nb * OUT * 4);
-  w.part = (float*)take((nz * H * H + ((nb + CS_ROWS - 1) / CS_ROWS) * H * (IN + 1)) * 4);
-  w.red = (float*)take(((nb + 255) / 256 + 64) * 4);
-  w.A1 = (uint16_t*)take(nb * H * 2);
-  w.A2 = (uint16_t*)take(nb * H * 2);
-  w.A3 = (uint16_t*)take(nb * H * 2);
-  w.dZb = (uint16_t*)take(nb * H * 2);
-  w.dYb = (uint16_t*)take(nb * OUT * 2);
-  w.W2b = (uint16_t*)take(H * H * 2);
-  w.W3b = (uint16_t*)take(H * H * 2);
-  w.W4b = (uint16_t*)take(OUT * H * 2);
+  auto f32 = [&](int64_t n) { return (float*)take(n * 4); };
+  auto b16 = [&](int64_t n) { return (uint16_t*)take(n * 2); };
+  const int64_t nz = splitk_for(nb), nc = chunks_of(nb);
+  w.ldt = (nb + 7) / 8 * 8;
+  w.Z1 = f32(nb * H); w.Z2 = f32(nb * H); w.Z3 = f32(nb * H);
+  w.dZ3 = f32(nb * H); w.dZ2 = f32(nb * H); w.dZ1 = w.dZ3;  // dZ3 is done with before dZ1
+  w.dY = f32(nb * OUT); w.ytmp = f32(nb * OUT);
+  w.loss_part = f32((nb + GT - 1) / GT);
+  w.pW4 = f32(nz * OUT * H); w.pW3 = f32(nz * H * H); w.pW2 = f32(nz * H * H);
+  w.pb4 = f32(nc * OUT); w.pb3 = f32(nc * H); w.pb2 = f32(nc * H); w.pl1 = f32(nc * H * (IN + 1));
+  w.A1 = b16(nb * H); w.A2 = b16(nb * H); w.A3 = b16(nb * H);
+  w.A1t = b16(w.ldt * H); w.A2t = b16(w.ldt * H); w.A3t = b16(w.ldt * H);
+  w.dZb = b16(2 * nb * H);  // two layers in turn: one is read while the next is written
+  w.dZ3t = b16(w.ldt * H); w.dZ2t = b16(w.ldt * H);
+  w.dYb = b16(nb * OUT); w.dYt = b16(w.ldt * OUT);
+  w.W2b = b16(H * H); w.W3b = b16(H * H); w.W4b = b16(OUT * H);
+  w.W2t = b16(H * H); w.W3t = b16(H * H);
+  w.bytes = off + 64;  // room to align the caller's base
   return w;
 }
 
+int64_t ws_bytes(int64_t nb) { return carve(nullptr, nb).bytes; }
+
 inline unsigned nblk(int64_t n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-void colsum(const float* D, int64_t ld, int64_t nb, int ncol, float* out, float* scratch,
-            hipStream_t st) {
-  const int nz = (int)((nb + CS_ROWS - 1) / CS_ROWS);
-  hipLaunchKernelGGL(colsum_partial_kernel, dim3((ncol + 63) / 64, nz), dim3(256), 0, st, D, ld, nb,
-                     ncol, scratch);
-  hipLaunchKernelGGL(chunk_sum_kernel, dim3(nblk(ncol)), dim3(256), 0, st, scratch, nz, ncol, out);
+Product make_product(Operand a, Operand b, int K, int nz, int epi) {
+  Product g = {};
+  g.a = a;
+  g.b = b;
+  g.K = K;
+  g.kchunk = ((K + nz - 1) / nz + GK - 1) / GK * GK;
+  g.tm = (int)nblk(a.rows, GT);
+  g.tn = (int)nblk(b.rows, GT);
+  g.epi = epi;
+  return g;
+}
+int product_blocks(const Product& g) {
+  return g.tm * g.tn * ((g.K + g.kchunk - 1) / g.kchunk);
 }
 
-// Loader layout of an operand X(r, k) = X[r * sr + k * sk] (see TileLoad).
-int gemm_layout(const uint16_t* X, int64_t sr, int64_t sk) {
-  if ((reinterpret_cast<uintptr_t>(X) & 15) != 0) return GL_ANY;
-  if (sk == 1 && sr % 8 == 0) return GL_K;
-  if (sr == 1 && sk % 8 == 0) return GL_R;
-  return GL_ANY;
-}
-
-template <int LA, int LB>
-void gemm_launch(dim3 grid, hipStream_t st, const uint16_t* A, int64_t sAm, int64_t sAk,
-                 const uint16_t* B, int64_t sBk, int64_t sBn, float* C, int64_t ldc, int64_t cz,
-                 int M, int N, int K, int kchunk, const float* bias) {
-  hipLaunchKernelGGL((gemm_kernel<LA, LB>), grid, dim3(256), 0, st, A, sAm, sAk, B, sBk, sBn, C,
-                     ldc, cz, M, N, K, kchunk, bias);
-}
-
-template <int LA>
-void gemm_launch_b(int lb, dim3 grid, hipStream_t st, const uint16_t* A, int64_t sAm, int64_t sAk,
-                   const uint16_t* B, int64_t sBk, int64_t sBn, float* C, int64_t ldc, int64_t cz,
-                   int M, int N, int K, int kchunk, const float* bias) {
-  if (lb == GL_K)
-    gemm_launch<LA, GL_K>(grid, st, A, sAm, sAk, B, sBk, sBn, C, ldc, cz, M, N, K, kchunk, bias);
-  else if (lb == GL_R)
-    gemm_launch<LA, GL_R>(grid, st, A, sAm, sAk, B, sBk, sBn, C, ldc, cz, M, N, K, kchunk, bias);
+void launch_product(const Product& p, hipStream_t st) {
+  ProductJobs j = {};
+  j.p[0] = p;
+  j.blocks[1] = product_blocks(p);
+  const dim3 grid((unsigned)j.blocks[1]);
+  if (p.epi == EPI_ACT)
+    hipLaunchKernelGGL((products_kernel<EPI_ACT, false>), grid, dim3(256), 0, st, j);
   else
-    gemm_launch<LA, GL_ANY>(grid, st, A, sAm, sAk, B, sBk, sBn, C, ldc, cz, M, N, K, kchunk, bias);
+    hipLaunchKernelGGL((products_kernel<EPI_OUT, false>), grid, dim3(256), 0, st, j);
+}
+// One backward launch: bias column sums, the layer below's gradient, the weight gradient.
+void launch_backward(const ColSum& cs, const Product& d, const Product& w, hipStream_t st) {
+  ProductJobs j = {};
+  j.cs = cs;
+  j.blocks[0] = (int)(((cs.ncol + 63) / 64) * chunks_of(cs.nb));
+  j.p[0] = d;
+  j.blocks[1] = product_blocks(d);
+  j.p[1] = w;
+  j.blocks[2] = product_blocks(w);
+  hipLaunchKernelGGL((products_kernel<EPI_DACT, true>),
+                     dim3((unsigned)(j.blocks[0] + j.blocks[1] + j.blocks[2])), dim3(256), 0, st, j);
 }
 
-void gemm_dispatch(dim3 grid, hipStream_t st, const uint16_t* A, int64_t sAm, int64_t sAk,
-                   const uint16_t* B, int64_t sBk, int64_t sBn, float* C, int64_t ldc, int64_t cz,
-                   int M, int N, int K, int kchunk, const float* bias) {
-  const int la = gemm_layout(A, sAm, sAk), lb = gemm_layout(B, sBn, sBk);
-  if (la == GL_K)
-    gemm_launch_b<GL_K>(lb, grid, st, A, sAm, sAk, B, sBk, sBn, C, ldc, cz, M, N, K, kchunk, bias);
-  else if (la == GL_R)
-    gemm_launch_b<GL_R>(lb, grid, st, A, sAm, sAk, B, sBk, sBn, C, ldc, cz, M, N, K, kchunk, bias);
-  else
-    gemm_launch_b<GL_ANY>(lb, grid, st, A, sAm, sAk, B, sBk, sBn, C, ldc, cz, M, N, K, kchunk,
-                          bias);
-}
+// Loss of the training step: targets, weights and their sum (1 / sum, or the sum in device memory).
+struct LossArgs {
+  const float *target, *weight, *wsum_dev;
+  float inv_wsum;
+};
 
-void gemm(const uint16_t* A, int64_t sAm, int64_t sAk, const uint16_t* B, int64_t sBk,
-          int64_t sBn, float* C, int M, int N, int K, const float* bias, hipStream_t st,
-          float* part = nullptr, int nz = 1) {
-  if (nz <= 1 || !part) {
-    gemm_dispatch(dim3(nblk(M, GT), nblk(N, GT), 1), st, A, sAm, sAk, B, sBk, sBn, C, (int64_t)N,
-                  (int64_t)0, M, N, K, K, bias);
-    return;
-  }
-  int kchunk = (K + nz - 1) / nz;
-  kchunk = (kchunk + GK - 1) / GK * GK;
-  nz = (K + kchunk - 1) / kchunk;
-  gemm_dispatch(dim3(nblk(M, GT), nblk(N, GT), nz), st, A, sAm, sAk, B, sBk, sBn, part, (int64_t)N,
-                (int64_t)M * N, M, N, K, kchunk, nullptr);
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(nblk((int64_t)M * N)), dim3(256), 0, st, part, nz,
-                     (int64_t)M * N, C);
-}
-
-void round_weights(const float* p, Workspace& w, hipStream_t st) {
-  hipLaunchKernelGGL(round_weights_kernel, dim3(nblk(2 * H * H + OUT * H)), dim3(256), 0, st, p,
-                     w.W2b, w.W3b, w.W4b);
-}
-
-void forward(const float* p, const float* x, int64_t nb, float* y, Workspace& w, hipStream_t st) {
-  round_weights(p, w, st);
-  hipLaunchKernelGGL(layer1_fwd_kernel, dim3(nblk(nb * H)), dim3(256), 0, st, p, x, nb, w.Z1, w.A1);
-  gemm(w.A1, H, 1, w.W2b, 1, H, w.Z2, (int)nb, H, H, p + OB2, st);
-  hipLaunchKernelGGL(act_fwd_kernel, dim3(nblk(nb * H)), dim3(256), 0, st, w.Z2, w.A2, nb * H);
-  gemm(w.A2, H, 1, w.W3b, 1, H, w.Z3, (int)nb, H, H, p + OB3, st);
-  hipLaunchKernelGGL(act_fwd_kernel, dim3(nblk(nb * H)), dim3(256), 0, st, w.Z3, w.A3, nb * H);
-  gemm(w.A3, H, 1, w.W4b, 1, H, y, (int)nb, OUT, H, p + OB4, st);
-}
-
-// Backward from dY (fp32 in w.dY, BF16 in w.dYb) given a forward with the same workspace.
-void backward(const float* x, int64_t nb, float* g, Workspace& w, hipStream_t st) {
-  const int nz = (int)splitk_for(nb);
-  // output layer
-  gemm(w.dYb, 1, OUT, w.A3, H, 1, g + OW4, OUT, H, (int)nb, nullptr, st, w.part, nz);
-  colsum(w.dY, OUT, nb, OUT, g + OB4, w.part, st);
-  gemm(w.dYb, OUT, 1, w.W4b, H, 1, w.dA, (int)nb, H, OUT, nullptr, st);
-  // hidden layers 3 and 2
-  const float* Zs[2] = {w.Z3, w.Z2};
-  const uint16_t* Ain[2] = {w.A2, w.A1};
-  const uint16_t* Wb[2] = {w.W3b, w.W2b};
-  const int64_t oW[2] = {OW3, OW2}, oB[2] = {OB3, OB2};
+// grad: keep the transposed activations for the backward pass; loss: form dY as well.
+void forward(const float* p, const float* x, int64_t nb, float* y, Workspace& w, bool grad,
+             const LossArgs* loss, hipStream_t st) {
+  const unsigned wblocks = nblk(2 * H * H + OUT * H);
+  hipLaunchKernelGGL(first_kernel, dim3(wblocks + nblk(nb, L1_PTS)), dim3(256), 0, st, p, x, nb,
+                     (int)wblocks, w.W2b, w.W3b, w.W4b, w.W2t, w.W3t, w.Z1, w.A1,
+                     grad ? w.A1t : nullptr, w.ldt);
+  const uint16_t* Ain[2] = {w.A1, w.A2};
+  uint16_t *Aout[2] = {w.A2, w.A3}, *At[2] = {w.A2t, w.A3t};
+  const uint16_t* Wb[2] = {w.W2b, w.W3b};
+  float* Z[2] = {w.Z2, w.Z3};
+  const int64_t ob[2] = {OB2, OB3};
   for (int s = 0; s < 2; ++s) {
-    hipLaunchKernelGGL(act_bwd_kernel, dim3(nblk(nb * H)), dim3(256), 0, st, w.dA, Zs[s], w.dZb, nb * H);
-    gemm(w.dZb, 1, H, Ain[s], H, 1, g + oW[s], H, H, (int)nb, nullptr, st, w.part, nz);
-    colsum(w.dA, H, nb, H, g + oB[s], w.part, st);
-    gemm(w.dZb, H, 1, Wb[s], H, 1, w.dA, (int)nb, H, H, nullptr, st);
+    Product g = make_product({Ain[s], H, 1, (int)nb}, {Wb[s], H, 1, H}, H, 1, EPI_ACT);
+    g.bias = p + ob[s];
+    g.out = Z[s];
+    g.out16 = Aout[s];
+    g.out16t = grad ? At[s] : nullptr;
+    g.ldt = w.ldt;
+    launch_product(g, st);
   }
-  // first layer (fp32)
-  hipLaunchKernelGGL(act_bwd_kernel, dim3(nblk(nb * H)), dim3(256), 0, st, w.dA, w.Z1,
-                     (uint16_t*)nullptr, nb * H);
-  const int nz1 = (int)((nb + CS_ROWS - 1) / CS_ROWS);
-  hipLaunchKernelGGL(layer1_grad_partial_kernel, dim3(H / 64, nz1), dim3(256), 0, st, w.dA, x, nb,
-                     w.part);
-  hipLaunchKernelGGL(layer1_grad_finish, dim3(1), dim3(H), 0, st, w.part, nz1, g + OW1, g + OB1);
+  Product g = make_product({w.A3, H, 1, (int)nb}, {w.W4b, H, 1, OUT}, H, 1, EPI_OUT);
+  g.bias = p + OB4;
+  g.out = y;
+  if (loss) {
+    g.target = loss->target;
+    g.weight = loss->weight;
+    g.wsum_dev = loss->wsum_dev;
+    g.inv_wsum = loss->inv_wsum;
+    g.dY = w.dY;
+    g.out16 = w.dYb;
+    g.out16t = w.dYt;
+    g.ldt = w.ldt;
+    g.loss_part = w.loss_part;
+  }
+  launch_product(g, st);
+}
+
+// Backward from dY (fp32 in w.dY, BF16 in w.dYb and w.dYt) given a forward with the same
+// workspace and its transposed activations; loss: also add up the loss partials.
+void backward(const float* x, int64_t nb, float* g, Workspace& w, float* loss, hipStream_t st) {
+  const int nz = (int)splitk_for(nb), n = (int)nb;
+  const int nc = (int)chunks_of(nb);
+  uint16_t* dZb[2] = {w.dZb, w.dZb + nb * H};
+  // each launch: the gradient of one layer's weights and biases, and the next layer down
+  Product w4 = make_product({w.dYt, w.ldt, 1, OUT}, {w.A3t, w.ldt, 1, H}, n, nz, EPI_PART);
+  w4.out = w.pW4;
+  Product d3 = make_product({w.dYb, OUT, 1, n}, {w.W4b, 1, H, H}, OUT, 1, EPI_DACT);
+  d3.Z = w.Z3; d3.out = w.dZ3; d3.out16 = dZb[0]; d3.out16t = w.dZ3t; d3.ldt = w.ldt;
+  const ColSum b4{w.dY, w.pb4, nb, OUT};
+  launch_backward(b4, d3, w4, st);
+
+  Product w3 = make_product({w.dZ3t, w.ldt, 1, H}, {w.A2t, w.ldt, 1, H}, n, nz, EPI_PART);
+  w3.out = w.pW3;
+  Product d2 = make_product({dZb[0], H, 1, n}, {w.W3t, H, 1, H}, H, 1, EPI_DACT);
+  d2.Z = w.Z2; d2.out = w.dZ2; d2.out16 = dZb[1]; d2.out16t = w.dZ2t; d2.ldt = w.ldt;
+  const ColSum b3{w.dZ3, w.pb3, nb, H};
+  launch_backward(b3, d2, w3, st);
+
+  Product w2 = make_product({w.dZ2t, w.ldt, 1, H}, {w.A1t, w.ldt, 1, H}, n, nz, EPI_PART);
+  w2.out = w.pW2;
+  Product d1 = make_product({dZb[1], H, 1, n}, {w.W2t, H, 1, H}, H, 1, EPI_DACT);
+  d1.Z = w.Z1; d1.out = w.dZ1;
+  const ColSum b2{w.dZ2, w.pb2, nb, H};
+  launch_backward(b2, d1, w2, st);
+
+  FinishJobs f = {};
+  f.l1 = Layer1Grad{w.dZ1, x, w.pl1, nb};
+  f.blocks[0] = (H / 64) * nc;
+  const int z = (n + w3.kchunk - 1) / w3.kchunk;  // chunks written by the weight products
+  const Reduce r[NRED] = {{w.pW3, g + OW3, z, H * H}, {w.pW2, g + OW2, z, H * H},
+                          {w.pW4, g + OW4, z, OUT * H}, {w.pb4, g + OB4, nc, OUT},
+                          {w.pb3, g + OB3, nc, H}, {w.pb2, g + OB2, nc, H}};
+  unsigned total = f.blocks[0];
+  for (int q = 0; q < NRED; ++q) {
+    f.r[q] = r[q];
+    f.blocks[1 + q] = (int)nblk(r[q].ne);
+    total += f.blocks[1 + q];
+  }
+  if (loss) {
+    f.loss_part = w.loss_part;
+    f.n_loss = (int)nblk(nb, GT);
+    f.loss = loss;
+    ++total;
+  }
+  hipLaunchKernelGGL(finish_kernel, dim3(total), dim3(256), 0, st, f);
+  hipLaunchKernelGGL(layer1_grad_finish, dim3(1), dim3(H), 0, st, w.pl1, nc, g + OW1, g + OB1);
 }
 
 }  // namespace
@@ -618,7 +754,7 @@ int ssc_mlp_forward(const float* params, const float* x, int64_t batch, float* y
   if (batch > (1 << 24)) return fail(SSC_E_LIMIT, "ssc_mlp_forward: batch above 16M");
   if (workspace_bytes < ws_bytes(batch)) return fail(SSC_E_ARG, "ssc_mlp_forward: workspace too small");
   Workspace w = carve(workspace, batch);
-  forward(params, x, batch, y, w, (hipStream_t)stream);
+  forward(params, x, batch, y, w, false, nullptr, (hipStream_t)stream);
   return check_launch("ssc_mlp_forward");
 }
 
@@ -635,13 +771,9 @@ static int loss_backward(const char* name, const float* params, const float* x,
     return fail(SSC_E_ARG, std::string(name) + ": weight_sum must be > 0");
   hipStream_t st = (hipStream_t)stream;
   Workspace w = carve(workspace, batch);
-  forward(params, x, batch, y, w, st);
-  const unsigned nbk = nblk(batch);
-  hipLaunchKernelGGL(mse_kernel, dim3(nbk), dim3(256), 0, st, y, target, weight,
-                     weight_sum_dev ? 0.0f : 1.0f / weight_sum, weight_sum_dev, batch, w.dY,
-                     w.dYb, w.red);
-  hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, st, w.red, (int)nbk, loss);
-  backward(x, batch, grads, w, st);
+  const LossArgs la{target, weight, weight_sum_dev, weight_sum_dev ? 0.0f : 1.0f / weight_sum};
+  forward(params, x, batch, y, w, true, &la, st);
+  backward(x, batch, grads, w, loss, st);
   return check_launch(name);
 }
 
@@ -669,12 +801,11 @@ int ssc_mlp_backward(const float* params, const float* x, const float* dy, int64
   if (workspace_bytes < ws_bytes(batch)) return fail(SSC_E_ARG, "ssc_mlp_backward: workspace too small");
   hipStream_t st = (hipStream_t)stream;
   Workspace w = carve(workspace, batch);
-  // recompute the forward into the workspace, then copy dy into the fp32/BF16 buffers
-  float* ytmp = w.dY + batch * OUT;
-  forward(params, x, batch, ytmp, w, st);
-  hipMemcpyAsync(w.dY, dy, batch * OUT * 4, hipMemcpyDeviceToDevice, st);
-  hipLaunchKernelGGL(round_kernel, dim3(nblk(batch * OUT)), dim3(256), 0, st, dy, w.dYb, batch * OUT);
-  backward(x, batch, grads, w, st);
+  // recompute the forward into the workspace; dy takes the place of the loss gradient
+  forward(params, x, batch, w.ytmp, w, true, nullptr, st);
+  hipLaunchKernelGGL(seed_kernel, dim3(nblk(batch * OUT)), dim3(256), 0, st, dy, batch, w.dY, w.dYb,
+                     w.dYt, w.ldt);
+  backward(x, batch, grads, w, nullptr, st);
   return check_launch("ssc_mlp_backward");
 }
 
