@@ -228,7 +228,7 @@ int ssc_release_seeds(const ssc_host_potential* host, const ssc_sources* src, co
  *   w_out[n][6], dw_out[n][m][D] at grid index nsteps (must not alias w0, dw0 when a
  *                   workspace is given)
  *   workspace       NULL, or device memory of workspace_bytes (ssc_perturb_workspace_bytes
- *                   gives a size of at most 2 GiB): the base orbits are then advanced once per
+ *                   gives a size of at most 4 GiB): the base orbits are then advanced once per
  *                   particle through segments of grid rows, recording position and host Hessian
  *                   per row for the responses; without it every lane that holds responses of a
  *                   particle recomputes them (about twice the arithmetic; the source forces

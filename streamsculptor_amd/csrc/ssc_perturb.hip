@@ -14,10 +14,11 @@
 // Layout: L = ceil(m / G) lanes per particle; lane g of a particle owns the G responses g,
 // g + L, g + 2L, ... (strided: at every response slot the L lanes read consecutive source
 // records, which keeps their LDS reads free of bank conflicts).  With a workspace the
-// grid is cut into segments of rows: perturb_base_kernel (one particle per lane) advances the
-// base orbits through a segment and records, at every row a particle is kicked at, its position
-// and the host Hessian; perturb_rows_kernel then advances the responses through the segment
-// from those records.  Without one, perturb_kernel has each of the L lanes recompute the base
+// grid is cut into segments of rows: base_rows (one particle per lane) advances the base orbits
+// through a segment and records, at every row a particle is kicked at, its position and the host
+// Hessian; response_rows then advances the responses through the segment from those records.
+// One launch carries the base rows of segment s + 1 beside the responses of segment s: the first
+// waits for memory (72 B a particle and row), the second for FP64 issue.  Without a workspace perturb_kernel has each of the L lanes recompute the base
 // orbit and the host Hessian (2.2x the arithmetic of the split form, measured by counters).
 // Velocities are carried at half steps so that forces are consumed as soon as they are formed.
 #include <hip/hip_runtime.h>
@@ -39,6 +40,29 @@ __device__ __forceinline__ void host_grad_hess(const ssc_host_potential& hp, dou
                                                double z, double* g, double* H) {
   double phi;
   host_full_sig<HS, true>(hp, x, y, z, phi, g, H);
+}
+
+// The same from the components' four numbers, accumulated into g and H's upper triangle: the
+// spherical components are added up before their 3 x 3 terms are formed.
+template <int HS>
+__device__ __forceinline__ void host_quads(const ssc_host_potential& hp, double x, double y,
+                                           double z, double* g, double* H) {
+  if constexpr (HS == HS_GENERIC) {
+    for (int c = 0; c < hp.n_components; ++c) quad_add(comp_quad(hp.c[c], x, y, z), x, y, g, H);
+  } else {
+    const CompQuad d = comp_quad<hs_kind(HS, 0)>(hp.c[0], x, y, z);
+    CompQuad q = comp_quad<hs_kind(HS, 1)>(hp.c[1], x, y, z);
+    const CompQuad q2 = comp_quad<hs_kind(HS, 2)>(hp.c[2], x, y, z);
+    q.f += q2.f;
+    q.k += q2.k;
+    if constexpr (hs_components(HS) > 3) {
+      const CompQuad q3 = comp_quad<hs_kind(HS, 3)>(hp.c[3], x, y, z);
+      q.f += q3.f;
+      q.k += q3.k;
+    }
+    quad_add(d, x, y, g, H);
+    quad_add(q, x, y, g, H);
+  }
 }
 
 template <int SK, int G, int RAD, int HS>
@@ -206,48 +230,80 @@ __global__ void pt_zero_kernel(double* __restrict__ p, int64_t n) {
   if (e < n) p[e] = 0.0;
 }
 
-// Base orbits in place in w (initialised to w0): one particle per lane.
+// Base orbits in place in w (initialised to w0), rows [ka, kb]: one particle per lane.  A wave's
+// 64 records of a row go through LDS, so that they leave as nine stores of 512 consecutive bytes
+// (80,000 orbits x 4,000 rows 6.3 ms by itself; 7.6 ms written by their own lanes 72 B apart).
+constexpr int BASE_LDS = PT_BLOCK * PR_REC * 8;
+
 template <int HS>
-__global__ __launch_bounds__(256) void perturb_base_kernel(
-    ssc_host_potential hp, double* __restrict__ w, const int32_t* __restrict__ start, int64_t n,
-    double dt, int nsteps, int ka, int kb, double* __restrict__ rows) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  int s = start ? start[i] : 0;
+__device__ __forceinline__ void base_rows(const ssc_host_potential& hp, int block, char* lds_raw,
+                                          double* __restrict__ w, const int32_t* __restrict__ start,
+                                          int64_t n, double dt, int nsteps, int ka, int kb,
+                                          double* __restrict__ rows) {
+  const int lane = threadIdx.x & 63;
+  const int64_t i0 = (int64_t)block * PT_BLOCK + (threadIdx.x & ~63);  // the wave's first particle
+  const int64_t i = i0 + lane;
+  if (i0 >= n) return;  // whole waves only: the others keep together below
+  int s = i < n ? (start ? start[i] : 0) : nsteps;
   s = s < 0 ? 0 : (s > nsteps ? nsteps : s);
-  if (s >= nsteps || s > kb) return;
+  const bool moves = i < n && s < nsteps && s <= kb;
   double* wi = w + 6 * i;
-  double x = wi[0], y = wi[1], z = wi[2], vx = wi[3], vy = wi[4], vz = wi[5];
+  double x = 1.0, y = 0.0, z = 0.0, vx = 0.0, vy = 0.0, vz = 0.0;
+  if (moves) {
+    x = wi[0]; y = wi[1]; z = wi[2]; vx = wi[3]; vy = wi[4]; vz = wi[5];
+  }
+  int first = moves ? (ka > s ? ka : s) : INT_MAX;  // the wave's first row
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 64));
   const double h = 0.5 * dt;
-  for (int k = ka > s ? ka : s; k <= kb; ++k) {
-    if (k > s) {
+  double* buf = reinterpret_cast<double*>(lds_raw) + (threadIdx.x >> 6) * (64 * PR_REC);
+  const int64_t tail = (n - i0) * PR_REC;  // doubles of the wave's particles that exist
+  for (int k = first; k <= kb; ++k) {
+    const bool on = moves && k >= s;
+    if (on && k > s) {
       x += dt * vx; y += dt * vy; z += dt * vz;
     }
-    double g[3], H[9];
-    host_grad_hess<HS>(hp, x, y, z, g, H);
-    double* r = rows + ((int64_t)(k - ka) * n + i) * PR_REC;
-    r[0] = x; r[1] = y; r[2] = z;
-    r[3] = H[0]; r[4] = H[1]; r[5] = H[2]; r[6] = H[4]; r[7] = H[5]; r[8] = H[8];
-    const double c = (k == s || k == nsteps) ? h : dt;
-    vx -= c * g[0]; vy -= c * g[1]; vz -= c * g[2];
+    double g[3] = {0.0, 0.0, 0.0}, H[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) H[q] = 0.0;
+    host_quads<HS>(hp, x, y, z, g, H);
+    // records of particles that have not started are written and never read
+    double* b = buf + lane * PR_REC;
+    b[0] = x; b[1] = y; b[2] = z;
+    b[3] = H[0]; b[4] = H[1]; b[5] = H[2]; b[6] = H[4]; b[7] = H[5]; b[8] = H[8];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    double* r = rows + ((int64_t)(k - ka) * n + i0) * PR_REC;
+#pragma unroll
+    for (int e = 0; e < PR_REC; ++e) {
+      const int o = 64 * e + lane;
+      if (o < tail) r[o] = buf[o];
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (on) {
+      const double c = (k == s || k == nsteps) ? h : dt;
+      vx -= c * g[0]; vy -= c * g[1]; vz -= c * g[2];
+    }
   }
-  wi[0] = x; wi[1] = y; wi[2] = z; wi[3] = vx; wi[4] = vy; wi[5] = vz;
+  if (moves) {
+    wi[0] = x; wi[1] = y; wi[2] = z; wi[3] = vx; wi[4] = vy; wi[5] = vz;
+  }
 }
 
 // Responses in place in dw ([n][m][DD], initialised to dw0 or zeros) through rows [ka, kb].
 template <int SK, int G, int RAD>
-__global__ __launch_bounds__(PT_BLOCK) void perturb_rows_kernel(
-    ssc_sources pert, const double* __restrict__ rows, const int32_t* __restrict__ start,
-    int64_t n, int m, int L, double t0, double dt, int nsteps, int ka, int kb,
-    double* __restrict__ dw) {
-  extern __shared__ __align__(16) char lds_raw[];
-  __shared__ int kmin_sh;
+__device__ __forceinline__ void response_rows(const ssc_sources& pert, int block, char* lds_raw,
+                                              int& kmin_sh, const double* __restrict__ rows,
+                                              const int32_t* __restrict__ start, int64_t n, int m,
+                                              int L, double t0, double dt, int nsteps, int ka,
+                                              int kb, double* __restrict__ dw) {
   constexpr int DD = RAD ? 12 : 6;
   constexpr bool HQ = SK == SSC_SRC_LINE_HERNQUIST;
   constexpr bool FOLD = (SK == SSC_SRC_STATIC || SK == SSC_SRC_TRACK) && !RAD;
   const int ppb = PT_BLOCK / L;
   const int lp = threadIdx.x / L, grp = threadIdx.x - lp * L;
-  const int64_t i = (int64_t)blockIdx.x * ppb + lp;
+  const int64_t i = (int64_t)block * ppb + lp;
   const bool valid = lp < ppb && i < n;
   int s = nsteps;
   if (valid) {
@@ -282,6 +338,9 @@ __global__ __launch_bounds__(PT_BLOCK) void perturb_rows_kernel(
   for (int k = kfirst; k <= kb; ++k) {
     lds.stage(pert, k, nsteps + 1);
     if (!(moves && k >= s)) continue;
+    const double* r = rows + ((int64_t)(k - ka) * n + i) * PR_REC;
+    const double x = r[0], y = r[1], z = r[2];
+    const double H[9] = {r[3], r[4], r[5], r[4], r[6], r[7], r[5], r[7], r[8]};
     if (k > s) {
 #pragma unroll
       for (int q = 0; q < G; ++q)
@@ -291,15 +350,15 @@ __global__ __launch_bounds__(PT_BLOCK) void perturb_rows_kernel(
           if (RAD) rx[q][c] += dt * rv[q][c];
         }
     }
-    const double* r = rows + ((int64_t)(k - ka) * n + i) * PR_REC;
-    const double x = r[0], y = r[1], z = r[2];
-    const double H[9] = {r[3], r[4], r[5], r[4], r[6], r[7], r[5], r[7], r[8]};
     const double t = t0 + k * dt;
     const double c = (k == s || k == nsteps) ? h : dt;
     if constexpr (FOLD) {
       // Plummer sources that are always active: no branch per response, the folded
-      // reciprocal-square-root correction of plummer_grad_k, and the source force added into
-      // the Hessian product by one FMA per component
+      // reciprocal-square-root correction of plummer_grad_k, and the kick c folded into the
+      // Hessian (once a row) and the source's factor, so that a velocity component takes four
+      // FMAs: 28 instructions a response.  A slot beyond the last source computes a response
+      // that is never stored.
+      const double C[6] = {-c * H[0], -c * H[1], -c * H[2], -c * H[4], -c * H[5], -c * H[8]};
 #pragma unroll
       for (int q = 0; q < G; ++q) {
         const int j = grp + L * q;
@@ -309,14 +368,11 @@ __global__ __launch_bounds__(PT_BLOCK) void perturb_rows_kernel(
         const double s2 = fma(ex, ex, fma(ey, ey, fma(ez, ez, q2)));
         const double yr = __builtin_amdgcn_rsq(s2);
         const double y2 = yr * yr;
-        double f = yr * y2 * fma(s2 * y2, c1, c2);
-        f = j < m ? f : 0.0;
-        const double hx = fma(H[2], dx[q][2], fma(H[1], dx[q][1], H[0] * dx[q][0]));
-        const double hy = fma(H[5], dx[q][2], fma(H[4], dx[q][1], H[3] * dx[q][0]));
-        const double hz = fma(H[8], dx[q][2], fma(H[7], dx[q][1], H[6] * dx[q][0]));
-        dv[q][0] = fma(-c, fma(f, ex, hx), dv[q][0]);
-        dv[q][1] = fma(-c, fma(f, ey, hy), dv[q][1]);
-        dv[q][2] = fma(-c, fma(f, ez, hz), dv[q][2]);
+        const double f = (-c * yr) * y2 * fma(s2 * y2, c1, c2);
+        double* u = dx[q];
+        dv[q][0] = fma(f, ex, fma(C[2], u[2], fma(C[1], u[1], fma(C[0], u[0], dv[q][0]))));
+        dv[q][1] = fma(f, ey, fma(C[4], u[2], fma(C[3], u[1], fma(C[1], u[0], dv[q][1]))));
+        dv[q][2] = fma(f, ez, fma(C[5], u[2], fma(C[4], u[1], fma(C[2], u[0], dv[q][2]))));
       }
       continue;
     }
@@ -385,11 +441,47 @@ __global__ __launch_bounds__(PT_BLOCK) void perturb_rows_kernel(
   }
 }
 
+// One launch: base rows [na, nb_] of the next segment in the first bblocks blocks, the responses
+// of rows [ka, kb] in the others.
+template <int SK, int G, int RAD, int HS>
+__global__ __launch_bounds__(PT_BLOCK) void perturb_segment_kernel(
+    ssc_host_potential hp, ssc_sources pert, int bblocks, double* __restrict__ w,
+    const int32_t* __restrict__ start, int64_t n, int m, int L, double t0, double dt, int nsteps,
+    int ka, int kb, const double* __restrict__ rows, int na, int nb_,
+    double* __restrict__ next_rows, double* __restrict__ dw) {
+  extern __shared__ __align__(16) char lds_raw[];
+  __shared__ int kmin_sh;
+  if ((int)blockIdx.x < bblocks)
+    base_rows<HS>(hp, blockIdx.x, lds_raw, w, start, n, dt, nsteps, na, nb_, next_rows);
+  else
+    response_rows<SK, G, RAD>(pert, blockIdx.x - bblocks, lds_raw, kmin_sh, rows, start, n, m, L,
+                              t0, dt, nsteps, ka, kb, dw);
+}
+
+// Responses per lane of the split form: two while the lanes of eight would give the chip fewer than
+// two waves per SIMD, and with the radius block always (twelve numbers a response: 118 registers
+// with two, 374 and one wave per SIMD with eight); eight otherwise, since a lane's row record and
+// Hessian then serve eight responses.  Up to 512 sources with two (256 lanes a particle).
+// Measured (ms, 2 / 4 / 8 a lane): 80,000 particles x 64 sources, 4,000 steps 26.1 / 22.8 / 21.0,
+// with the radius block 40.0 / 40.5 / 54.3; 40,000 x 64, 2,000 steps 8.0 / 7.1 / 6.7; 8,100 x 33,
+// 900 steps 2.00 / 2.08 / 2.33; 1,000 x 7, 500 steps 1.09 / 1.17 / 1.33.
+static bool split_few(int64_t n, int m, bool radius) {
+  if (m > 2 * PT_BLOCK) return false;
+  int L = 1;
+  while (8 * L < m) L <<= 1;
+  return radius || n * L < (int64_t)2 * 1024 * 64;
+}
+
 // Rows per segment that fit in workspace_bytes (0 when not even one does).
 static int64_t perturb_segment_rows(int64_t n, int nsteps, int64_t workspace_bytes) {
   const int64_t per_row = n * PR_REC * 8;
   const int64_t e = per_row > 0 ? workspace_bytes / per_row : 0;
   return e < (int64_t)nsteps + 1 ? e : (int64_t)nsteps + 1;
+}
+
+// Segments take turns in the two halves of a workspace that holds at least two rows but not all.
+static int64_t perturb_buffer_rows(int64_t E, int nsteps) {
+  return E > nsteps || E < 2 ? E : E / 2;
 }
 
 template <int SK, int G, int RAD, int HS>
@@ -403,9 +495,9 @@ static int launch_perturb_split(const ssc_host_potential& hp, const ssc_sources&
   int Lp = 1;
   while (Lp < L) Lp <<= 1;
   if (Lp > PT_BLOCK) return fail(SSC_E_LIMIT, "ssc_perturb_leapfrog: too many sources");
-  const size_t lds = SourceLDS<SK>::bytes(pert);
+  const size_t lds = std::max<size_t>(SourceLDS<SK>::bytes(pert), BASE_LDS);
   if (lds > 60 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)perturb_rows_kernel<SK, G, RAD>,
+    hipError_t e = hipFuncSetAttribute((const void*)perturb_segment_kernel<SK, G, RAD, HS>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return fail(SSC_E_HIP, std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
   }
@@ -415,14 +507,29 @@ static int launch_perturb_split(const ssc_host_potential& hp, const ssc_sources&
   else
     hipLaunchKernelGGL(pt_zero_kernel, dim3((unsigned)((n * m * DD + 255) / 256)), dim3(256), 0,
                        st, dw_out, n * m * DD);
-  const unsigned bblocks = (unsigned)((n + 255) / 256);
+  const unsigned bblocks = (unsigned)((n + PT_BLOCK - 1) / PT_BLOCK);
   const unsigned rblocks = (unsigned)((n + PT_BLOCK / Lp - 1) / (PT_BLOCK / Lp));
-  for (int64_t ka = 0; ka <= nsteps; ka += E) {
-    const int kb = (int)std::min<int64_t>(ka + E - 1, nsteps);
-    hipLaunchKernelGGL((perturb_base_kernel<HS>), dim3(bblocks), dim3(256), 0, st, hp, w_out,
-                       start, n, dt, nsteps, (int)ka, kb, rows);
-    hipLaunchKernelGGL((perturb_rows_kernel<SK, G, RAD>), dim3(rblocks), dim3(PT_BLOCK), lds, st,
-                       pert, rows, start, n, m, Lp, t0, dt, nsteps, (int)ka, kb, dw_out);
+  const int64_t B = perturb_buffer_rows(E, nsteps);
+  double* buf[2] = {rows, B < E ? rows + B * n * PR_REC : rows};
+  auto launch = [&](unsigned nb, unsigned nr, int64_t ka, int64_t kb, const double* cur,
+                    int64_t na, int64_t nbk, double* next) {
+    hipLaunchKernelGGL((perturb_segment_kernel<SK, G, RAD, HS>), dim3(nb + nr), dim3(PT_BLOCK), lds,
+                       st, hp, pert, (int)nb, w_out, start, n, m, Lp, t0, dt, nsteps, (int)ka,
+                       (int)kb, cur, (int)na, (int)nbk, next, dw_out);
+  };
+  auto last = [&](int64_t ka) { return std::min<int64_t>(ka + B - 1, nsteps); };
+  launch(bblocks, 0, 0, 0, buf[0], 0, last(0), buf[0]);
+  int cur = 0;
+  for (int64_t ka = 0; ka <= nsteps; ka += B) {
+    const int64_t na = ka + B;
+    const bool more = na <= nsteps;
+    if (more && buf[0] != buf[1]) {
+      launch(bblocks, rblocks, ka, last(ka), buf[cur], na, last(na), buf[cur ^ 1]);
+      cur ^= 1;
+    } else {
+      launch(0, rblocks, ka, last(ka), buf[cur], 0, 0, nullptr);
+      if (more) launch(bblocks, 0, 0, 0, buf[cur], na, last(na), buf[cur]);
+    }
   }
   return check_launch("ssc_perturb_leapfrog");
 }
@@ -456,7 +563,7 @@ using namespace ssc;
 extern "C" int64_t ssc_perturb_workspace_bytes(int64_t n, int32_t nsteps) {
   if (n <= 0 || nsteps < 0) return 0;
   const int64_t per_row = n * PR_REC * 8;
-  int64_t e = ((int64_t)1 << 31) / per_row;  // rows of at most 2 GiB per segment
+  int64_t e = ((int64_t)1 << 32) / per_row;  // two segments of rows of at most 2 GiB each
   if (e < 1) e = 1;
   if (e > (int64_t)nsteps + 1) e = (int64_t)nsteps + 1;
   return e * per_row;
@@ -488,9 +595,12 @@ extern "C" int ssc_perturb_leapfrog(const ssc_host_potential* host, const ssc_so
     if (w_out == w0 || (dw0 && dw_out == dw0))
       return fail(SSC_E_ARG, "ssc_perturb_leapfrog: outputs must not alias the inputs");
   }
+  const bool few = split_few(n, s.n, with_radius != 0);
+#define SSC_PTS(K, G, R, H)                                                                      \
+  launch_perturb_split<K, G, R, H>(*host, s, w0, dw0, start_step, n, t0, dt, nsteps, w_out,       \
+                                   dw_out, (double*)workspace, E, st)
 #define SSC_PT3(K, R, H)                                                                        \
-  (E > 0 ? launch_perturb_split<K, 8, R, H>(*host, s, w0, dw0, start_step, n, t0, dt, nsteps,    \
-                                            w_out, dw_out, (double*)workspace, E, st)           \
+  (E > 0 ? (few ? SSC_PTS(K, 2, R, H) : SSC_PTS(K, (R ? 4 : 8), R, H))                           \
          : launch_perturb<K, 8, R, H>(*host, s, w0, dw0, start_step, n, t0, dt, nsteps, w_out,  \
                                       dw_out, st))
 #define SSC_PT(K, R)                                                                 \
@@ -514,5 +624,6 @@ extern "C" int ssc_perturb_leapfrog(const ssc_host_potential* host, const ssc_so
   }
 #undef SSC_PT
 #undef SSC_PT3
+#undef SSC_PTS
   return fail(SSC_E_ARG, "ssc_perturb_leapfrog: bad source kind");
 }
