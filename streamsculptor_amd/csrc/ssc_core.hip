@@ -600,25 +600,48 @@ static int set_lds(const void* fn, size_t lds) {
   return SSC_OK;
 }
 
-// Launch shape: one wave per orbit for a handful of orbits in a large source table; two
-// particles per lane once the batch alone fills the chip; G lanes per orbit for mid-sized
-// batches with sources; for up to 65536 orbits in a host of no known signature, host components
-// over waves; one particle per lane otherwise (with straight-line host code for the known
-// hosts, which is faster still).
+// Lanes per orbit: the G of 1 ... 16 with the smallest estimate of a step's time.  A step lasts
+// as long as the SIMD with the most waves, w = ceil(n G / 65536), and about a quarter of a wave's
+// time on top (its chain of dependent instructions, not overlapped); a wave's time is its share
+// of the sources plus the host terms and log2 G exchanges, worth 4 + 3 log2 G sources.  The
+// whole-number w is what matters: at 1e5 orbits two lanes need 3.05 -> 4 waves' time and one
+// lane 1.5 -> 2.  Measured per step, the previous rule (three waves per SIMD wanted) -> this one,
+// 64 tracked subhalos: 12,500 orbits 2.44 -> 1.54 us (16 -> 4 lanes), 25,000 3.13 -> 2.39 (8 -> 2),
+// 50,000 4.41 -> 4.09 (4 -> 1), 100,000 7.21 -> 6.53 (2 -> 1); 512 static clumps: 10,000
+// 6.85 -> 6.80, 25,000 14.5 -> 14.1, 200,000 90.7 -> 84.8 (1 -> 4), 400,000 169 -> 153.
+inline int leapfrog_lanes(int64_t n, int nsrc) {
+  int best = 1;
+  double least = 0.0;
+  for (int lg = 0; lg <= 4; ++lg) {
+    const int64_t g = 1 << lg, waves = (n * g + 65535) / 65536;
+    const double cost = (4.0 * waves + 1.0) * (double)((nsrc + g - 1) / g + 4 + 3 * lg);
+    if (lg == 0 || cost <= least) { least = cost; best = (int)g; }
+  }
+  return best;
+}
+
+// Launch shape: one wave per orbit while every orbit has a SIMD of its own and the table is
+// large (512 clumps: 1,000 orbits 1.81 us a step against 2.87 with 16 lanes an orbit, 2,000
+// orbits 4.39 against 2.96); two particles per lane for batches that fill the chip several times
+// over, unless the pairing costs a round of waves (512 clumps: 1e6 orbits 326 us against 331,
+// 4e5 169 against 153); leapfrog_lanes otherwise.  Without sources: for up to 65536 orbits in a
+// host of no known signature, host components over waves; one particle per lane otherwise (with
+// straight-line host code for the known hosts, which is faster still).
 template <int SK, int HS>
 static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src, const double* w0,
                            const int32_t* start, int64_t n, double t0, double dt, int nsteps,
                            double* w_out, const int32_t* save_idx, int nsave, double* ys,
                            hipStream_t st) {
   const size_t lds = SourceLDS<SK>::bytes(src);
-  if (SK != SSC_SRC_NONE && src.n >= 64 && n <= 8192) {
+  if (SK != SSC_SRC_NONE && src.n >= 64 && n <= 1024) {
     int rc = set_lds((const void*)leapfrog_wave_kernel<SK, HS>, lds);
     if (rc) return rc;
     hipLaunchKernelGGL((leapfrog_wave_kernel<SK, HS>), dim3((unsigned)n), dim3(WAVE), lds, st, hp, src,
                        w0, start, n, t0, dt, nsteps, w_out, save_idx, nsave, ys);
     return check_launch("ssc_leapfrog");
   }
-  if (SK != SSC_SRC_NONE && src.n >= 16 && n >= 393216) {
+  if (SK != SSC_SRC_NONE && src.n >= 16 && n >= 393216 &&
+      2 * ((n + 131071) / 131072) <= (n + 65535) / 65536) {
     int rc = set_lds((const void*)leapfrog_kernel<SK, 2, HS>, lds);
     if (rc) return rc;
     const int64_t blocks = (n + 2 * LF_BLOCK - 1) / (2 * LF_BLOCK);
@@ -633,7 +656,7 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                        w_out, save_idx, nsave, ys);
     return check_launch("ssc_leapfrog");
   }
-  const int g = SK == SSC_SRC_NONE ? 1 : group_lanes(n, src.n);
+  const int g = SK == SSC_SRC_NONE ? 1 : leapfrog_lanes(n, src.n);
 #define SSC_GROUP(GV)                                                                              \
   if (g == GV) {                                                                                   \
     int rc = set_lds((const void*)leapfrog_group_kernel<SK, GV, HS>, lds);                            \

@@ -75,13 +75,25 @@ struct SourceLDS<SSC_SRC_STATIC> {
   template <int P>
   __device__ void add_grad(int, double, const double* x, const double* y, const double* z,
                            double* gx, double* gy, double* gz, int j0, int js) const {
-    for (int j = j0; j < n; j += js) {
-      const SrcGeo g = geo[j];
-      const SrcK c = kc[j];
+    auto term = [&](const SrcGeo& g, const SrcK& c) {
 #pragma unroll
       for (int p = 0; p < P; ++p)
         plummer_grad_k(x[p] - g.x, y[p] - g.y, z[p] - g.z, g.rs2, c.c1, c.c2, gx[p], gy[p], gz[p]);
+    };
+    // four sources at a time, in order (see TrackLDS)
+    int j = j0;
+    for (; j + 3 * js < n; j += 4 * js) {
+      SrcGeo g[4];
+      SrcK c[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        g[u] = geo[j + u * js];
+        c[u] = kc[j + u * js];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) term(g[u], c[u]);
     }
+    for (; j < n; j += js) term(geo[j], kc[j]);
   }
   __device__ bool get(int, double, int j, double& sx, double& sy, double& sz, double& gm,
                       double& q) const {
@@ -173,9 +185,7 @@ struct TrackLDS {
   __device__ void add_grad(int k, double, const double* x, const double* y, const double* z,
                            double* gx, double* gy, double* gz, int j0, int js) const {
     const SrcGeo* row = rec + (k - kb) * n;
-    for (int j = j0; j < n; j += js) {
-      const SrcGeo g = row[j];
-      const SrcK c = kc[j];
+    auto term = [&](const SrcGeo& g, const SrcK& c, int j) {
 #pragma unroll
       for (int p = 0; p < P; ++p) {
         if (HQ)
@@ -184,7 +194,22 @@ struct TrackLDS {
           plummer_grad_k(x[p] - g.x, y[p] - g.y, z[p] - g.z, g.rs2, c.c1, c.c2, gx[p], gy[p],
                          gz[p]);
       }
+    };
+    // four sources at a time, in order: their reads are in flight together and their chains
+    // interleave (one source per iteration waited for its LDS reads and its 15-instruction chain)
+    int j = j0;
+    for (; j + 3 * js < n; j += 4 * js) {
+      SrcGeo g[4];
+      SrcK c[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        g[u] = row[j + u * js];
+        c[u] = kc[j + u * js];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) term(g[u], c[u], j + u * js);
     }
+    for (; j < n; j += js) term(row[j], kc[j], j);
   }
   __device__ bool get(int k, double, int j, double& sx, double& sy, double& sz, double& gm,
                       double& q) const {
