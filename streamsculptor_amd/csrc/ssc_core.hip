@@ -2,6 +2,7 @@
 // stream kernel (one particle per lane, FP64 state in VGPRs, Plummer source tables in LDS).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstdio>
 #include <cstring>
@@ -609,11 +610,17 @@ static int set_lds(const void* fn, size_t lds) {
 // 64 tracked subhalos: 12,500 orbits 2.44 -> 1.54 us (16 -> 4 lanes), 25,000 3.13 -> 2.39 (8 -> 2),
 // 50,000 4.41 -> 4.09 (4 -> 1), 100,000 7.21 -> 6.53 (2 -> 1); 512 static clumps: 10,000
 // 6.85 -> 6.80, 25,000 14.5 -> 14.1, 200,000 90.7 -> 84.8 (1 -> 4), 400,000 169 -> 153.
-inline int leapfrog_lanes(int64_t n, int nsrc) {
+// Orbits that start all along the grid (`ragged`) fill the SIMDs unevenly whatever G is, and each
+// wave ends when its latest block's work does: half the waves' work, not rounded up, but at least
+// one wave's (1e5 orbits of one stream, 64 tracked subhalos, 4,000 rows: two lanes 13.8 ms, one
+// lane 16.3 ms).
+inline int leapfrog_lanes(int64_t n, int nsrc, bool ragged) {
   int best = 1;
   double least = 0.0;
   for (int lg = 0; lg <= 4; ++lg) {
-    const int64_t g = 1 << lg, waves = (n * g + 65535) / 65536;
+    const int64_t g = 1 << lg;
+    const double waves = ragged ? std::max(1.0, n * g / 131072.0)
+                                : (double)((n * g + 65535) / 65536);
     const double cost = (4.0 * waves + 1.0) * (double)((nsrc + g - 1) / g + 4 + 3 * lg);
     if (lg == 0 || cost <= least) { least = cost; best = (int)g; }
   }
@@ -630,7 +637,7 @@ inline int leapfrog_lanes(int64_t n, int nsrc) {
 template <int SK, int HS>
 static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src, const double* w0,
                            const int32_t* start, int64_t n, double t0, double dt, int nsteps,
-                           double* w_out, const int32_t* save_idx, int nsave, double* ys,
+                           double* w_out, const int32_t* save_idx, int nsave, double* ys, bool ragged,
                            hipStream_t st) {
   const size_t lds = SourceLDS<SK>::bytes(src);
   if (SK != SSC_SRC_NONE && src.n >= 64 && n <= 1024) {
@@ -656,7 +663,7 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                        w_out, save_idx, nsave, ys);
     return check_launch("ssc_leapfrog");
   }
-  const int g = SK == SSC_SRC_NONE ? 1 : leapfrog_lanes(n, src.n);
+  const int g = SK == SSC_SRC_NONE ? 1 : leapfrog_lanes(n, src.n, ragged);
 #define SSC_GROUP(GV)                                                                              \
   if (g == GV) {                                                                                   \
     int rc = set_lds((const void*)leapfrog_group_kernel<SK, GV, HS>, lds);                            \
@@ -682,6 +689,42 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
 }  // namespace ssc
 
 using namespace ssc;
+
+int ssc::leapfrog_run(const ssc_host_potential* host, const ssc_sources* src, const double* w0,
+                      const int32_t* start_step, int64_t n, double t0, double dt, int32_t nsteps,
+                      double* w_out, const int32_t* save_idx, int32_t nsave, double* ys,
+                      bool ragged, void* stream) {
+  int rc = validate_host(host);
+  if (rc) return rc;
+  if (n < 0 || nsteps < 0 || nsave < 0) return fail(SSC_E_ARG, "ssc_leapfrog: negative size");
+  if (n == 0) return SSC_OK;
+  if (!w0 || !w_out) return fail(SSC_E_ARG, "ssc_leapfrog: w0 or w_out is NULL");
+  if (nsave > 0 && (!save_idx || !ys)) return fail(SSC_E_ARG, "ssc_leapfrog: nsave > 0 needs save_idx and ys");
+  if (nsave == 0) { save_idx = nullptr; ys = nullptr; }
+  if ((n + LF_BLOCK - 1) / LF_BLOCK > (int64_t)INT_MAX)
+    return fail(SSC_E_LIMIT, "ssc_leapfrog: too many particles");
+  rc = validate_sources(src, nsteps);
+  if (rc) return rc;
+  ssc_sources s = src ? *src : empty_sources();
+  if (s.n == 0) s.kind = SSC_SRC_NONE;
+  hipStream_t st = (hipStream_t)stream;
+  const int hs = host_signature(*host);
+#define SSC_LF3(K, H) launch_leapfrog<K, H>(*host, s, w0, start_step, n, t0, dt, nsteps, w_out, save_idx, nsave, ys, ragged, st)
+#define SSC_LF(K)                                                                                 \
+  (hs == HS_MN_HQ_NFW ? SSC_LF3(K, HS_MN_HQ_NFW)                                                 \
+                      : (hs == HS_MN_HQ_HQ_NFW ? SSC_LF3(K, HS_MN_HQ_HQ_NFW) : SSC_LF3(K, HS_GENERIC)))
+  switch (s.kind) {
+    case SSC_SRC_NONE: return SSC_LF(SSC_SRC_NONE);
+    case SSC_SRC_STATIC: return SSC_LF(SSC_SRC_STATIC);
+    case SSC_SRC_TRACK: return SSC_LF(SSC_SRC_TRACK);
+    case SSC_SRC_LINE: return SSC_LF(SSC_SRC_LINE);
+    case SSC_SRC_LINE_HERNQUIST: return SSC_LF(SSC_SRC_LINE_HERNQUIST);
+    case SSC_SRC_TRACK_HERNQUIST: return SSC_LF(SSC_SRC_TRACK_HERNQUIST);
+    default: return fail(SSC_E_ARG, "ssc_leapfrog: bad source kind");
+  }
+#undef SSC_LF
+#undef SSC_LF3
+}
 
 extern "C" {
 
@@ -723,36 +766,8 @@ int ssc_leapfrog(const ssc_host_potential* host, const ssc_sources* src, const d
                  const int32_t* start_step, int64_t n, double t0, double dt, int32_t nsteps,
                  double* w_out, const int32_t* save_idx, int32_t nsave, double* ys,
                  void* stream) {
-  int rc = validate_host(host);
-  if (rc) return rc;
-  if (n < 0 || nsteps < 0 || nsave < 0) return fail(SSC_E_ARG, "ssc_leapfrog: negative size");
-  if (n == 0) return SSC_OK;
-  if (!w0 || !w_out) return fail(SSC_E_ARG, "ssc_leapfrog: w0 or w_out is NULL");
-  if (nsave > 0 && (!save_idx || !ys)) return fail(SSC_E_ARG, "ssc_leapfrog: nsave > 0 needs save_idx and ys");
-  if (nsave == 0) { save_idx = nullptr; ys = nullptr; }
-  if ((n + LF_BLOCK - 1) / LF_BLOCK > (int64_t)INT_MAX)
-    return fail(SSC_E_LIMIT, "ssc_leapfrog: too many particles");
-  rc = validate_sources(src, nsteps);
-  if (rc) return rc;
-  ssc_sources s = src ? *src : empty_sources();
-  if (s.n == 0) s.kind = SSC_SRC_NONE;
-  hipStream_t st = (hipStream_t)stream;
-  const int hs = host_signature(*host);
-#define SSC_LF3(K, H) launch_leapfrog<K, H>(*host, s, w0, start_step, n, t0, dt, nsteps, w_out, save_idx, nsave, ys, st)
-#define SSC_LF(K)                                                                                 \
-  (hs == HS_MN_HQ_NFW ? SSC_LF3(K, HS_MN_HQ_NFW)                                                 \
-                      : (hs == HS_MN_HQ_HQ_NFW ? SSC_LF3(K, HS_MN_HQ_HQ_NFW) : SSC_LF3(K, HS_GENERIC)))
-  switch (s.kind) {
-    case SSC_SRC_NONE: return SSC_LF(SSC_SRC_NONE);
-    case SSC_SRC_STATIC: return SSC_LF(SSC_SRC_STATIC);
-    case SSC_SRC_TRACK: return SSC_LF(SSC_SRC_TRACK);
-    case SSC_SRC_LINE: return SSC_LF(SSC_SRC_LINE);
-    case SSC_SRC_LINE_HERNQUIST: return SSC_LF(SSC_SRC_LINE_HERNQUIST);
-    case SSC_SRC_TRACK_HERNQUIST: return SSC_LF(SSC_SRC_TRACK_HERNQUIST);
-    default: return fail(SSC_E_ARG, "ssc_leapfrog: bad source kind");
-  }
-#undef SSC_LF
-#undef SSC_LF3
+  return leapfrog_run(host, src, w0, start_step, n, t0, dt, nsteps, w_out, save_idx, nsave, ys,
+                      false, stream);
 }
 
 }  // extern "C"

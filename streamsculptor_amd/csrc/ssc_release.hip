@@ -1,9 +1,10 @@
-// Spray-stream release conditions on the GPU: one release per lane.  Restates the reference
+// Spray-stream release conditions on the GPU.  Restates the reference
 // Potential.release_model (streamsculptor/main.py:209-280) with the closed-form host Hessian
 // in place of nested autodiff, and the reference's key scheme on a Threefry-2x32-20 counter
 // PRNG (Salmon et al., SC'11) for the Gaussian offsets.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -98,35 +99,47 @@ struct ReleaseFrame {
   double x[3], v[3], rh[3], zh[3], ph[3], rt, relv;
 };
 
-// Release i happens at time t_rel[i] (LINE sources) and source-table row step_rel[i] (TRACK
-// sources); the point sources add their Hessian to the host's, since the reference takes
-// d2phidr2 of the whole potential.  A TRACK row outside the table gives NaN rows.
-__device__ void release_frame(const ssc_host_potential& hp, const ssc_sources& src,
-                              const double* __restrict__ prog_w, const double* __restrict__ t_rel,
-                              const int32_t* __restrict__ step_rel,
-                              const double* __restrict__ g_msat, int i, ReleaseFrame& f) {
+// The point sources' part of the Hessian at release i, which happens at time t_rel[i] (LINE
+// sources) and source-table row step_rel[i] (TRACK sources): LANES lanes, lane `lane` of them
+// every LANES-th source, the sums (six distinct entries) in every lane.  A TRACK row outside the
+// table gives NaN, and so NaN rows.
+template <int LANES>
+__device__ void release_sources(const ssc_sources& src, const double* __restrict__ prog_w,
+                                const double* __restrict__ t_rel,
+                                const int32_t* __restrict__ step_rel, int i, int lane, double* S) {
+  const double* w = prog_w + 6 * (int64_t)i;
+  const int step = step_rel ? step_rel[i] : 0;
+  const double t = t_rel ? t_rel[i] : 0.0;
+  const bool outside = (src.kind == SSC_SRC_TRACK || src.kind == SSC_SRC_TRACK_HERNQUIST) &&
+                       (step < 0 || step >= src.n_track);
+  double phi = 0.0, g[3] = {}, H[9] = {};
+  for (int j = outside ? src.n : lane; j < src.n; j += LANES) {
+    double sx, sy, sz;
+    if (!source_position(src, j, step, t, sx, sy, sz)) continue;
+    const double rs = src.rs[j];
+    if (src.kind == SSC_SRC_LINE_HERNQUIST || src.kind == SSC_SRC_TRACK_HERNQUIST)
+      hernquist_full(w[0] - sx, w[1] - sy, w[2] - sz, src.gm[j], rs, phi, g, H);
+    else
+      plummer_full(w[0] - sx, w[1] - sy, w[2] - sz, src.gm[j], rs * rs, phi, g, H);
+  }
+  constexpr int at[6] = {0, 1, 2, 4, 5, 8};
+#pragma unroll
+  for (int k = 0; k < 6; ++k) S[k] = outside ? __builtin_nan("") : group_sum<LANES>(H[at[k]]);
+}
+
+// The frame of release i; S, if any, is the point sources' Hessian, which is added to the host's,
+// since the reference takes d2phidr2 of the whole potential.
+__device__ void release_frame(const ssc_host_potential& hp, const double* __restrict__ prog_w,
+                              const double* __restrict__ g_msat, int i, const double* S,
+                              ReleaseFrame& f) {
   const double* w = prog_w + 6 * (int64_t)i;
   const double x[3] = {w[0], w[1], w[2]}, v[3] = {w[3], w[4], w[5]};
   double phi, g[3], H[9];
   host_full(hp, x[0], x[1], x[2], phi, g, H);
-  if (src.kind != SSC_SRC_NONE) {
-    const int step = step_rel ? step_rel[i] : 0;
-    const double t = t_rel ? t_rel[i] : 0.0;
-    if ((src.kind == SSC_SRC_TRACK || src.kind == SSC_SRC_TRACK_HERNQUIST) &&
-        (step < 0 || step >= src.n_track)) {
-#pragma unroll
-      for (int k = 0; k < 9; ++k) H[k] = __builtin_nan("");
-    } else {
-      for (int j = 0; j < src.n; ++j) {
-        double sx, sy, sz;
-        if (!source_position(src, j, step, t, sx, sy, sz)) continue;
-        const double rs = src.rs[j];
-        if (src.kind == SSC_SRC_LINE_HERNQUIST || src.kind == SSC_SRC_TRACK_HERNQUIST)
-          hernquist_full(x[0] - sx, x[1] - sy, x[2] - sz, src.gm[j], rs, phi, g, H);
-        else
-          plummer_full(x[0] - sx, x[1] - sy, x[2] - sz, src.gm[j], rs * rs, phi, g, H);
-      }
-    }
+  if (S) {
+    H[0] += S[0]; H[1] += S[1]; H[2] += S[2];
+    H[3] += S[1]; H[4] += S[3]; H[5] += S[4];
+    H[6] += S[2]; H[7] += S[4]; H[8] += S[5];
   }
   const double rad = sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
   const double rh[3] = {x[0] / rad, x[1] / rad, x[2] / rad};
@@ -157,75 +170,104 @@ __device__ void release_frame(const ssc_host_potential& hp, const ssc_sources& s
   }
 }
 
-// The two released rows of frame f with release index ridx and seed: Gaussian multipliers
-// with keys PRNGKey(ridx * r_k) (main.py:220-228,263-266); trailing arm = far, leading arm =
-// close (main.py:269-278).  pc/pf/vc/vf may alias the strided slots of one output row.
-__device__ void release_rows(const ReleaseFrame& f, int64_t ridx, int64_t seed, const KVals& kv,
-                             double* pc, double* pf, double* vc, double* vf) {
+// One of the two released rows' four vectors of frame f, release index ridx and seed, by four
+// consecutive lanes: lane q of them draws Gaussian multiplier q (key PRNGKey(ridx * r_q), main.py:
+// 220-228,263-266) and gets the others' by shuffles, then forms the close position, far position,
+// close velocity or far velocity (trailing arm = far, leading arm = close; main.py:269-278).
+__device__ void release_vector(const ReleaseFrame& f, int64_t ridx, int64_t seed, const KVals& kv,
+                               int q, double* o) {
+  // products and sums in the roundings written here, whatever is inlined around them
+#pragma clang fp contract(off)
+  const double z = prng_normal(ridx * randint1000(seed, q));
   double zr[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) zr[k] = prng_normal(ridx * randint1000(seed, k));
-  const double kr = kv.k[0] + zr[0] * kv.k[4];
-  const double kvphi = kr * (kv.k[1] + zr[1] * kv.k[5]);
-  const double kz = kv.k[2] + zr[2] * kv.k[6];
-  const double kvz = kv.k[3] + zr[3] * kv.k[7];
+  for (int k = 0; k < 4; ++k) zr[k] = __shfl(z, k, 4);
+  const double kr = fma(zr[0], kv.k[4], kv.k[0]);
+  const double kvphi = kr * fma(zr[1], kv.k[5], kv.k[1]);
+  const double kz = fma(zr[2], kv.k[6], kv.k[2]);
+  const double kvz = fma(zr[3], kv.k[7], kv.k[3]);
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    const double ptr = f.x[a] + kr * f.rh[a] * f.rt + f.zh[a] * kz * f.rt;
+    const double pr = kr * f.rh[a], pz = f.zh[a] * kz;
+    const double ptr = fma(pz, f.rt, fma(pr, f.rt, f.x[a]));
     const double vtr = f.v[a] + kvphi * f.relv * f.ph[a] + kvz * f.relv * f.zh[a];
-    const double pld = f.x[a] - kr * f.rh[a] * f.rt - f.zh[a] * kz * f.rt;
+    const double pld = fma(-pz, f.rt, fma(-pr, f.rt, f.x[a]));
     const double vld = f.v[a] - kvphi * f.relv * f.ph[a] - kvz * f.relv * f.zh[a];
-    pc[a] = pld;
-    pf[a] = ptr;
-    vc[a] = vld;
-    vf[a] = vtr;
+    o[a] = q == 0 ? pld : (q == 1 ? ptr : (q == 2 ? vld : vtr));
   }
 }
 
-__global__ __launch_bounds__(256) void release_kernel(ssc_host_potential hp, ssc_sources src,
-                                                      const double* __restrict__ prog_w,
-                                                      const int32_t* __restrict__ rel_idx,
-                                                      const double* __restrict__ t_rel,
-                                                      const int32_t* __restrict__ step_rel,
-                                                      const double* __restrict__ g_msat, int nrel,
-                                                      int64_t seed, KVals kv,
-                                                      double* __restrict__ pos_close,
-                                                      double* __restrict__ pos_far,
-                                                      double* __restrict__ vel_close,
-                                                      double* __restrict__ vel_far) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nrel) return;
-  ReleaseFrame f;
-  release_frame(hp, src, prog_w, t_rel, step_rel, g_msat, i, f);
-  const int64_t ridx = rel_idx ? (int64_t)rel_idx[i] : (int64_t)i;
-  const int64_t o = 3 * (int64_t)i;
-  release_rows(f, ridx, seed, kv, pos_close + o, pos_far + o, vel_close + o, vel_far + o);
-}
+// Where the vectors of (seed s, release i) go: v[q] + s * seed + i * row doubles.
+struct ReleaseOut {
+  double* v[4];  // close position, far position, close velocity, far velocity
+  int64_t seed, row;
+};
 
-// nseed seeds of the same releases: a block forms the frames of RS_REL releases once (the
-// tidal radius needs the Hessian of the whole potential, a sum over every point source), then
-// its threads draw the rows of every (release, seed) pair from them.
-// rows[s][arm][i][6] = (position, velocity), arm 0 = close (leading), 1 = far (trailing).
-constexpr int RS_REL = 32;
-__global__ __launch_bounds__(256) void release_seeds_kernel(
+// nseed seeds of nrel releases.  A launch of some hundred releases is latency: one lane per
+// release walked the source table alone and drew its four normals (a Threefry, a logarithm and
+// three error functions each) in turn.  Here L lanes sum a release's sources (64 lanes for large
+// tables, 16 for small ones, L = 1: no sources), a block of R releases keeps the sums and the
+// frames in LDS (one lane each forms a frame, so that the host terms are not repeated), and four
+// lanes draw each (release, seed).  500 releases x 100 seeds among 512 clumps 29 us (318 before,
+// and 3.8 ms beside a launch that fills the chip), 500 x 1 in the host alone 12.5 us (19.6),
+// 20,000 x 4 among 512 clumps 70 us (178).  Blocks of the same releases share the seeds (grid y).
+constexpr int release_block(int lanes) { return lanes == 64 ? 8 : 16; }
+template <int L>
+__global__ __launch_bounds__(256) void release_kernel(
     ssc_host_potential hp, ssc_sources src, const double* __restrict__ prog_w,
     const int32_t* __restrict__ rel_idx, const double* __restrict__ t_rel,
     const int32_t* __restrict__ step_rel, const double* __restrict__ g_msat, int nrel,
-    int64_t seed0, int nseed, KVals kv, double* __restrict__ rows) {
-  __shared__ ReleaseFrame fr[RS_REL];
-  const int i0 = blockIdx.x * RS_REL;
-  const int nb = min(RS_REL, nrel - i0);
-  if ((int)threadIdx.x < nb)
-    release_frame(hp, src, prog_w, t_rel, step_rel, g_msat, i0 + threadIdx.x, fr[threadIdx.x]);
-  __syncthreads();
-  const int64_t arm = (int64_t)nrel * 6, seed_stride = 2 * arm;
-  for (int it = threadIdx.x; it < nb * nseed; it += blockDim.x) {
-    const int r = it % nb, s = it / nb, i = i0 + r;
-    const int64_t ridx = rel_idx ? (int64_t)rel_idx[i] : (int64_t)i;
-    double* close = rows + s * seed_stride + 6 * (int64_t)i;
-    double* far = close + arm;
-    release_rows(fr[r], ridx, seed0 + s, kv, close, far, close + 3, far + 3);
+    int64_t seed0, int nseed, KVals kv, ReleaseOut out) {
+  constexpr int R = release_block(L), SEEDS = 64 / R;  // releases, seeds a block draws at once
+  __shared__ ReleaseFrame fr[R];
+  __shared__ double sums[R][6];
+  const int64_t i0 = (int64_t)blockIdx.x * R;
+  const int nb = (int)(nrel - i0 < R ? nrel - i0 : R);
+  if (L > 1) {
+    for (int r = threadIdx.x / L; r < R; r += 256 / L) {  // whole waves: R L is a multiple of 256
+      double S[6];
+      release_sources<L>(src, prog_w, t_rel, step_rel, (int)i0 + (r < nb ? r : nb - 1),
+                         threadIdx.x % L, S);
+      if (threadIdx.x % L == 0)
+        for (int k = 0; k < 6; ++k) sums[r][k] = S[k];
+    }
+    __syncthreads();
   }
+  if ((int)threadIdx.x < nb)
+    release_frame(hp, prog_w, g_msat, (int)i0 + threadIdx.x, L > 1 ? sums[threadIdx.x] : nullptr,
+                  fr[threadIdx.x]);
+  __syncthreads();
+  const int q = threadIdx.x & 3, r = (threadIdx.x >> 2) % R;
+  const int64_t i = i0 + r;
+  if (i >= nrel) return;
+  const int64_t ridx = rel_idx ? (int64_t)rel_idx[i] : i;
+  const ReleaseFrame f = fr[r];
+  double* const base = out.v[q] + i * out.row;
+  for (int64_t s = (int64_t)blockIdx.y * SEEDS + (threadIdx.x >> 2) / R; s < nseed;
+       s += (int64_t)gridDim.y * SEEDS) {
+    double o[3];
+    release_vector(f, ridx, seed0 + s, kv, q, o);
+    double* w = base + s * out.seed;
+    w[0] = o[0]; w[1] = o[1]; w[2] = o[2];
+  }
+}
+
+static void launch_release(const ssc_host_potential& hp, const ssc_sources& src,
+                           const double* prog_w, const int32_t* rel_idx, const double* t_rel,
+                           const int32_t* step_rel, const double* g_msat, int nrel, int64_t seed0,
+                           int nseed, const KVals& kv, const ReleaseOut& out, hipStream_t st) {
+  auto go = [&](auto kernel, int R) {
+    // up to four rounds of seeds a block while that leaves the chip short of blocks
+    const int64_t bx = ((int64_t)nrel + R - 1) / R, rounds = ((int64_t)nseed * R + 63) / 64;
+    const int64_t by = std::max<int64_t>(1, std::min<int64_t>((rounds + 3) / 4, 4096 / bx));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)bx, (unsigned)by), dim3(256), 0, st, hp, src,
+                       prog_w, rel_idx, t_rel, step_rel, g_msat, nrel, seed0, nseed, kv, out);
+  };
+  // The lanes depend on the source table alone, so that a release's rows are the same bits
+  // whatever else its launch holds.
+  if (src.kind == SSC_SRC_NONE) go(release_kernel<1>, release_block(1));
+  else if (src.n < 64) go(release_kernel<16>, release_block(16));
+  else go(release_kernel<64>, release_block(64));
 }
 
 // ------------------------------------------------------------------------------------------
@@ -421,9 +463,9 @@ extern "C" int ssc_release(const ssc_host_potential* host, const ssc_sources* sr
   KVals kv;
   const double def[8] = {2.0, 0.3, 0.0, 0.0, 0.4, 0.4, 0.5, 0.5};
   for (int k = 0; k < 8; ++k) kv.k[k] = kvals ? kvals[k] : def[k];
-  hipLaunchKernelGGL(release_kernel, dim3((nrel + 255) / 256), dim3(256), 0, (hipStream_t)stream,
-                     *host, with_src ? *src : none, prog_w, rel_idx, t_rel, step_rel, g_msat,
-                     nrel, seed, kv, pos_close, pos_far, vel_close, vel_far);
+  const ReleaseOut out = {{pos_close, pos_far, vel_close, vel_far}, 0, 3};
+  launch_release(*host, with_src ? *src : none, prog_w, rel_idx, t_rel, step_rel, g_msat, nrel,
+                 seed, 1, kv, out, (hipStream_t)stream);
   return check_launch("ssc_release");
 }
 
@@ -451,9 +493,11 @@ extern "C" int ssc_release_seeds(const ssc_host_potential* host, const ssc_sourc
   KVals kv;
   const double def[8] = {2.0, 0.3, 0.0, 0.0, 0.4, 0.4, 0.5, 0.5};
   for (int k = 0; k < 8; ++k) kv.k[k] = kvals ? kvals[k] : def[k];
-  hipLaunchKernelGGL(release_seeds_kernel, dim3((nrel + RS_REL - 1) / RS_REL), dim3(256), 0,
-                     (hipStream_t)stream, *host, with_src ? *src : none, prog_w, rel_idx, t_rel,
-                     step_rel, g_msat, nrel, seed0, nseed, kv, rows);
+  // rows[s][arm][i][6] = (position, velocity), arm 0 = close (leading), 1 = far (trailing)
+  const int64_t arm = (int64_t)nrel * 6;
+  const ReleaseOut out = {{rows, rows + arm, rows + 3, rows + arm + 3}, 2 * arm, 6};
+  launch_release(*host, with_src ? *src : none, prog_w, rel_idx, t_rel, step_rel, g_msat, nrel,
+                 seed0, nseed, kv, out, (hipStream_t)stream);
   return check_launch("ssc_release_seeds");
 }
 
