@@ -15,6 +15,7 @@
 #include <climits>
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "ssc_device.h"
 #include "ssc_sources_lds.h"
@@ -67,20 +68,31 @@ __device__ __forceinline__ void adj_apply(const ssc_host_potential& hp, const So
   for (int r = 0; r < 3; ++r) hw[r] = H[3 * r] * W[0] + H[3 * r + 1] * W[1] + H[3 * r + 2] * W[2];
   if (SK != SSC_SRC_NONE) {
     double sw[3] = {0.0, 0.0, 0.0};
-    for (int j = rl; j < lds.n; j += G) {
-      double sx, sy, sz, gm, q2;
-      if (!lds.get(k, t, j, sx, sy, sz, gm, q2)) continue;
-      // H_j W = G m (W / s^3 - 3 d (d.W) / s^5), accumulated by two FMAs per component
-      const double dx = x - sx, dy = y - sy, dz = z - sz;
-      const double s2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, q2)));
-      const double is = rsq(s2);
-      const double is2 = is * is;
-      const double i3 = gm * (is2 * is);
-      const double c = (i3 * is2) * (-3.0 * fma(dx, W[0], fma(dy, W[1], dz * W[2])));
-      sw[0] = fma(i3, W[0], sw[0]); sw[0] = fma(c, dx, sw[0]);
-      sw[1] = fma(i3, W[1], sw[1]); sw[1] = fma(c, dy, sw[1]);
-      sw[2] = fma(i3, W[2], sw[2]); sw[2] = fma(c, dz, sw[2]);
-    }
+    // U sources of the lane: their reads first, then H_j W = G m (W / s^3 - 3 d (d.W) / s^5),
+    // accumulated by two FMAs per component
+    auto terms = [&](auto count, int j) {
+      constexpr int U = decltype(count)::value;
+      double sx[U], sy[U], sz[U], gm[U], q2[U];
+      bool on[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) on[u] = lds.get(k, t, j + u * G, sx[u], sy[u], sz[u], gm[u], q2[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (!on[u]) continue;
+        const double dx = x - sx[u], dy = y - sy[u], dz = z - sz[u];
+        const double s2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, q2[u])));
+        const double is = rsq(s2);
+        const double is2 = is * is;
+        const double i3 = gm[u] * (is2 * is);
+        const double c = (i3 * is2) * (-3.0 * fma(dx, W[0], fma(dy, W[1], dz * W[2])));
+        sw[0] = fma(i3, W[0], sw[0]); sw[0] = fma(c, dx, sw[0]);
+        sw[1] = fma(i3, W[1], sw[1]); sw[1] = fma(c, dy, sw[1]);
+        sw[2] = fma(i3, W[2], sw[2]); sw[2] = fma(c, dz, sw[2]);
+      }
+    };
+    int j = rl;
+    for (; j + 3 * G < lds.n; j += 4 * G) terms(std::integral_constant<int, 4>{}, j);
+    for (; j < lds.n; j += G) terms(std::integral_constant<int, 1>{}, j);
 #pragma unroll
     for (int c = 0; c < 3; ++c) hw[c] += group_sum<G>(sw[c]);
   }
@@ -208,8 +220,19 @@ __global__ __launch_bounds__(AJ_BLOCK) void adjoint_segment_kernel(
         }
       }
     }
+    // the row below's positions are read while this row is formed
+    double xn[3] = {1.0, 1.0, 1.0};
+    auto read_row = [&](int k) {
+      if (act && k >= kb) {
+        const double* xp = X + ((int64_t)(k - k0) * n + i) * xs;
+        xn[0] = xp[0]; xn[1] = xp[1]; xn[2] = xp[2];
+      }
+    };
+    read_row(k1 - 1);
     for (int k = k1 - 1; k >= kmin; --k) {
       lds.stage_row(src, k, nsteps + 1);
+      const double xk[3] = {xn[0], xn[1], xn[2]};
+      if (k > kmin) read_row(k - 1);
       if (act && k >= kb) {
         double lh[3], W[3];
 #pragma unroll
@@ -218,8 +241,7 @@ __global__ __launch_bounds__(AJ_BLOCK) void adjoint_segment_kernel(
         for (int c = 0; c < 3; ++c) { lv[c] = lh[c] + F(k, 3 + c); lx[c] += F(k, c); }
 #pragma unroll
         for (int c = 0; c < 3; ++c) W[c] = h * lh[c] + (k > s ? h * lv[c] : 0.0);
-        const double* xp = X + ((int64_t)(k - k0) * n + i) * xs;
-        adj_apply<SK, G, HS>(hp, lds, k, t0 + k * dt, rl, xp[0], xp[1], xp[2], W, lx, gh);
+        adj_apply<SK, G, HS>(hp, lds, k, t0 + k * dt, rl, xk[0], xk[1], xk[2], W, lx, gh);
         if (lead) {
           double* wb = Wb + ((int64_t)(k - k0) * n + i) * 3;
           wb[0] = W[0]; wb[1] = W[1]; wb[2] = W[2];
@@ -258,21 +280,32 @@ __global__ __launch_bounds__(AJ_BLOCK) void adjoint_segment_kernel(
   }
 }
 
-// Source adjoints of one segment: lanes = sources, one (row, particle chunk) per block.
+// Source adjoints of one segment: one wave per (row, chunk of particles).
 //   part[chunk][r][j][4] = (dL/dS_jk (3), dL/d(Gm_j)) summed over the chunk's particles
-constexpr int SR_CHUNK = 2048;
+// Per pair: 3 differences, 3 FMAs for s^2, 1/s (hardware estimate + Newton step), s^-3 and s^-5,
+// d.W, and 7 accumulating FMAs -- about 130 issue cycles of a wave; G m multiplies the sums once
+// at the end.  A lane holds two sources and H lanes one particle's 2 H, so that a wave takes
+// 64 / H particles at a time: one particle's row read from LDS serves two pairs per lane (with
+// one source per lane the six-double broadcast kept the LDS as busy as the pairs kept the
+// SIMDs), and tables smaller than the wave leave no lanes idle.  The chunk's rows are staged 64
+// at a time with one coalesced load (lane l reads particle l of the tile, the next tile's row
+// while this one is processed); the particles with a non-zero weight (those that move at this
+// row) are packed to the front, padded with zero weights to whole iterations of two particles
+// per group.  1e5 particles of one stream, 4,000 rows, 64 sources:
+// 23.0 -> 15.3 ms.
 
-// The chunk's particle rows are staged 64 at a time through LDS with one coalesced load (lane l
-// reads particle l of the tile), and every lane then reads each particle as an LDS broadcast:
-// a wave-uniform load per particle straight from memory left the loop waiting on one round trip
-// per particle.  The tile's particles with a non-zero weight (those that move at this row) form
-// a wave-uniform bit mask, and the pair loop visits only its set bits.  Per pair: 3 differences,
-// 3 FMAs for s^2, 1/s (hardware estimate + Newton step), s^-3 and s^-5, d.W, and 7 accumulating
-// FMAs; G m multiplies the sums once at the end.
-// One particle's term for one source: H_j W / (G m) and -(d.W) / s^3 added to (gx, gy, gz, gg).
+// Particles per chunk: about 192 chunks of 64 to 512 (a segment's rows x chunks then fill the chip
+// for small streams too, and where only the early part of a stream moves yet; 2,048 a chunk: 5 %
+// slower for 1e5 particles of a stream), and no fewer than there are sources, so that the
+// partials take no more memory than the recorded rows.
+static int64_t sr_chunk(int64_t n, int m) {
+  const int64_t c = std::min<int64_t>(512, std::max<int64_t>(64, (n / 192 + 63) / 64 * 64));
+  return std::max<int64_t>(c, ((int64_t)m + 63) / 64 * 64);
+}
+
+// One particle's term for one source: H_j W / (G m) and -(d.W) / s^3 added to g[0..2] and g[3].
 __device__ __forceinline__ void pair_adjoint(const double* t, double sx, double sy, double sz,
-                                             double q2, double& gx, double& gy, double& gz,
-                                             double& gg) {
+                                             double q2, double* g) {
   const double W0 = t[3], W1 = t[4], W2 = t[5];
   const double dx = t[0] - sx, dy = t[1] - sy, dz = t[2] - sz;
   const double s2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, q2)));
@@ -281,32 +314,35 @@ __device__ __forceinline__ void pair_adjoint(const double* t, double sx, double 
   const double i3 = is2 * is;
   const double dW = fma(dx, W0, fma(dy, W1, dz * W2));
   const double c = (i3 * is2) * (-3.0 * dW);
-  gx = fma(i3, W0, gx); gx = fma(c, dx, gx);
-  gy = fma(i3, W1, gy); gy = fma(c, dy, gy);
-  gz = fma(i3, W2, gz); gz = fma(c, dz, gz);
-  gg = fma(-i3, dW, gg);
+  g[0] = fma(i3, W0, g[0]); g[0] = fma(c, dx, g[0]);
+  g[1] = fma(i3, W1, g[1]); g[1] = fma(c, dy, g[1]);
+  g[2] = fma(i3, W2, g[2]); g[2] = fma(c, dz, g[2]);
+  g[3] = fma(-i3, dW, g[3]);
 }
 
-template <int SK>
+template <int SK, int H>
 __global__ __launch_bounds__(64) void source_adjoint_kernel(
     ssc_sources src, const double* __restrict__ X, int xs, const double* __restrict__ Wb, int64_t n,
-    int k0, int rows, double t0, double dt, double* __restrict__ part) {
-  __shared__ double tile[64][6];  // x, y, z, W0, W1, W2 of 64 particles
+    int64_t chunk_size, int k0, int rows, double t0, double dt, double* __restrict__ part) {
+  constexpr int GRP = 64 / H;     // particles at a time
+  __shared__ double tile[64][6];  // x, y, z, W0, W1, W2 of up to 64 particles
   const int r = blockIdx.y, chunk = blockIdx.x;
+  const int lane = threadIdx.x, h = lane % H, grp = lane / H;
   const int k = k0 + r;
   const double t = t0 + k * dt;
-  const int64_t ib = (int64_t)chunk * SR_CHUNK, ie = min(n, ib + SR_CHUNK);
-  const int nj = (src.n + 63) / 64;  // block-uniform trip count (barriers inside)
-  for (int jj = 0; jj < nj; ++jj) {
-    const int j = jj * 64 + threadIdx.x;
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    const bool on = j < src.n && source_position(src, j, k, t, sx, sy, sz);
-    const double q2 = j < src.n ? src.rs[j] * src.rs[j] : 1.0;  // finite pairs on idle lanes
-    double gx = 0.0, gy = 0.0, gz = 0.0, gg = 0.0, hx = 0.0, hy = 0.0, hz = 0.0, hg = 0.0;
-    // the next tile's row is loaded into registers while the current tile is processed
-    double nx[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  const int64_t ib = (int64_t)chunk * chunk_size, ie = min(n, ib + chunk_size);
+  for (int jb = 0; jb < src.n; jb += 2 * H) {  // block-uniform (barriers inside)
+    double s[2][3] = {}, q2[2], g[2][4] = {};
+    bool on[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int j = jb + u * H + h;
+      on[u] = j < src.n && source_position(src, j, k, t, s[u][0], s[u][1], s[u][2]);
+      q2[u] = j < src.n ? src.rs[j] * src.rs[j] : 1.0;  // finite pairs on idle lanes
+    }
+    double nx[6] = {};
     auto fetch = [&](int64_t i0) {
-      const int64_t i = i0 + threadIdx.x;
+      const int64_t i = i0 + lane;
       if (i < ie) {
         const double* xp = X + ((int64_t)r * n + i) * xs;
         const double* w = Wb + ((int64_t)r * n + i) * 3;
@@ -318,66 +354,89 @@ __global__ __launch_bounds__(64) void source_adjoint_kernel(
     fetch(ib);
     for (int64_t i0 = ib; i0 < ie; i0 += 64) {
       __syncthreads();  // the previous tile has been read
+      const bool moves = nx[3] != 0.0 || nx[4] != 0.0 || nx[5] != 0.0;
+      const uint64_t mask = __ballot(moves);
+      const int cnt = __popcll(mask), pad = (cnt + 2 * GRP - 1) / (2 * GRP) * (2 * GRP);
+      if (moves) {
+        double* o = tile[__popcll(mask & ((1ull << lane) - 1))];
 #pragma unroll
-      for (int c = 0; c < 6; ++c) tile[threadIdx.x][c] = nx[c];
-      const uint64_t mask = __ballot(nx[3] != 0.0 || nx[4] != 0.0 || nx[5] != 0.0);
+        for (int c = 0; c < 6; ++c) o[c] = nx[c];
+      }
+      if (lane >= cnt && lane < pad) {  // far away and weightless: adds exact zeros
+        double* o = tile[lane];
+        o[0] = o[1] = o[2] = 1e30;
+        o[3] = o[4] = o[5] = 0.0;
+      }
       __syncthreads();
       if (i0 + 64 < ie) fetch(i0 + 64);
-      // two particles per iteration into separate sums: their dependent chains interleave
-      uint64_t mk = mask;
-      while (mk != 0) {
-        const int p = __builtin_ctzll(mk);
-        mk &= mk - 1;
-        pair_adjoint(tile[p], sx, sy, sz, q2, gx, gy, gz, gg);
-        if (mk != 0) {
-          const int p2 = __builtin_ctzll(mk);
-          mk &= mk - 1;
-          pair_adjoint(tile[p2], sx, sy, sz, q2, hx, hy, hz, hg);
-        }
+      for (int p = grp; p < pad; p += 2 * GRP) {
+        double a[6], b[6];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) { a[c] = tile[p][c]; b[c] = tile[p + GRP][c]; }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) pair_adjoint(a, s[u][0], s[u][1], s[u][2], q2[u], g[u]);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) pair_adjoint(b, s[u][0], s[u][1], s[u][2], q2[u], g[u]);
       }
     }
-    gx += hx; gy += hy; gz += hz; gg += hg;
-    if (j < src.n) {
-      const double gm = on ? src.gm[j] : 0.0;
-      double* o = part + (((int64_t)chunk * rows + r) * src.n + j) * 4;
-      o[0] = gm * gx; o[1] = gm * gy; o[2] = gm * gz; o[3] = on ? gg : 0.0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int x = H; x < 64; x *= 2) g[u][c] += __shfl_xor(g[u][c], x, 64);
+      const int j = jb + u * H + h;
+      if (grp == 0 && j < src.n) {
+        const double gm = on[u] ? src.gm[j] : 0.0;
+        double* o = part + (((int64_t)chunk * rows + r) * src.n + j) * 4;
+        o[0] = gm * g[u][0]; o[1] = gm * g[u][1]; o[2] = gm * g[u][2];
+        o[3] = on[u] ? g[u][3] : 0.0;
+      }
     }
   }
 }
 
-// Sum the chunk partials of each (row, source) into row_sums[row][j][4] (one thread per
-// (row, j)); TRACK sources own one position row per grid row, so their g_pos[k0 + row][j] is
-// added here directly.
-__global__ void source_adjoint_reduce(const double* __restrict__ part, int nchunk, int rows, int m,
-                                      int k0, int track, double* __restrict__ g_pos,
-                                      double* __restrict__ row_sums) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)rows * m) return;
-  const int r = (int)(e / m), j = (int)(e - (int64_t)r * m);
-  double a[4] = {0, 0, 0, 0};
-  for (int c = 0; c < nchunk; ++c) {
-    const double* p = part + (((int64_t)c * rows + r) * m + j) * 4;
-    a[0] += p[0]; a[1] += p[1]; a[2] += p[2]; a[3] += p[3];
+// Sum the chunk partials of each (row, source) into row_sums[row][j][4]; TRACK sources own one
+// position row per grid row, so their g_pos[k0 + row][j] is added here directly.  A block sums 64
+// consecutive doubles of the table, four waves a quarter of the chunks each: coalesced reads,
+// eight in flight a lane (one thread per (row, source) walked 196 chunks in 42 us; 22 us).
+__global__ __launch_bounds__(256) void source_adjoint_reduce(const double* __restrict__ part,
+                                                             int nchunk, int rows, int m, int k0,
+                                                             int track,
+                                                             double* __restrict__ g_pos,
+                                                             double* __restrict__ row_sums) {
+  __shared__ double sums[4][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t tot = (int64_t)rows * m * 4, e = (int64_t)blockIdx.x * 64 + lane;
+  double a = 0.0;
+  if (e < tot) {
+#pragma unroll 8
+    for (int c = wv; c < nchunk; c += 4) a += part[c * tot + e];
   }
-  if (g_pos && track) {
-    double* o = g_pos + ((int64_t)(k0 + r) * m + j) * 3;
-    o[0] += a[0]; o[1] += a[1]; o[2] += a[2];
-  }
-  double* s = row_sums + ((int64_t)r * m + j) * 4;
-  s[0] = a[0]; s[1] = a[1]; s[2] = a[2]; s[3] = a[3];
+  sums[wv][lane] = a;
+  __syncthreads();
+  if (wv != 0 || e >= tot) return;
+  a = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
+  row_sums[e] = a;
+  const int c = (int)(e & 3);
+  if (g_pos && track && c < 3) g_pos[((int64_t)k0 * m + (e >> 2)) * 3 + c] += a;
 }
 
-// Sum a segment's rows per source (one thread per source, the only writer of its outputs):
-// g_gm[j] always, and g_pos[j] for STATIC sources, whose one position every row shares.
-__global__ void rows_reduce(const double* __restrict__ row_sums, int rows, int m, int track,
-                            double* __restrict__ g_pos, double* __restrict__ g_gm) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= m) return;
+// Sum a segment's rows per source (one wave per source, the only writer of its outputs; one
+// thread per source walked the 101 rows in 33 us): g_gm[j] always, and g_pos[j] for STATIC
+// sources, whose one position every row shares.
+__global__ __launch_bounds__(64) void rows_reduce(const double* __restrict__ row_sums, int rows,
+                                                  int m, int track, double* __restrict__ g_pos,
+                                                  double* __restrict__ g_gm) {
+  const int j = blockIdx.x;
   double a[4] = {0, 0, 0, 0};
-  for (int r = 0; r < rows; ++r) {
+  for (int r = threadIdx.x; r < rows; r += 64) {
     const double* s = row_sums + ((int64_t)r * m + j) * 4;
     a[0] += s[0]; a[1] += s[1]; a[2] += s[2]; a[3] += s[3];
   }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) a[c] = group_sum<64>(a[c]);
+  if (threadIdx.x != 0) return;
   if (g_gm) g_gm[j] += a[3];
   if (g_pos && !track) {
     g_pos[3 * j] += a[0];
@@ -385,7 +444,6 @@ __global__ void rows_reduce(const double* __restrict__ row_sums, int rows, int m
     g_pos[3 * j + 2] += a[2];
   }
 }
-
 
 __global__ void ckpt_index_kernel(int32_t* __restrict__ idx, int64_t nseg, int E, int nsteps) {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -423,9 +481,10 @@ static int seg_len(int E) { return E == 1 ? AJ_STORED_SEG : E; }
 
 static int64_t adj_bytes(int64_t n, int nsteps, int E, int m, AdjWs* w, char* base) {
   const int64_t nseg = nseg_of(nsteps, E);
-  // segment-kernel blocks: G lanes per particle (the same choice adjoint_backward makes)
-  const int64_t nblk = (n * group_lanes(n, m) + AJ_BLOCK - 1) / AJ_BLOCK;
-  const int64_t nchunk = (n + SR_CHUNK - 1) / SR_CHUNK;
+  // segment-kernel blocks: G lanes per particle, with or without start rows
+  const int64_t nblk = (n * std::max(group_lanes(n, m, false), group_lanes(n, m, true)) +
+                        AJ_BLOCK - 1) / AJ_BLOCK;
+  const int64_t nchunk = (n + sr_chunk(n, m) - 1) / sr_chunk(n, m);
   const int64_t rows = (int64_t)seg_len(E) + 1;
   int64_t off = 0;
   auto take = [&](int64_t bytes) {
@@ -459,9 +518,9 @@ static int adjoint_backward(const ssc_host_potential& hp, const ssc_sources& src
   const int m = SK == SSC_SRC_NONE ? 0 : src.n;
   const bool stored = E == 1;
   const int L = seg_len(E);
-  const int G = SK == SSC_SRC_NONE ? 1 : group_lanes(n, m);
+  const int G = SK == SSC_SRC_NONE ? 1 : group_lanes(n, m, start != nullptr);
   const unsigned nblk = (unsigned)((n * G + AJ_BLOCK - 1) / AJ_BLOCK);
-  const int64_t nchunk = (n + SR_CHUNK - 1) / SR_CHUNK;
+  const int64_t nchunk = (n + sr_chunk(n, m) - 1) / sr_chunk(n, m);
   const size_t lds = SourceLDS<SK>::bytes(src);
   auto seg_kernel = [&](void) -> const void* {
     switch (G) {
@@ -504,12 +563,16 @@ static int adjoint_backward(const ssc_host_potential& hp, const ssc_sources& src
     }
 #undef SSC_SEG
     if (m > 0 && (g_gm || g_pos)) {
-      hipLaunchKernelGGL(source_adjoint_kernel<SK>, dim3((unsigned)nchunk, (unsigned)rows), dim3(64),
-                         0, st, src, X, xs, w.Wb, n, k0, rows, t0, dt, w.part);
-      hipLaunchKernelGGL(source_adjoint_reduce, dim3((unsigned)((rows * m + 255) / 256)), dim3(256),
-                         0, st, w.part, (int)nchunk, rows, m, k0, SK == SSC_SRC_TRACK ? 1 : 0,
+      // the narrowest groups whose 2 H sources hold the table, at most half a wave
+      auto source_kernel = m <= 16   ? source_adjoint_kernel<SK, 8>
+                           : m <= 32 ? source_adjoint_kernel<SK, 16>
+                                     : source_adjoint_kernel<SK, 32>;
+      hipLaunchKernelGGL(source_kernel, dim3((unsigned)nchunk, (unsigned)rows), dim3(64), 0, st,
+                         src, X, xs, w.Wb, n, sr_chunk(n, m), k0, rows, t0, dt, w.part);
+      hipLaunchKernelGGL(source_adjoint_reduce, dim3((unsigned)(((int64_t)rows * m + 15) / 16)),
+                         dim3(256), 0, st, w.part, (int)nchunk, rows, m, k0, SK == SSC_SRC_TRACK ? 1 : 0,
                          g_pos, w.gm_rows);
-      hipLaunchKernelGGL(rows_reduce, dim3((m + 255) / 256), dim3(256), 0, st, w.gm_rows, rows, m,
+      hipLaunchKernelGGL(rows_reduce, dim3(m), dim3(64), 0, st, w.gm_rows, rows, m,
                          SK == SSC_SRC_TRACK ? 1 : 0, g_pos, g_gm);
     }
     k1 = k0;

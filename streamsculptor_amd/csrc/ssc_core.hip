@@ -601,37 +601,11 @@ static int set_lds(const void* fn, size_t lds) {
   return SSC_OK;
 }
 
-// Lanes per orbit: the G of 1 ... 16 with the smallest estimate of a step's time.  A step lasts
-// as long as the SIMD with the most waves, w = ceil(n G / 65536), and about a quarter of a wave's
-// time on top (its chain of dependent instructions, not overlapped); a wave's time is its share
-// of the sources plus the host terms and log2 G exchanges, worth 4 + 3 log2 G sources.  The
-// whole-number w is what matters: at 1e5 orbits two lanes need 3.05 -> 4 waves' time and one
-// lane 1.5 -> 2.  Measured per step, the previous rule (three waves per SIMD wanted) -> this one,
-// 64 tracked subhalos: 12,500 orbits 2.44 -> 1.54 us (16 -> 4 lanes), 25,000 3.13 -> 2.39 (8 -> 2),
-// 50,000 4.41 -> 4.09 (4 -> 1), 100,000 7.21 -> 6.53 (2 -> 1); 512 static clumps: 10,000
-// 6.85 -> 6.80, 25,000 14.5 -> 14.1, 200,000 90.7 -> 84.8 (1 -> 4), 400,000 169 -> 153.
-// Orbits that start all along the grid (`ragged`) fill the SIMDs unevenly whatever G is, and each
-// wave ends when its latest block's work does: half the waves' work, not rounded up, but at least
-// one wave's (1e5 orbits of one stream, 64 tracked subhalos, 4,000 rows: two lanes 13.8 ms, one
-// lane 16.3 ms).
-inline int leapfrog_lanes(int64_t n, int nsrc, bool ragged) {
-  int best = 1;
-  double least = 0.0;
-  for (int lg = 0; lg <= 4; ++lg) {
-    const int64_t g = 1 << lg;
-    const double waves = ragged ? std::max(1.0, n * g / 131072.0)
-                                : (double)((n * g + 65535) / 65536);
-    const double cost = (4.0 * waves + 1.0) * (double)((nsrc + g - 1) / g + 4 + 3 * lg);
-    if (lg == 0 || cost <= least) { least = cost; best = (int)g; }
-  }
-  return best;
-}
-
 // Launch shape: one wave per orbit while every orbit has a SIMD of its own and the table is
 // large (512 clumps: 1,000 orbits 1.81 us a step against 2.87 with 16 lanes an orbit, 2,000
 // orbits 4.39 against 2.96); two particles per lane for batches that fill the chip several times
 // over, unless the pairing costs a round of waves (512 clumps: 1e6 orbits 326 us against 331,
-// 4e5 169 against 153); leapfrog_lanes otherwise.  Without sources: for up to 65536 orbits in a
+// 4e5 169 against 153); group_lanes otherwise.  Without sources: for up to 65536 orbits in a
 // host of no known signature, host components over waves; one particle per lane otherwise (with
 // straight-line host code for the known hosts, which is faster still).
 template <int SK, int HS>
@@ -663,7 +637,7 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                        w_out, save_idx, nsave, ys);
     return check_launch("ssc_leapfrog");
   }
-  const int g = SK == SSC_SRC_NONE ? 1 : leapfrog_lanes(n, src.n, ragged);
+  const int g = SK == SSC_SRC_NONE ? 1 : group_lanes(n, src.n, ragged);
 #define SSC_GROUP(GV)                                                                              \
   if (g == GV) {                                                                                   \
     int rc = set_lds((const void*)leapfrog_group_kernel<SK, GV, HS>, lds);                            \

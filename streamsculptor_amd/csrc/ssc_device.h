@@ -4,6 +4,8 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 #include <stdint.h>
 #include <string>
 
@@ -113,24 +115,40 @@ __device__ __forceinline__ double log1p_nonneg(double u) {
   return fma(fe, ln2_hi, fma(fe, ln2_lo, lm) + c * __builtin_amdgcn_rcp(t));
 }
 
+// Lanes per orbit: the G of 1 ... 16 with the smallest estimate of a step's time.  A step lasts
+// as long as the SIMD with the most waves, w = ceil(n G / 65536), and about a quarter of a wave's
+// time on top (its chain of dependent instructions, not overlapped); a wave's time is its share
+// of the sources plus the host terms and log2 G exchanges, worth 4 + 3 log2 G sources.  The
+// whole-number w is what matters: at 1e5 orbits two lanes need 3.05 -> 4 waves' time and one
+// lane 1.5 -> 2.  Measured per step, the previous rule (three waves per SIMD wanted) -> this one,
+// 64 tracked subhalos: 12,500 orbits 2.44 -> 1.54 us (16 -> 4 lanes), 25,000 3.13 -> 2.39 (8 -> 2),
+// 50,000 4.41 -> 4.09 (4 -> 1), 100,000 7.21 -> 6.53 (2 -> 1); 512 static clumps: 10,000
+// 6.85 -> 6.80, 25,000 14.5 -> 14.1, 200,000 90.7 -> 84.8 (1 -> 4), 400,000 169 -> 153.
+// Orbits that start all along the grid (`ragged`) fill the SIMDs unevenly whatever G is, and each
+// wave ends when its latest block's work does: half the waves' work, not rounded up, but at least
+// one wave's (1e5 orbits of one stream, 64 tracked subhalos, 4,000 rows: two lanes 13.8 ms, one
+// lane 16.3 ms).  The backward sweep uses the same rule, the previous one (three waves per SIMD
+// wanted) against it, per row and 64 sources: 25,000 orbits 10.1 -> 7.6 us, 50,000 14.7 -> 12.9,
+// 100,000 24.3 -> 22.0.
+inline int group_lanes(int64_t n, int nsrc, bool ragged) {
+  int best = 1;
+  double least = 0.0;
+  for (int lg = 0; lg <= 4; ++lg) {
+    const int64_t g = 1 << lg;
+    const double waves = ragged ? std::max(1.0, n * g / 131072.0)
+                                : (double)((n * g + 65535) / 65536);
+    const double cost = (4.0 * waves + 1.0) * (double)((nsrc + g - 1) / g + 4 + 3 * lg);
+    if (lg == 0 || cost <= least) { least = cost; best = (int)g; }
+  }
+  return best;
+}
+
 // ------------------------------------------------------------------------------------------
 // Sum of a double over aligned groups of G consecutive lanes (G = 1, 2, 4, ..., 64), the result
 // in every lane of the group.  Within a 16-lane row the exchanges are DPP moves (quad
 // permutations, then the half-row and row mirrors), which need no trip through the LDS unit;
 // the 32- and 64-lane steps use lane shuffles.  Every lane of the wave must be active.
 // ------------------------------------------------------------------------------------------
-// Lanes per orbit for the grouped kernels: enough to give the launch about three waves per SIMD
-// (3 x 1024 SIMDs x 64 lanes), at most 16, and at least four sources per lane.  (1e5 orbits in
-// 64 live subhalos: two lanes per orbit 18.4 ms, four 19.0 ms, eight 25.9 ms per stream.)
-inline int group_lanes(int64_t n, int nsrc) {
-  if (nsrc < 16 || n <= 0) return 1;
-  const double want = 196608.0 / (double)n;
-  int g = 1;
-  while (g < want && g < 16) g *= 2;
-  while (g > 1 && nsrc / g < 4) g /= 2;
-  return g;
-}
-
 template <int CTRL>
 __device__ __forceinline__ double dpp_move(double v) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
