@@ -343,13 +343,15 @@ class Potential:
         return torch.cat([xv[..., 3:], -self.gradient(xv[..., :3], t)], dim=-1)
 
     # ------------------------------------------------------------------ integration
-    def _leapfrog(self, w0, t0, dt, nsteps, start=None, save_idx=None, src_override=False):
-        """Run ssc_leapfrog on rows w0 (n, 6); returns (w_final, ys or None)."""
+    def _leapfrog(self, w0, t0, dt, nsteps, start=None, save_idx=None, src_override=False,
+                  out=None):
+        """Run ssc_leapfrog on rows w0 (n, 6); returns (w_final, ys or None); ``out``: contiguous
+        rows for w_final, other than w0."""
         h, src = self._descriptor()
         w0 = _lib.f64(w0).reshape(-1, 6).contiguous()
         n = w0.shape[0]
         dev = w0.device
-        out = torch.empty_like(w0)
+        out = torch.empty_like(w0) if out is None else out
         st = None if start is None else _lib.i32(start)
         si = None if save_idx is None else _lib.i32(save_idx)
         nsave = 0 if si is None else si.numel()
@@ -476,12 +478,26 @@ class Potential:
         outs = self._release(w, idx, gms, seed_num, kval_arr, t_rel=tt)
         return tuple(o.reshape(*shape, 3) for o in outs)
 
+    def _release_at(self, t_rel):
+        """What a release at times t_rel needs of this potential's point sources: (descriptor,
+        times, table rows of TRACK sources, the source set the descriptor points into), all None
+        without sources.  A part of the releases takes a slice of the times and rows."""
+        _, src = self._descriptor()
+        if src is None:
+            return None, None, None, None
+        if t_rel is None:
+            raise ValueError("the release in a potential with point sources needs the "
+                             "release times")
+        tr = np.asarray(_as_float(t_rel), dtype=np.float64).reshape(-1)
+        src, steps = src.rows_for(tr)
+        return src.desc(), _lib.f64(tr), None if steps is None else _lib.i32(steps), src
+
     def _release(self, prog_w, rel_idx, g_msat, seed_num, kval_arr, t_rel=None):
         """Release model of rows prog_w (n, 6) at times t_rel (n,) in this whole potential: its
         point sources enter the tidal radius through d2phidr2 (reference main.py:77-85,
         230-237).  t_rel is needed when the potential has point sources (LINE: their positions;
         TRACK: the table row of each release)."""
-        h, src = self._descriptor()
+        h, _ = self._descriptor()
         n = prog_w.shape[0]
         kv = np.asarray(_as_float(kval_arr), dtype=np.float64)
         kvp = None
@@ -489,17 +505,7 @@ class Potential:
             kv = np.ascontiguousarray(np.ones(8) * kv)
             kvp = kv.ctypes.data_as(_lib.ctypes.c_void_p)
         dev = prog_w.device
-        sd, t_dev, step_dev = None, None, None
-        if src is not None:
-            if t_rel is None:
-                raise ValueError("the release in a potential with point sources needs the "
-                                 "release times")
-            tr = np.asarray(_as_float(t_rel), dtype=np.float64).reshape(-1)
-            src, steps = src.rows_for(tr)
-            if steps is not None:
-                step_dev = _lib.i32(steps)
-            t_dev = _lib.f64(tr)
-            sd = src.desc()
+        sd, t_dev, step_dev, _src = self._release_at(t_rel)
         outs = [torch.empty(n, 3, dtype=torch.float64, device=dev) for _ in range(4)]
         _lib.call("ssc_release", _lib.ctypes.byref(h),
                   None if sd is None else _lib.ctypes.byref(sd), _lib.ptr(prog_w.contiguous()),
@@ -508,11 +514,13 @@ class Potential:
                   *[_lib.ptr(o) for o in outs])
         return outs  # pos_close (lead), pos_far (trail), vel_close, vel_far
 
-    def _release_seeds(self, prog_w, rel_idx, g_msat, seed0, nseed, kval_arr, t_rel=None):
+    def _release_seeds(self, prog_w, rel_idx, g_msat, seed0, nseed, kval_arr, t_rel=None,
+                       at=None):
         """``_release`` for seeds seed0 .. seed0 + nseed - 1 in one launch (ssc_release_seeds):
         returns rows (nseed, 2, n, 6), arm 0 = (pos_close, vel_close) (lead), arm 1 =
-        (pos_far, vel_far) (trail), equal to the per-seed calls bit for bit."""
-        h, src = self._descriptor()
+        (pos_far, vel_far) (trail), equal to the per-seed calls bit for bit.  ``at``: these
+        releases' part of a ``_release_at`` in place of t_rel."""
+        h, _ = self._descriptor()
         n = prog_w.shape[0]
         kv = np.asarray(_as_float(kval_arr), dtype=np.float64)
         kvp = None
@@ -520,17 +528,7 @@ class Potential:
             kv = np.ascontiguousarray(np.ones(8) * kv)
             kvp = kv.ctypes.data_as(_lib.ctypes.c_void_p)
         dev = prog_w.device
-        sd, t_dev, step_dev = None, None, None
-        if src is not None:
-            if t_rel is None:
-                raise ValueError("the release in a potential with point sources needs the "
-                                 "release times")
-            tr = np.asarray(_as_float(t_rel), dtype=np.float64).reshape(-1)
-            src, steps = src.rows_for(tr)
-            if steps is not None:
-                step_dev = _lib.i32(steps)
-            t_dev = _lib.f64(tr)
-            sd = src.desc()
+        sd, t_dev, step_dev, _src = at or self._release_at(t_rel)
         rows = torch.empty(int(nseed), 2, n, 6, dtype=torch.float64, device=dev)
         _lib.call("ssc_release_seeds", _lib.ctypes.byref(h),
                   None if sd is None else _lib.ctypes.byref(sd), _lib.ptr(prog_w.contiguous()),

@@ -56,10 +56,11 @@ def _restartable(pot):
 _SIDE = {}
 
 
-def _side_stream(dev):
-    """One second stream per device, kept for the process: a stream of its own keeps its
-    hardware queue, and creating one per call costs host time ahead of the first launch."""
-    key = torch.device(dev).index
+def _side_stream(dev, which=0):
+    """A second (``which`` = 1: third) stream per device, kept for the process: a stream of its
+    own keeps its hardware queue, and creating one per call costs host time ahead of the first
+    launch."""
+    key = (torch.device(dev).index, which)
     if key not in _SIDE:
         _SIDE[key] = torch.cuda.Stream(device=dev)
     return _SIDE[key]
@@ -68,17 +69,17 @@ def _side_stream(dev):
 def _leapfrog_stream_pipelined(prog_pot, release_pot, particle_pot, ts_np, prog_w0, Msat,
                                seed_num, kval_arr, dt0, chunks):
     """The fixed-step spray stream in ``chunks`` windows of grid rows on two streams: the
-    current stream advances the progenitor orbit through a window and releases the particles
-    of that window; a second stream then advances every particle released so far through the
-    same window while the progenitor moves on through the next.  The single-orbit chain (one
-    lane, latency-bound) thus overlaps the particles' integration instead of preceding all of
-    it, and two streams keep clear of hardware-queue sharing, which serialises streams mapped
-    to one queue.  Every orbit takes the steps of the one-pass path (a restart at a grid row
-    recomputes the acceleration there from the same state; a particle starts at its own row):
-    in the host alone the rows are the same bit for bit; with sources the acceleration at a
-    window's first row comes from the kernel's prologue, whose FMA contraction can differ from
-    the step loop's in the last bit.  Returns the particle rows (2T, 6), lead/trail
-    interleaved, in release order."""
+    current stream advances the progenitor orbit through window after window and does nothing
+    else; a second stream releases each window's particles and advances every particle released
+    so far through it.  The single-orbit chain (one lane, latency-bound) is the longest, so the
+    releases and their copies stay off it (4,000 steps and 8,000 particles: 2.56 ms with them on
+    the current stream, 2.29 ms so; 1.98 ms with the progenitor saved in straight code), and two
+    streams keep clear of hardware-queue sharing, which serialises streams mapped to one queue.
+    Every orbit takes the steps of the one-pass path (a restart at a grid row recomputes the
+    acceleration there from the same state; a particle starts at its own row): in the host alone
+    the rows are the same bit for bit; with sources the acceleration at a window's first row comes
+    from the kernel's prologue, whose FMA contraction can differ from the step loop's in the last
+    bit.  Returns the particle rows (2T, 6), lead/trail interleaved, in release order."""
     from .main import _as_float
     t0, dt, nsteps, kidx = release_grid(ts_np, dt0)
     T = len(ts_np) - 1
@@ -101,33 +102,34 @@ def _leapfrog_stream_pipelined(prog_pot, release_pot, particle_pot, ts_np, prog_
     save_all = [flat[o:o + k] for o, k in spans[0::2]]
     start_all = [flat[o:o + k] for o, k in spans[1::2]]
     idx_all = torch.arange(T, dtype=torch.int32, device=dev)
+    sd, t_all, step_all, src = release_pot._release_at(ts_np[:T])
+    # particle rows before and after a window, in turn
+    rows = [torch.empty(2 * T, 6, dtype=torch.float64, device=dev) for _ in range(2)]
     main = torch.cuda.current_stream(dev)
     side = _side_stream(dev)
-    state = None
-    keep = []
-    for c in range(len(cuts) - 1):
-        a, b = cuts[c], cuts[c + 1]
-        g0 = int(kidx[a])
-        g1 = int(kidx[b]) if b < T else nsteps
-        # progenitor rows kidx[a..b-1], and its state at the next window's first row g1
-        pn = (g1 if b < T else int(kidx[T - 1])) - g0
-        w_next, ys = prog_pot._leapfrog(w, t0 + g0 * dt, dt, pn, save_idx=save_all[c])
-        ws = ys[:, 0, :].contiguous()
-        pc, pf, vc, vf = release_pot._release(ws, idx_all[a:b].contiguous(),
-                                              gms_all[a:b].contiguous(), seed_num, kval_arr,
-                                              t_rel=ts_np[a:b])
-        new = torch.empty(2 * (b - a), 6, dtype=torch.float64, device=dev)
-        new[0::2, :3], new[0::2, 3:] = pc, vc
-        new[1::2, :3], new[1::2, 3:] = pf, vf
-        side.wait_stream(main)
-        with torch.cuda.stream(side):
-            w_in = new if state is None else torch.cat([state, new], 0)
-            state, _ = particle_pot._leapfrog(w_in, t0 + g0 * dt, dt, g1 - g0,
-                                              start=start_all[c])
-        keep.append((new, w_in))
-        w = w_next
-    main.wait_stream(side)
-    return state
+    keep = []  # read on the second stream: held until the current one has waited for it
+    try:
+        for c in range(len(cuts) - 1):
+            a, b = cuts[c], cuts[c + 1]
+            g0 = int(kidx[a])
+            g1 = int(kidx[b]) if b < T else nsteps
+            # progenitor rows kidx[a..b-1], and its state at the next window's first row g1
+            pn = (g1 if b < T else int(kidx[T - 1])) - g0
+            w, ys = prog_pot._leapfrog(w, t0 + g0 * dt, dt, pn, save_idx=save_all[c])
+            keep.append(ys)
+            side.wait_stream(main)
+            with torch.cuda.stream(side):
+                at = (sd, None if t_all is None else t_all[a:b],
+                      None if step_all is None else step_all[a:b], src)
+                table = release_pot._release_seeds(ys[:, 0, :], idx_all[a:b], gms_all[a:b],
+                                                   seed_num, 1, kval_arr, at=at)
+                w_in, w_out = rows[c % 2][:2 * b], rows[(c + 1) % 2][:2 * b]
+                w_in[2 * a:].view(b - a, 2, 6).copy_(table[0].transpose(0, 1))
+                particle_pot._leapfrog(w_in, t0 + g0 * dt, dt, g1 - g0, start=start_all[c],
+                                       out=w_out)
+    finally:
+        main.wait_stream(side)
+    return w_out
 
 
 def gen_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, solver=None, kval_arr=1.0,
@@ -196,14 +198,15 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
     its order, advanced with the fixed-step leapfrog to the last grid row -- with the progenitor
     orbit pipelined with the particles over ``chunks`` windows of grid rows on two streams, as
     ``gen_stream`` does for two particles per step: the current stream advances the progenitor
-    through a window and releases that window's particles (every seed in one launch); the
-    second stream then advances every particle released so far through the window while the
-    progenitor moves on.  ``integrate(w, t0, dt, nsteps, start)`` advances rows (default: the
-    leapfrog in ``particle_pot``, else ``prog_pot``); TRACK tables are cut to each window's
-    rows.  The rows equal the one-pass order (``spray_particles``, then one integration) up to
-    the last bits of the accelerations re-formed at the windows' first rows.  Fewer than
-    4 * chunks release steps, or sources that form their positions from the time (straight
-    lines, sampled tracks): one pass."""
+    through the windows, a third one releases each window's particles (every seed in one launch)
+    and the second advances every particle released so far through it: the release waits for
+    neither of the two chains, whichever is the longer.
+    ``integrate(w, t0, dt, nsteps, start)`` advances rows (default: the leapfrog in
+    ``particle_pot``, else ``prog_pot``); TRACK tables are cut to each window's rows.  The rows
+    equal the one-pass order (``spray_particles``, then one integration) up to the last bits of
+    the accelerations re-formed at the windows' first rows.  Fewer than 4 * chunks release
+    steps, or sources that form their positions from the time (straight lines, sampled tracks):
+    one pass."""
     from .main import _as_float
     from .workloads import spray_layout
     particle_pot = particle_pot or prog_pot
@@ -225,42 +228,53 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
     gms_all = release_pot._G * _lib.f64(np.ascontiguousarray(msat[:T]))
     idx_all = torch.arange(T, dtype=torch.int32, device=dev)
     cuts = sorted({0, T} | {T * j // chunks for j in range(1, chunks)})
-    # every window's index arrays in one host-to-device copy: the progenitor rows it saves,
-    # (seed, arm, release) of its new particles, and the start rows of all particles so far
-    parts, spans = [], []
+    # every window's index arrays in two host-to-device copies: the progenitor rows it saves and
+    # the start rows of all particles so far; the rows of its new particles in the release's
+    # (seed, arm, release) table
+    parts, spans, picks = [], [], []
     for c in range(len(cuts) - 1):
         a, b = cuts[c], cuts[c + 1]
         g0 = int(kidx[a])
         sel = lay[np.arange(a, b) % 2]                            # (b - a, per_step, 2)
         rel_all = np.repeat(np.arange(b), per_step)
-        for arr in (kidx[a:b] - g0, sel[..., 0].reshape(-1), sel[..., 1].reshape(-1),
-                    np.repeat(np.arange(b - a), per_step), np.maximum(kidx[rel_all] - g0, 0)):
+        picks.append(((sel[..., 0] * 2 + sel[..., 1]) * (b - a)
+                      + np.arange(b - a)[:, None]).reshape(-1))
+        for arr in (kidx[a:b] - g0, np.maximum(kidx[rel_all] - g0, 0)):
             spans.append((sum(p.size for p in parts), arr.size))
             parts.append(np.asarray(arr).astype(np.int32))
     flat = _lib.i32(np.concatenate(parts))
     views = [flat[o:o + k] for o, k in spans]
+    pick_all = torch.as_tensor(np.concatenate(picks), device=dev)
+    sd, t_all, step_all, src = release_pot._release_at(ts_np[:T])
     main = torch.cuda.current_stream(dev)
     side = _side_stream(dev)
     w = _lib.f64(prog_w0).reshape(1, 6)
-    state, keep = None, []
-    for c in range(len(cuts) - 1):
-        a, b = cuts[c], cuts[c + 1]
-        g0 = int(kidx[a])
-        g1 = int(kidx[b]) if b < T else nsteps
-        save, s_i, a_i, r_i, start = views[5 * c:5 * c + 5]
-        pn = (g1 if b < T else int(kidx[T - 1])) - g0
-        w_next, ys = prog_pot._leapfrog(w, t0 + g0 * dt, dt, pn, save_idx=save)
-        table = release_pot._release_seeds(ys[:, 0, :].contiguous(), idx_all[a:b].contiguous(),
-                                           gms_all[a:b].contiguous(), seed_num, nseed,
-                                           kval_arr, t_rel=ts_np[a:b])
-        new = table[s_i.long(), a_i.long(), r_i.long()]
-        side.wait_stream(main)
-        with torch.cuda.stream(side):
-            w_in = new if state is None else torch.cat([state, new], 0)
-            state = integrate(w_in, t0 + g0 * dt, dt, g1 - g0, start)
-        keep.append((new, w_in))
-        w = w_next
-    main.wait_stream(side)
+    spray = _side_stream(dev, 1)
+    state, keep = None, []  # keep: read on another stream than its own
+    try:
+        for c in range(len(cuts) - 1):
+            a, b = cuts[c], cuts[c + 1]
+            g0 = int(kidx[a])
+            g1 = int(kidx[b]) if b < T else nsteps
+            save, start = views[2 * c:2 * c + 2]
+            pn = (g1 if b < T else int(kidx[T - 1])) - g0
+            w, ys = prog_pot._leapfrog(w, t0 + g0 * dt, dt, pn, save_idx=save)
+            spray.wait_stream(main)
+            with torch.cuda.stream(spray):
+                at = (sd, None if t_all is None else t_all[a:b],
+                      None if step_all is None else step_all[a:b], src)
+                table = release_pot._release_seeds(ys[:, 0, :], idx_all[a:b], gms_all[a:b],
+                                                   seed_num, nseed, kval_arr, at=at)
+                new = table.view(-1, 6).index_select(0, pick_all[a * per_step:b * per_step])
+            keep.append((ys, new))
+            side.wait_stream(spray)
+            with torch.cuda.stream(side):
+                w_in = new if state is None else torch.cat([state, new], 0)
+                state = integrate(w_in, t0 + g0 * dt, dt, g1 - g0, start)
+    finally:
+        main.wait_stream(spray)
+        main.wait_stream(side)
+    state.record_stream(main)
     return state
 
 
