@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 
 #include "ssc_device.h"
 #include "ssc_sources_lds.h"
@@ -268,7 +269,50 @@ __device__ __forceinline__ void accel_P(const ssc_host_potential& hp, const Sour
   }
 }
 
-template <int SK, int P, int HS>
+// The rows a launch saves, walked in order; the grid index of the save after the next is read a
+// save ahead, so that no step waits for it.  One wave's step is a serial chain in which each
+// branch and scalar instruction is seen, so the steps run in an inner loop up to the next saved
+// row, which compares with nothing else; launches that save most of their steps (DENSE: the
+// progenitors of streams) save inside the step instead, in straight code, because the way out of
+// the inner loop and back costs 190 ns.  One orbit in the host, ns a step: not saved 296, saved
+// every tenth step 391 -> 326 (inner loop), at every step 478 -> 390 (DENSE).
+struct SaveRows {
+  const int32_t* idx;
+  int n, next, k, k_after;
+  __device__ SaveRows(const int32_t* i, int nsave)
+      : idx(i), n(nsave), next(0), k(at(0)), k_after(at(1)) {}
+  __device__ int at(int j) const { return j < n ? idx[j] : INT_MIN; }  // none left
+  __device__ bool up_to(int row) const { return next < n && k <= row; }
+  __device__ bool due(int row) const { return k == row; }  // rows are >= 0
+  // the row to step to from `row`: the next saved one, or the last
+  __device__ int stop(int row, int last) const { return k > row && k < last ? k : last; }
+  __device__ void advance() {
+    ++next;
+    k = k_after;
+    k_after = at(next + 1);
+  }
+  // advance() if `hit`, without a branch (n > 0); the value read is first looked at a step later
+  __device__ void advance_if(bool hit) {
+    next += hit ? 1 : 0;
+    k = hit ? (next < n ? k_after : INT_MIN) : k;
+    k_after = idx[next + 1 < n ? next + 1 : n - 1];
+  }
+};
+
+// The same walk for kernels whose step is long (many orbits among sources): the index is read
+// where it is compared, and the step loop knows nothing of it (the two-level loop cost 3 to 7 %
+// of a step of 12,500 to 100,000 orbits among 64 subhalos).
+struct SaveScan {
+  const int32_t* idx;
+  int n, next;
+  __device__ SaveScan(const int32_t* i, int nsave) : idx(i), n(nsave), next(0) {}
+  __device__ bool up_to(int row) const { return next < n && idx[next] <= row; }
+  __device__ bool due(int row) const { return next < n && idx[next] == row; }
+  __device__ int stop(int row, int) const { return row + 1; }
+  __device__ void advance() { ++next; }
+};
+
+template <int SK, int P, int HS, bool DENSE>
 __global__ __launch_bounds__(LF_BLOCK) void leapfrog_kernel(
     ssc_host_potential hp, ssc_sources src, const double* __restrict__ w0,
     const int32_t* __restrict__ start, int64_t n, double t0, double dt, int nsteps,
@@ -303,15 +347,15 @@ __global__ __launch_bounds__(LF_BLOCK) void leapfrog_kernel(
   __syncthreads();
   const int kmin = kmin_sh;
   // Save rows at grid indices <= kmin hold the initial state of every particle.
-  int next = 0;
-  while (next < nsave && save_idx[next] <= kmin) {
+  typename std::conditional<SK == SSC_SRC_NONE, SaveRows, SaveScan>::type rows(save_idx, nsave);
+  while (rows.up_to(kmin)) {
 #pragma unroll
     for (int p = 0; p < P; ++p)
       if (valid[p]) {
-        double* o = ys + ((int64_t)next * n + idx[p]) * 6;
+        double* o = ys + ((int64_t)rows.next * n + idx[p]) * 6;
         o[0] = x[p]; o[1] = y[p]; o[2] = z[p]; o[3] = vx[p]; o[4] = vy[p]; o[5] = vz[p];
       }
-    ++next;
+    rows.advance();
   }
   const double h = 0.5 * dt;
   if (kmin < nsteps) {
@@ -320,29 +364,52 @@ __global__ __launch_bounds__(LF_BLOCK) void leapfrog_kernel(
   }
   // A particle that has not started keeps its initial row; the force evaluated there at
   // t_{k+1} is exactly the initial force it needs when it starts at k + 1.
-  for (int k = kmin; k < nsteps; ++k) {
-    lds.stage(src, k, nsteps + 1);
+  double* o_next[P];  // DENSE: where the next saved row goes
+  auto aim = [&]() {
 #pragma unroll
-    for (int p = 0; p < P; ++p)
-      if (k >= s[p]) {
-        vx[p] = vx[p] + h * ax[p]; vy[p] = vy[p] + h * ay[p]; vz[p] = vz[p] + h * az[p];
-        x[p] = x[p] + dt * vx[p]; y[p] = y[p] + dt * vy[p]; z[p] = z[p] + dt * vz[p];
-      }
-    accel_P<SK, P, HS>(hp, lds, k + 1, t0 + (k + 1) * dt, x, y, z, ax, ay, az);
+    for (int p = 0; p < P; ++p) o_next[p] = ys + ((int64_t)rows.next * n + idx[p]) * 6;
+  };
+  if (DENSE) aim();
+  for (int k = kmin; k < nsteps;) {
+    const int stop = DENSE ? nsteps : rows.stop(k, nsteps);
+    for (; k < stop; ++k) {
+      lds.stage(src, k, nsteps + 1);
 #pragma unroll
-    for (int p = 0; p < P; ++p)
-      if (k >= s[p]) {
-        vx[p] = vx[p] + h * ax[p]; vy[p] = vy[p] + h * ay[p]; vz[p] = vz[p] + h * az[p];
+      for (int p = 0; p < P; ++p)
+        if (k >= s[p]) {
+          vx[p] = vx[p] + h * ax[p]; vy[p] = vy[p] + h * ay[p]; vz[p] = vz[p] + h * az[p];
+          x[p] = x[p] + dt * vx[p]; y[p] = y[p] + dt * vy[p]; z[p] = z[p] + dt * vz[p];
+        }
+      accel_P<SK, P, HS>(hp, lds, k + 1, t0 + (k + 1) * dt, x, y, z, ax, ay, az);
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        if (k >= s[p]) {
+          vx[p] = vx[p] + h * ax[p]; vy[p] = vy[p] + h * ay[p]; vz[p] = vz[p] + h * az[p];
+        }
+      if constexpr (DENSE) {
+        const bool hit = rows.k == k + 1;
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          if (hit && valid[p]) {
+            double* o = o_next[p];
+            o[0] = x[p]; o[1] = y[p]; o[2] = z[p]; o[3] = vx[p]; o[4] = vy[p]; o[5] = vz[p];
+          }
+#pragma unroll
+        for (int p = 0; p < P; ++p) o_next[p] += hit ? 6 * n : 0;
+        rows.advance_if(hit);
+        if (rows.k == k + 1) { ++k; break; }  // the same row again
       }
-    // block-uniform: every particle is now at grid index k + 1 (or holds its initial row)
-    while (next < nsave && save_idx[next] == k + 1) {
+    }
+    // block-uniform: every particle is now at grid index k (or holds its initial row)
+    while (rows.due(k)) {
 #pragma unroll
       for (int p = 0; p < P; ++p)
         if (valid[p]) {
-          double* o = ys + ((int64_t)next * n + idx[p]) * 6;
+          double* o = ys + ((int64_t)rows.next * n + idx[p]) * 6;
           o[0] = x[p]; o[1] = y[p]; o[2] = z[p]; o[3] = vx[p]; o[4] = vy[p]; o[5] = vz[p];
         }
-      ++next;
+      rows.advance();
+      if (DENSE) aim();
     }
   }
 #pragma unroll
@@ -399,13 +466,13 @@ __global__ __launch_bounds__(LF_BLOCK) void leapfrog_group_kernel(
   lds.init(src, lds_raw);
   __syncthreads();
   const int kmin = kmin_sh;
-  int next = 0;
-  while (next < nsave && save_idx[next] <= kmin) {
+  SaveScan rows(save_idx, nsave);
+  while (rows.up_to(kmin)) {
     if (lead) {
-      double* o = ys + ((int64_t)next * n + i) * 6;
+      double* o = ys + ((int64_t)rows.next * n + i) * 6;
       o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
     }
-    ++next;
+    rows.advance();
   }
   const double h = 0.5 * dt;
   double ax = 0.0, ay = 0.0, az = 0.0;
@@ -413,23 +480,26 @@ __global__ __launch_bounds__(LF_BLOCK) void leapfrog_group_kernel(
     lds.stage(src, kmin, nsteps + 1);
     accel_group<SK, G, HS>(hp, lds, kmin, t0 + kmin * dt, r, x, y, z, ax, ay, az);
   }
-  for (int k = kmin; k < nsteps; ++k) {
-    lds.stage(src, k, nsteps + 1);
-    const bool act = k >= s;
-    if (act) {
-      vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
-      x = x + dt * vx; y = y + dt * vy; z = z + dt * vz;
+  for (int k = kmin; k < nsteps;) {
+    const int stop = rows.stop(k, nsteps);
+    for (; k < stop; ++k) {
+      lds.stage(src, k, nsteps + 1);
+      const bool act = k >= s;
+      if (act) {
+        vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
+        x = x + dt * vx; y = y + dt * vy; z = z + dt * vz;
+      }
+      accel_group<SK, G, HS>(hp, lds, k + 1, t0 + (k + 1) * dt, r, x, y, z, ax, ay, az);
+      if (act) {
+        vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
+      }
     }
-    accel_group<SK, G, HS>(hp, lds, k + 1, t0 + (k + 1) * dt, r, x, y, z, ax, ay, az);
-    if (act) {
-      vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
-    }
-    while (next < nsave && save_idx[next] == k + 1) {
+    while (rows.due(k)) {
       if (lead) {
-        double* o = ys + ((int64_t)next * n + i) * 6;
+        double* o = ys + ((int64_t)rows.next * n + i) * 6;
         o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
       }
-      ++next;
+      rows.advance();
     }
   }
   if (lead) {
@@ -459,7 +529,7 @@ __device__ __forceinline__ void accel_wave(const ssc_host_potential& hp, const S
   az = -(hz + gz);
 }
 
-template <int SK, int HS>
+template <int SK, int HS, bool DENSE>
 __global__ __launch_bounds__(WAVE) void leapfrog_wave_kernel(
     ssc_host_potential hp, ssc_sources src, const double* __restrict__ w0,
     const int32_t* __restrict__ start, int64_t n, double t0, double dt, int nsteps,
@@ -475,13 +545,13 @@ __global__ __launch_bounds__(WAVE) void leapfrog_wave_kernel(
   SourceLDS<SK> lds;
   lds.init(src, lds_raw);
   __syncthreads();
-  int next = 0;
-  while (next < nsave && save_idx[next] <= s) {
+  SaveRows rows(save_idx, nsave);
+  while (rows.up_to(s)) {
     if (lead) {
-      double* o = ys + ((int64_t)next * n + i) * 6;
+      double* o = ys + ((int64_t)rows.next * n + i) * 6;
       o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
     }
-    ++next;
+    rows.advance();
   }
   const double h = 0.5 * dt;
   double ax = 0, ay = 0, az = 0;
@@ -489,18 +559,33 @@ __global__ __launch_bounds__(WAVE) void leapfrog_wave_kernel(
     lds.template stage<8>(src, s, nsteps + 1);
     accel_wave<SK, HS>(hp, lds, s, t0 + s * dt, x, y, z, ax, ay, az);
   }
-  for (int k = s; k < nsteps; ++k) {
-    lds.template stage<8>(src, k, nsteps + 1);
-    vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
-    x = x + dt * vx; y = y + dt * vy; z = z + dt * vz;
-    accel_wave<SK, HS>(hp, lds, k + 1, t0 + (k + 1) * dt, x, y, z, ax, ay, az);
-    vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
-    while (next < nsave && save_idx[next] == k + 1) {
+  double* o_next = ys + ((int64_t)rows.next * n + i) * 6;  // DENSE: where the next saved row goes
+  for (int k = s; k < nsteps;) {
+    const int stop = DENSE ? nsteps : rows.stop(k, nsteps);
+    for (; k < stop; ++k) {
+      lds.template stage<8>(src, k, nsteps + 1);
+      vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
+      x = x + dt * vx; y = y + dt * vy; z = z + dt * vz;
+      accel_wave<SK, HS>(hp, lds, k + 1, t0 + (k + 1) * dt, x, y, z, ax, ay, az);
+      vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
+      if (DENSE) {
+        const bool hit = rows.k == k + 1;
+        if (hit && lead) {
+          double* o = o_next;
+          o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
+        }
+        o_next += hit ? 6 * n : 0;
+        rows.advance_if(hit);
+        if (rows.k == k + 1) { ++k; break; }  // the same row again
+      }
+    }
+    while (rows.due(k)) {
       if (lead) {
-        double* o = ys + ((int64_t)next * n + i) * 6;
+        double* o = ys + ((int64_t)rows.next * n + i) * 6;
         o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
       }
-      ++next;
+      rows.advance();
+      o_next += 6 * n;
     }
   }
   if (lead) {
@@ -555,35 +640,38 @@ __global__ __launch_bounds__(WAVE * SSC_MAX_COMPONENTS) void leapfrog_comp_kerne
     ax = -gx; ay = -gy; az = -gz;
     buf ^= 1;
   };
-  int next = 0;
-  while (next < nsave && save_idx[next] <= kmin) {
+  SaveRows rows(save_idx, nsave);
+  while (rows.up_to(kmin)) {
     if (writer) {
-      double* o = ys + ((int64_t)next * n + i) * 6;
+      double* o = ys + ((int64_t)rows.next * n + i) * 6;
       o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
     }
-    ++next;
+    rows.advance();
   }
   const double h = 0.5 * dt;
   double ax = 0.0, ay = 0.0, az = 0.0;
   if (kmin < nsteps) accel(ax, ay, az);
   // A particle that has not started keeps its initial row; the force evaluated there is the
   // initial force it needs when it starts.
-  for (int k = kmin; k < nsteps; ++k) {
-    const bool act = k >= s;
-    if (act) {
-      vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
-      x = x + dt * vx; y = y + dt * vy; z = z + dt * vz;
+  for (int k = kmin; k < nsteps;) {
+    const int stop = rows.stop(k, nsteps);
+    for (; k < stop; ++k) {
+      const bool act = k >= s;
+      if (act) {
+        vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
+        x = x + dt * vx; y = y + dt * vy; z = z + dt * vz;
+      }
+      accel(ax, ay, az);
+      if (act) {
+        vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
+      }
     }
-    accel(ax, ay, az);
-    if (act) {
-      vx = vx + h * ax; vy = vy + h * ay; vz = vz + h * az;
-    }
-    while (next < nsave && save_idx[next] == k + 1) {
+    while (rows.due(k)) {
       if (writer) {
-        double* o = ys + ((int64_t)next * n + i) * 6;
+        double* o = ys + ((int64_t)rows.next * n + i) * 6;
         o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
       }
-      ++next;
+      rows.advance();
     }
   }
   if (writer) {
@@ -614,19 +702,21 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                            double* w_out, const int32_t* save_idx, int nsave, double* ys, bool ragged,
                            hipStream_t st) {
   const size_t lds = SourceLDS<SK>::bytes(src);
+  const bool dense = nsave > nsteps / 2;  // see SaveRows
   if (SK != SSC_SRC_NONE && src.n >= 64 && n <= 1024) {
-    int rc = set_lds((const void*)leapfrog_wave_kernel<SK, HS>, lds);
+    auto kernel = dense ? leapfrog_wave_kernel<SK, HS, true> : leapfrog_wave_kernel<SK, HS, false>;
+    int rc = set_lds((const void*)kernel, lds);
     if (rc) return rc;
-    hipLaunchKernelGGL((leapfrog_wave_kernel<SK, HS>), dim3((unsigned)n), dim3(WAVE), lds, st, hp, src,
-                       w0, start, n, t0, dt, nsteps, w_out, save_idx, nsave, ys);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(WAVE), lds, st, hp, src, w0,
+                       start, n, t0, dt, nsteps, w_out, save_idx, nsave, ys);
     return check_launch("ssc_leapfrog");
   }
   if (SK != SSC_SRC_NONE && src.n >= 16 && n >= 393216 &&
       2 * ((n + 131071) / 131072) <= (n + 65535) / 65536) {
-    int rc = set_lds((const void*)leapfrog_kernel<SK, 2, HS>, lds);
+    int rc = set_lds((const void*)leapfrog_kernel<SK, 2, HS, false>, lds);
     if (rc) return rc;
     const int64_t blocks = (n + 2 * LF_BLOCK - 1) / (2 * LF_BLOCK);
-    hipLaunchKernelGGL((leapfrog_kernel<SK, 2, HS>), dim3((unsigned)blocks), dim3(LF_BLOCK), lds, st,
+    hipLaunchKernelGGL((leapfrog_kernel<SK, 2, HS, false>), dim3((unsigned)blocks), dim3(LF_BLOCK), lds, st,
                        hp, src, w0, start, n, t0, dt, nsteps, w_out, save_idx, nsave, ys);
     return check_launch("ssc_leapfrog");
   }
@@ -652,11 +742,13 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
   SSC_GROUP(8)
   SSC_GROUP(16)
 #undef SSC_GROUP
-  int rc = set_lds((const void*)leapfrog_kernel<SK, 1, HS>, lds);
+  auto kernel = SK == SSC_SRC_NONE && dense ? leapfrog_kernel<SK, 1, HS, SK == SSC_SRC_NONE>
+                                            : leapfrog_kernel<SK, 1, HS, false>;
+  int rc = set_lds((const void*)kernel, lds);
   if (rc) return rc;
   const int64_t blocks = (n + LF_BLOCK - 1) / LF_BLOCK;
-  hipLaunchKernelGGL((leapfrog_kernel<SK, 1, HS>), dim3((unsigned)blocks), dim3(LF_BLOCK), lds, st, hp,
-                     src, w0, start, n, t0, dt, nsteps, w_out, save_idx, nsave, ys);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(LF_BLOCK), lds, st, hp, src, w0, start, n,
+                     t0, dt, nsteps, w_out, save_idx, nsave, ys);
   return check_launch("ssc_leapfrog");
 }
 
