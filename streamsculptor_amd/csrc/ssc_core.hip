@@ -689,9 +689,10 @@ static int set_lds(const void* fn, size_t lds) {
   return SSC_OK;
 }
 
-// Launch shape: one wave per orbit while every orbit has a SIMD of its own and the table is
-// large (512 clumps: 1,000 orbits 1.81 us a step against 2.87 with 16 lanes an orbit, 2,000
-// orbits 4.39 against 2.96); two particles per lane for batches that fill the chip several times
+// Launch shape: one wave per orbit while every orbit has a SIMD of its own (512 clumps: 1,000
+// orbits 1.81 us a step against 2.87 with 16 lanes an orbit, 2,000 orbits 4.39 against 2.96; one
+// orbit in 20 tracked subhalos saved at every step 0.85 against 1.12, in 4 clumps 0.74 unsaved
+// against 0.70: from 8 sources on); two particles per lane for batches that fill the chip several times
 // over, unless the pairing costs a round of waves (512 clumps: 1e6 orbits 326 us against 331,
 // 4e5 169 against 153); group_lanes otherwise.  Without sources: for up to 65536 orbits in a
 // host of no known signature, host components over waves; one particle per lane otherwise (with
@@ -703,7 +704,7 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                            hipStream_t st) {
   const size_t lds = SourceLDS<SK>::bytes(src);
   const bool dense = nsave > nsteps / 2;  // see SaveRows
-  if (SK != SSC_SRC_NONE && src.n >= 64 && n <= 1024) {
+  if (SK != SSC_SRC_NONE && src.n >= 8 && n <= 1024) {
     auto kernel = dense ? leapfrog_wave_kernel<SK, HS, true> : leapfrog_wave_kernel<SK, HS, false>;
     int rc = set_lds((const void*)kernel, lds);
     if (rc) return rc;

@@ -21,6 +21,8 @@ def _rel(a, b):
 @pytest.mark.parametrize("kind,m,n,nsteps", [
     ("static", 64, 1024, 60),      # one wave per orbit, the last size ...
     ("static", 64, 1025, 60),      # ... and the first with 16 lanes an orbit
+    ("static", 8, 1024, 60),       # the smallest table of the wave kernel ...
+    ("line", 7, 1024, 60),         # ... and the largest of the lane groups
     ("tracked", 67, 4096, 40),     # 16 lanes, one wave per SIMD exactly, 67 = 16 x 4 + 3 sources
     ("tracked", 67, 4097, 40),     # 8 lanes
     ("static", 1, 1300, 40),       # one lane, one source
