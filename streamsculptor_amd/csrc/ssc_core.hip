@@ -441,15 +441,12 @@ __device__ __forceinline__ void accel_group(const ssc_host_potential& hp, const 
 }
 
 template <int SK, int G, int HS>
-__global__ __launch_bounds__(LF_BLOCK) void leapfrog_group_kernel(
-    ssc_host_potential hp, ssc_sources src, const double* __restrict__ w0,
-    const int32_t* __restrict__ start, int64_t n, double t0, double dt, int nsteps,
+__device__ __forceinline__ void leapfrog_group(
+    const ssc_host_potential& hp, const ssc_sources& src, const double* __restrict__ w0,
+    const int32_t* __restrict__ start, int64_t i, int64_t n, double t0, double dt, int nsteps,
     double* __restrict__ w_out, const int32_t* __restrict__ save_idx, int nsave,
-    double* __restrict__ ys) {
-  extern __shared__ __align__(16) char lds_raw[];
-  __shared__ int kmin_sh;
+    double* __restrict__ ys, char* lds_raw, int& kmin_sh) {
   const int r = threadIdx.x % G;
-  const int64_t i = (int64_t)blockIdx.x * (LF_BLOCK / G) + threadIdx.x / G;
   const bool valid = i < n, lead = valid && r == 0;
   int s = nsteps;
   double x = 1.0, y = 0.0, z = 0.0, vx = 0.0, vy = 0.0, vz = 0.0;
@@ -506,6 +503,24 @@ __global__ __launch_bounds__(LF_BLOCK) void leapfrog_group_kernel(
     double* o = w_out + 6 * i;
     o[0] = x; o[1] = y; o[2] = z; o[3] = vx; o[4] = vy; o[5] = vz;
   }
+}
+
+// The first n_whole orbits (whole rounds of waves) take one lane each, the rest G lanes.
+template <int SK, int G, int HS>
+__global__ __launch_bounds__(LF_BLOCK) void leapfrog_group_kernel(
+    ssc_host_potential hp, ssc_sources src, const double* __restrict__ w0,
+    const int32_t* __restrict__ start, int64_t n_whole, int64_t n, double t0, double dt, int nsteps,
+    double* __restrict__ w_out, const int32_t* __restrict__ save_idx, int nsave,
+    double* __restrict__ ys) {
+  extern __shared__ __align__(16) char lds_raw[];
+  __shared__ int kmin_sh;
+  const int64_t first = (int64_t)blockIdx.x * LF_BLOCK;
+  if (first < n_whole)
+    leapfrog_group<SK, 1, HS>(hp, src, w0, start, first + threadIdx.x, n, t0, dt, nsteps, w_out,
+                              save_idx, nsave, ys, lds_raw, kmin_sh);
+  else
+    leapfrog_group<SK, G, HS>(hp, src, w0, start, n_whole + (first - n_whole + threadIdx.x) / G, n,
+                              t0, dt, nsteps, w_out, save_idx, nsave, ys, lds_raw, kmin_sh);
 }
 
 // One wave per orbit: for a handful of orbits in a large source table (the progenitor in a
@@ -728,15 +743,17 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                        w_out, save_idx, nsave, ys);
     return check_launch("ssc_leapfrog");
   }
-  const int g = SK == SSC_SRC_NONE ? 1 : group_lanes(n, src.n, ragged);
+  int64_t n_whole = 0;
+  const int g = SK == SSC_SRC_NONE ? 1 : group_lanes(n, src.n, ragged, &n_whole);
 #define SSC_GROUP(GV)                                                                              \
   if (g == GV) {                                                                                   \
-    int rc = set_lds((const void*)leapfrog_group_kernel<SK, GV, HS>, lds);                            \
+    int rc = set_lds((const void*)leapfrog_group_kernel<SK, GV, HS>, lds);                         \
     if (rc) return rc;                                                                             \
-    const int64_t blocks = (n + LF_BLOCK / GV - 1) / (LF_BLOCK / GV);                              \
-    hipLaunchKernelGGL((leapfrog_group_kernel<SK, GV, HS>), dim3((unsigned)blocks), dim3(LF_BLOCK),   \
-                       lds, st, hp, src, w0, start, n, t0, dt, nsteps, w_out, save_idx, nsave, ys); \
-    return check_launch("ssc_leapfrog");                                                          \
+    const int64_t blocks = n_whole / LF_BLOCK + (n - n_whole + LF_BLOCK / GV - 1) / (LF_BLOCK / GV); \
+    hipLaunchKernelGGL((leapfrog_group_kernel<SK, GV, HS>), dim3((unsigned)blocks),                \
+                       dim3(LF_BLOCK), lds, st, hp, src, w0, start, n_whole, n, t0, dt, nsteps,    \
+                       w_out, save_idx, nsave, ys);                                                \
+    return check_launch("ssc_leapfrog");                                                           \
   }
   SSC_GROUP(2)
   SSC_GROUP(4)

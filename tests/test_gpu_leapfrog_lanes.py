@@ -1,7 +1,8 @@
 """The fixed-step stepper over its launch shapes with sources: one wave per orbit up to its last
 size, every number of lanes per orbit (source counts that are no multiple of four times the
 lanes, so that the blocks of four sources leave remainders), the sizes beside which the rule
-changes, and one or two orbits per lane for batches that fill the chip several times over.
+changes, whole rounds of waves at one lane per orbit with the remainder at several, and two
+orbits per lane for batches that fill the chip several times over.
 Ragged starts, saved rows; against the oracle on a sample of the orbits, <= 1e-9 relative."""
 import numpy as np
 import pytest
@@ -34,6 +35,9 @@ def _rel(a, b):
     ("static", 21, 393215, 4),     # the last size without pairs of orbits
     ("static", 21, 400000, 4),     # pairs would cost a round of waves
     ("static", 21, 524288, 4),     # two orbits per lane
+    ("tracked", 64, 65537, 12),    # one lane each, and one orbit more with 16
+    ("tracked", 13, 70001, 12),    # ... and a remainder that ends inside a block
+    ("static", 100, 131500, 6),    # two whole rounds and a remainder
 ])
 def test_launch_shapes(oracle, ssc, kind, m, n, nsteps):
     from streamsculptor_amd import _lib
