@@ -734,7 +734,7 @@ def main():
                           "frac": fl_p * ps / kern_p / PEAK_FP64,
                           "traffic": (TRAFFIC_CLUMPS_PLAIN if args.workload == "clumps"
                                       and wl["total"] == 1_000_000 else None),
-                          "kernel": ("perturb_base_kernel + perturb_rows_kernel (one launch chain)"
+                          "kernel": ("perturb_segment_kernel (one launch chain)"
                                      if args.workload == "responses" else
                                      "the whole stream: progenitor orbit, releases and particle "
                                      "leapfrog, pipelined" if args.workload in ("plain", "subhalos")

@@ -130,6 +130,13 @@ int ssc_leapfrog(const ssc_host_potential* host, const ssc_sources* src,
                  double t0, double dt, int32_t nsteps, double* w_out,
                  const int32_t* save_idx, int32_t nsave, double* ys, void* stream);
 
+/* ssc_leapfrog without saved rows for a window of a stream: the same rows up to rounding, for
+ * orbits most of which start at the window's first row (the launch is shaped for orbits that all
+ * walk the whole window; ssc_leapfrog with start_step for starts all along the grid). */
+int ssc_leapfrog_window(const ssc_host_potential* host, const ssc_sources* src,
+                        const double* w0, const int32_t* start_step, int64_t n,
+                        double t0, double dt, int32_t nsteps, double* w_out, void* stream);
+
 /* Step-size control of ssc_dopri5 (reference PIDController(rtol, atol, dtmin, dtmax,
  * force_dtmin=True, jump_ts), streamsculptor/main.py:146, fields.py:54). */
 typedef struct ssc_dopri5_options {

@@ -610,8 +610,8 @@ int ssc_adjoint_forward(const ssc_host_potential* host, const ssc_sources* src, 
   const int64_t nseg = nseg_of(nsteps, checkpoint_every);
   hipLaunchKernelGGL(ckpt_index_kernel, dim3((unsigned)((nseg + 256) / 256)), dim3(256), 0,
                      (hipStream_t)stream, w.save_idx, nseg, (int)checkpoint_every, (int)nsteps);
-  return leapfrog_run(host, src, w0, start_step, n, t0, dt, nsteps, w_out, w.save_idx,
-                      (int32_t)(nseg + 1), w.ckpt, start_step != nullptr, stream);
+  return ssc_leapfrog(host, src, w0, start_step, n, t0, dt, nsteps, w_out, w.save_idx,
+                      (int32_t)(nseg + 1), w.ckpt, stream);
 }
 
 int ssc_adjoint_checkpoints_from_rows(const double* rows, int64_t n, int32_t nsteps,

@@ -774,10 +774,11 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
 
 using namespace ssc;
 
-int ssc::leapfrog_run(const ssc_host_potential* host, const ssc_sources* src, const double* w0,
-                      const int32_t* start_step, int64_t n, double t0, double dt, int32_t nsteps,
-                      double* w_out, const int32_t* save_idx, int32_t nsave, double* ys,
-                      bool ragged, void* stream) {
+// ssc_leapfrog; `ragged`: the orbits start all along the grid (chooses the lanes per orbit only).
+static int leapfrog_run(const ssc_host_potential* host, const ssc_sources* src, const double* w0,
+                        const int32_t* start_step, int64_t n, double t0, double dt,
+                        int32_t nsteps, double* w_out, const int32_t* save_idx, int32_t nsave,
+                        double* ys, bool ragged, void* stream) {
   int rc = validate_host(host);
   if (rc) return rc;
   if (n < 0 || nsteps < 0 || nsave < 0) return fail(SSC_E_ARG, "ssc_leapfrog: negative size");
@@ -851,6 +852,13 @@ int ssc_leapfrog(const ssc_host_potential* host, const ssc_sources* src, const d
                  double* w_out, const int32_t* save_idx, int32_t nsave, double* ys,
                  void* stream) {
   return leapfrog_run(host, src, w0, start_step, n, t0, dt, nsteps, w_out, save_idx, nsave, ys,
+                      start_step != nullptr, stream);
+}
+
+int ssc_leapfrog_window(const ssc_host_potential* host, const ssc_sources* src, const double* w0,
+                        const int32_t* start_step, int64_t n, double t0, double dt,
+                        int32_t nsteps, double* w_out, void* stream) {
+  return leapfrog_run(host, src, w0, start_step, n, t0, dt, nsteps, w_out, nullptr, 0, nullptr,
                       false, stream);
 }
 

@@ -21,11 +21,6 @@ int fail(int code, const std::string& msg);
 int check_launch(const char* what);
 int validate_host(const ssc_host_potential* host);
 int validate_sources(const ssc_sources* src, int32_t nsteps_needed, bool allow_groups = false);
-// ssc_leapfrog; `ragged`: the orbits start all along the grid (chooses the lanes per orbit only).
-int leapfrog_run(const ssc_host_potential* host, const ssc_sources* src, const double* w0,
-                 const int32_t* start_step, int64_t n, double t0, double dt, int32_t nsteps,
-                 double* w_out, const int32_t* save_idx, int32_t nsave, double* ys, bool ragged,
-                 void* stream);
 
 // ------------------------------------------------------------------------------------------
 // small vector helpers

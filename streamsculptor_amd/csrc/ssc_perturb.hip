@@ -18,8 +18,9 @@
 // through a segment and records, at every row a particle is kicked at, its position and the host
 // Hessian; response_rows then advances the responses through the segment from those records.
 // One launch carries the base rows of segment s + 1 beside the responses of segment s: the first
-// waits for memory (72 B a particle and row), the second for FP64 issue.  Without a workspace perturb_kernel has each of the L lanes recompute the base
-// orbit and the host Hessian (2.2x the arithmetic of the split form, measured by counters).
+// waits for memory (72 B a particle and row), the second for FP64 issue.  Without a workspace
+// perturb_kernel has each of the L lanes recompute the base orbit and the host Hessian (2.2x the
+// arithmetic of the split form, measured by counters).
 // Velocities are carried at half steps so that forces are consumed as soon as they are formed.
 #include <hip/hip_runtime.h>
 

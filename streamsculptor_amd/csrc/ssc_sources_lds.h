@@ -80,9 +80,10 @@ struct SourceLDS<SSC_SRC_STATIC> {
       for (int p = 0; p < P; ++p)
         plummer_grad_k(x[p] - g.x, y[p] - g.y, z[p] - g.z, g.rs2, c.c1, c.c2, gx[p], gy[p], gz[p]);
     };
-    // four sources at a time, in order (see TrackLDS)
+    // four sources at a time, in order (see TrackLDS); two particles a lane interleave by
+    // themselves (1e6 particles of a stream, 512 clumps: 140.9 ms so, 137.6 one at a time)
     int j = j0;
-    for (; j + 3 * js < n; j += 4 * js) {
+    for (; P == 1 && j + 3 * js < n; j += 4 * js) {
       SrcGeo g[4];
       SrcK c[4];
 #pragma unroll

@@ -344,9 +344,10 @@ class Potential:
 
     # ------------------------------------------------------------------ integration
     def _leapfrog(self, w0, t0, dt, nsteps, start=None, save_idx=None, src_override=False,
-                  out=None):
+                  out=None, window=False):
         """Run ssc_leapfrog on rows w0 (n, 6); returns (w_final, ys or None); ``out``: contiguous
-        rows for w_final, other than w0."""
+        rows for w_final, other than w0; ``window``: most orbits start at the first row
+        (ssc_leapfrog_window, no saved rows)."""
         h, src = self._descriptor()
         w0 = _lib.f64(w0).reshape(-1, 6).contiguous()
         n = w0.shape[0]
@@ -359,10 +360,12 @@ class Potential:
         if src is not None and src.kind in _lib.TRACK_KINDS:
             src = src.on_grid(t0, dt, nsteps)
         sd = src.desc() if src is not None else None
-        _lib.call("ssc_leapfrog", _lib.ctypes.byref(h),
-                  None if sd is None else _lib.ctypes.byref(sd), _lib.ptr(w0), _lib.ptr(st), n,
-                  float(t0), float(dt), int(nsteps), _lib.ptr(out), _lib.ptr(si), nsave,
-                  _lib.ptr(ys))
+        args = (_lib.ctypes.byref(h), None if sd is None else _lib.ctypes.byref(sd), _lib.ptr(w0),
+                _lib.ptr(st), n, float(t0), float(dt), int(nsteps), _lib.ptr(out))
+        if window:
+            _lib.call("ssc_leapfrog_window", *args)
+        else:
+            _lib.call("ssc_leapfrog", *args, _lib.ptr(si), nsave, _lib.ptr(ys))
         return out, ys
 
     def integrate_orbit(self, w0=None, ts=None, dense=False, solver=None, rtol=1e-7, atol=1e-7,

@@ -126,7 +126,7 @@ def _leapfrog_stream_pipelined(prog_pot, release_pot, particle_pot, ts_np, prog_
                 w_in, w_out = rows[c % 2][:2 * b], rows[(c + 1) % 2][:2 * b]
                 w_in[2 * a:].view(b - a, 2, 6).copy_(table[0].transpose(0, 1))
                 particle_pot._leapfrog(w_in, t0 + g0 * dt, dt, g1 - g0, start=start_all[c],
-                                       out=w_out)
+                                       out=w_out, window=True)
     finally:
         main.wait_stream(side)
     return w_out
@@ -210,16 +210,20 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
     from .main import _as_float
     from .workloads import spray_layout
     particle_pot = particle_pot or prog_pot
+    whole = window = integrate
     if integrate is None:
-        def integrate(w, t_start, step, n, start):
+        def whole(w, t_start, step, n, start):
             return particle_pot._leapfrog(w, t_start, step, n, start=start)[0]
+
+        def window(w, t_start, step, n, start):
+            return particle_pot._leapfrog(w, t_start, step, n, start=start, window=True)[0]
     ts_np = np.asarray(ts, dtype=np.float64).reshape(-1)
     T = len(ts_np) - 1
     if (chunks <= 1 or T < 4 * chunks or not _restartable(prog_pot)
             or not _restartable(particle_pot)):
         w0, start, _, (t0, dt, nsteps, _) = spray_particles(
             prog_pot, release_pot, ts_np, prog_w0, Msat, seed_num, per_step, dt0, kval_arr)
-        return integrate(w0, t0, dt, nsteps, start)
+        return whole(w0, t0, dt, nsteps, start)
     t0, dt, nsteps, kidx = release_grid(ts_np, dt0)
     dev = _lib.device()
     nseed = (per_step + 1) // 2
@@ -270,7 +274,7 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
             side.wait_stream(spray)
             with torch.cuda.stream(side):
                 w_in = new if state is None else torch.cat([state, new], 0)
-                state = integrate(w_in, t0 + g0 * dt, dt, g1 - g0, start)
+                state = window(w_in, t0 + g0 * dt, dt, g1 - g0, start)
     finally:
         main.wait_stream(spray)
         main.wait_stream(side)

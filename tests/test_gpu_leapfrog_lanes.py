@@ -3,7 +3,8 @@ size, every number of lanes per orbit (source counts that are no multiple of fou
 lanes, so that the blocks of four sources leave remainders), the sizes beside which the rule
 changes, whole rounds of waves at one lane per orbit with the remainder at several, and two
 orbits per lane for batches that fill the chip several times over.
-Ragged starts, saved rows; against the oracle on a sample of the orbits, <= 1e-9 relative."""
+Ragged starts, saved rows, and the same rows by the entry point for a stream's window, whose rule
+the sizes are those of; against the oracle on a sample of the orbits, <= 1e-9 relative."""
 import numpy as np
 import pytest
 import torch
@@ -77,10 +78,15 @@ def test_launch_shapes(oracle, ssc, kind, m, n, nsteps):
     _lib.call("ssc_leapfrog", _lib.ctypes.byref(hd), _lib.ctypes.byref(sd), _lib.ptr(wd),
               _lib.ptr(st), n, t0, dt, nsteps, _lib.ptr(out), _lib.ptr(si), len(save),
               _lib.ptr(ys))
+    # the same starts through the launch shaped for orbits that all walk the whole window
+    win = torch.empty_like(wd)
+    _lib.call("ssc_leapfrog_window", _lib.ctypes.byref(hd), _lib.ctypes.byref(sd), _lib.ptr(wd),
+              _lib.ptr(st), n, t0, dt, nsteps, _lib.ptr(win))
     torch.cuda.synchronize()
     pick = np.unique(np.concatenate([[0, n - 1], rng.integers(0, n, 250)]))
     final, traj = oracle.leapfrog(h, w0[pick], t0, dt, nsteps, start=start[pick], src=osrc,
                                   traj=True)
     assert _rel(out.cpu().numpy()[pick], final) <= 1e-9
+    assert _rel(win.cpu().numpy()[pick], final) <= 1e-9
     for k, y in zip(save, ys.cpu().numpy()):
         assert _rel(y[pick], traj[k]) <= 1e-9
