@@ -25,21 +25,6 @@ constexpr double M1 = 6025192743.0 / 30085553152.0 / 2, M3 = 51252292925.0 / 654
                  M5 = 187940372067.0 / 1594534317056.0 / 2,
                  M6 = -1776094331.0 / 19743644256.0 / 2, M7 = 11237099.0 / 235043384.0 / 2;
 
-// The integral controller's step factor 0.9 (1 / e)^(1/5) before its limits [0.2 or 1, 10].  A
-// library pow takes about 870 cycles on a wave by itself, every step; here the inverse fifth
-// root comes from a single-precision exp2/log2 estimate (relative error below 1e-6) and one
-// third-order correction, y (1 + r/5 + 3 r^2/25), r = 1 - e y^5, whose first omitted term is
-// below 1e-18: about 20 instructions, within two units in the last place.  e is held to
-// [1e-7, 1e5], outside of which the limits decide; NaN counts as the upper end (the lower limit
-// of the factor, as with pow).
-__device__ __forceinline__ double step_factor(double e) {
-  const double ec = e < 1e5 ? fmax(e, 1e-7) : 1e5;
-  const double y = (double)__builtin_amdgcn_exp2f(-0.2f * __builtin_amdgcn_logf((float)ec));
-  const double y2 = y * y;
-  const double r = fma(-ec * y, y2 * y2, 1.0);
-  return 0.9 * fma(y * r, fma(0.12, r, 0.2), y);
-}
-
 struct Dp5Ctl {
   double rtol, atol, dtmin, dtmax, dt0;  // dtmin / dtmax / dt0 <= 0: none / none / heuristic
   int max_steps;

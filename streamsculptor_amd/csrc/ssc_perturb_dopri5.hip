@@ -17,15 +17,18 @@
 // the base row on its own first six lanes (the copies stay equal bit for bit), so the stage row
 // reaches the wave's lanes without a barrier.  The host terms are the long serial chain of a
 // stage: a group of several waves deals the host components out to its waves, each wave's
-// component fixed, so that the kinds of code run side by side, and they meet in LDS after one
+// components fixed, so that the kinds of code run side by side, and they meet in LDS after one
 // barrier (two buffers); a group of up to one wave forms all components in every lane and its
 // loop holds no barrier at all, so the waves of a block run on their own.  (Lanes of one wave
 // forming components of different kinds ran the kinds one after the other, their parameters
-// fetched through vector memory at every stage, between two barriers.)  What bounds a step now is
-// instruction latency: about 1,800 vector and 560 scalar instructions a wave and step, two waves
-// a SIMD in 256 registers.  One particle with 256 response vectors: 16.4 -> 8.2 us a step; 1,000
-// of them, their responses to 128 Hernquist subhalos with the radius block over 1,500 Myr on
-// average at rtol = atol = 1e-8: 29 -> 14.6 ms.
+// fetched through vector memory at every stage, between two barriers.)  The rows are that form's
+// bit for bit, which is why divisions, square roots, log1p and pow are the library's or equal to
+// them: shorter forms would take another 40 % off a step.  What bounds a step is instruction
+// latency -- the wave with the halo's log1p, 130 instructions in a chain, at every stage -- with
+// two waves a SIMD in 256 registers.  One particle with 256 response vectors: 16.4 -> 13.5 us a
+// step; 1,000 of them, their responses to 128 Hernquist subhalos with the radius block over
+// 1,500 Myr on average at rtol = atol = 1e-8: 29 -> 24.5 ms; 20,000 particles with 3 vectors
+// over 800 Myr 12.7 -> 8.8 ms.
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -47,17 +50,23 @@ constexpr int PD_GROUPS = PD_BLOCK / PD_MIN_L;
 constexpr int PD_WAVES = PD_BLOCK / 64;
 
 // Sum of v over the L lanes of a particle group, bit-identical in every lane of the group:
-// within a wave each pairwise sum has the same two operands in both partner lanes (data-parallel
-// moves and lane swaps, no trip through the LDS unit); groups wider than a wave add their wave
-// partials in wave order through LDS (one barrier, taken when L > 64, which is uniform over the
-// launch).  Every lane of the wave must be active.
+// within a wave the butterfly of lane ^ 32, 16, 8, 4, 2, 1 (those below L), the widest first, each
+// pairwise sum with the same two operands in both partner lanes.  It is made of data-parallel
+// moves and lane swaps, no trip through the LDS unit: after the lane ^ 8 sum a row of 16 lanes
+// repeats with period 8, so that a rotation by 4 brings lane ^ 4.  Groups wider than a wave add
+// their wave partials in wave order through LDS (one barrier, taken when L > 64, which is uniform
+// over the launch).  Every lane of the wave must be active.
 __device__ __forceinline__ double part_sum(double v, int L, double* part) {
-  switch (L) {
-    case 8: return group_sum<8>(v);
-    case 16: return group_sum<16>(v);
-    case 32: return group_sum<32>(v);
-    default: v = group_sum<64>(v);
+  if (L >= 64) v = swap_sum<32>(v);
+  if (L >= 32) v = swap_sum<16>(v);
+  if (L >= 16) {
+    v += dpp_move<0x128>(v);  // row_ror:8, lane ^ 8
+    v += dpp_move<0x124>(v);  // row_ror:4
+  } else {
+    v += dpp_move<0x141>(dpp_move<0x1B>(v));  // lane ^ 3 of lane ^ 7
   }
+  v += dpp_move<0x4E>(v);  // quad_perm [2,3,0,1], lane ^ 2
+  v += dpp_move<0xB1>(v);  // quad_perm [1,0,3,2], lane ^ 1
   if (L <= 64) return v;
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -67,20 +76,37 @@ __device__ __forceinline__ double part_sum(double v, int L, double* part) {
   return s;
 }
 
+// Roundings.  The step-size controller turns a last-bit change of a force into another, equally
+// valid step sequence, and the windows of the subhalos make the right-hand side jump inside
+// steps: last bits of the host forms moved a response by up to 5e-8.  Every sum of products is
+// therefore written as the FMAs it is (which product of a sum is fused must not follow from what
+// is inlined around it), and divisions and square roots are correctly rounded.
+
+// a x + b y: the first product fused into the rounded second.
+__device__ __forceinline__ double dot2(double a, double x, double b, double y) {
+  return fma(a, x, b * y);
+}
+// x y rounded, also where the next operation adds it.
+__device__ __forceinline__ double mul_rn(double x, double y) { return fma(x, y, 0.0); }
+
 // Stage inputs: S = 0 the state itself, 1..5 the Dormand-Prince stages 2..6, 6 the 5th-order
-// solution (input of the FSAL stage), 7 the starting-step probe y + h f0.
-template <int S>
+// solution (input of the FSAL stage), 7 the starting-step probe y + h f0.  B3FIRST: the order of
+// the solution's first two terms (the response vectors' velocities; the base row has B1 first).
+template <int S, bool B3FIRST = false>
 __device__ __forceinline__ double stage_in(double y, const double (&k)[7], double h) {
   if constexpr (S == 0) return y;
-  if constexpr (S == 1) return y + h * (A21 * k[0]);
-  if constexpr (S == 2) return y + h * (A31 * k[0] + A32 * k[1]);
-  if constexpr (S == 3) return y + h * (A41 * k[0] + A42 * k[1] + A43 * k[2]);
-  if constexpr (S == 4) return y + h * (A51 * k[0] + A52 * k[1] + A53 * k[2] + A54 * k[3]);
+  if constexpr (S == 1) return fma(h, A21 * k[0], y);
+  if constexpr (S == 2) return fma(h, dot2(A31, k[0], A32, k[1]), y);
+  if constexpr (S == 3) return fma(h, fma(A43, k[2], dot2(A41, k[0], A42, k[1])), y);
+  if constexpr (S == 4)
+    return fma(h, fma(A54, k[3], fma(A53, k[2], dot2(A51, k[0], A52, k[1]))), y);
   if constexpr (S == 5)
-    return y + h * (A61 * k[0] + A62 * k[1] + A63 * k[2] + A64 * k[3] + A65 * k[4]);
-  if constexpr (S == 6)
-    return y + h * (B1 * k[0] + B3 * k[2] + B4 * k[3] + B5 * k[4] + B6 * k[5]);
-  if constexpr (S == 7) return y + h * k[0];
+    return fma(h, fma(A65, k[4], fma(A64, k[3], fma(A63, k[2], dot2(A61, k[0], A62, k[1])))), y);
+  if constexpr (S == 6) {
+    const double b = B3FIRST ? dot2(B3, k[2], B1, k[0]) : dot2(B1, k[0], B3, k[2]);
+    return fma(h, fma(B6, k[5], fma(B5, k[4], fma(B4, k[3], b))), y);
+  }
+  if constexpr (S == 7) return fma(h, k[0], y);
   return 0.0;
 }
 // Output slot of stage S (the probe reuses slot 1, which the first step overwrites).
@@ -97,31 +123,33 @@ __device__ __forceinline__ double stage_c() {
   return 0.0;
 }
 
+// err / (atol + rtol max(|y|, |yn|)) of a component with stored slopes.
 __device__ __forceinline__ double err_of(double y, const double (&k)[7], double yn, double h,
                                          const Dp5Ctl& ctl) {
   const double err =
-      h * (E1 * k[0] + E3 * k[2] + E4 * k[3] + E5 * k[4] + E6 * k[5] + E7 * k[6]);
-  const double u = err * recip(ctl.atol + ctl.rtol * fmax(fabs(y), fabs(yn)));
-  return u * u;
+      h * fma(E7, k[6], fma(E6, k[5], fma(E5, k[4], fma(E4, k[3], dot2(E1, k[0], E3, k[2])))));
+  const double u = div_rn(err, fma(ctl.rtol, fmax(fabs(y), fabs(yn)), ctl.atol));
+  return u;
 }
 
 // Quartic through y (s = 0), yn (s = 1), slopes F0 = h f0 and F7 = h f7, and the midpoint
 // value ym, at s in (0, 1).
-__device__ __forceinline__ double quartic(double y, double yn, double F0, double F7, double ym,
-                                          double s) {
-  const double D1 = yn - y - F0, D2 = F7 - F0, D3 = ym - y - 0.5 * F0;
-  const double a4 = 2.0 * D2 - 8.0 * D1 + 16.0 * D3;
-  const double b3 = D2 - 2.0 * D1 - 2.0 * a4;
+__device__ __forceinline__ double quartic(double y, double yn, double h, double f0, double f7,
+                                          double ym, double s) {
+  const double F0 = h * f0;
+  const double D1 = fma(-h, f0, yn - y), D2 = fma(h, f7, -F0), D3 = fma(-0.5, F0, ym - y);
+  const double a4 = fma(16.0, D3, fma(-8.0, D1, 2.0 * D2));
+  const double b3 = fma(-2.0, a4, fma(-2.0, D1, D2));
   const double c2 = D1 - a4 - b3;
-  return y + s * (F0 + s * (c2 + s * (b3 + s * a4)));
+  return fma(s, fma(s, fma(s, fma(s, a4, b3), c2), F0), y);
 }
 
 // Dense output of a component with stored slopes k[0..6].
 __device__ __forceinline__ double dense_at(double y, const double (&k)[7], double yn, double h,
                                            double s) {
-  const double ym =
-      y + h * (M1 * k[0] + M3 * k[2] + M4 * k[3] + M5 * k[4] + M6 * k[5] + M7 * k[6]);
-  return quartic(y, yn, h * k[0], h * k[6], ym, s);
+  const double ym = fma(
+      h, fma(M7, k[6], fma(M6, k[5], fma(M5, k[4], fma(M4, k[3], dot2(M1, k[0], M3, k[2]))))), y);
+  return quartic(y, yn, h, k[0], k[6], ym, s);
 }
 
 // Position components of a response vector keep no slopes of their own: the slope of position
@@ -180,7 +208,7 @@ __device__ __forceinline__ double pos_sum(double x0, double v0, const double (&k
     return x0;
   } else {
     constexpr double c = ccoef(T);
-    return x0 + dir * h * (c * v0 + h * qsum<T, 5>(kv));
+    return fma(dir * h, dot2(c, v0, h, qsum<T, 5>(kv)), x0);
   }
 }
 
@@ -192,7 +220,82 @@ __device__ __forceinline__ double part_bcast(double v, int src, int w) {
   return __shfl(v, src, w);
 }
 
-template <int SK, int RAD, int G>
+// v^(1/5) by the library's pow, called: inlined, its constants took registers from the whole step
+// loop and 50 spills with them (1,000 particles x 16 Hernquist subhalos with the radius block, 800
+// Myr: 3.88 -> 3.48 ms).
+__device__ __noinline__ double fifth_root(double v) { return pow(v, 0.2); }
+
+// One host component's gradient and Hessian upper triangle, g[3] then H[0, 1, 2, 4, 5, 8] (the
+// forms of comp_full).
+constexpr int PARTS = 9;
+__device__ __forceinline__ void host_part(const ssc_component& c, double x, double y, double z,
+                                          double* o) {
+  const double gm = c.p[0];
+  const double xy2 = dot2(x, x, y, y);
+  double f = 0.0, k = 0.0;  // spherical components: grad = f (x, y, z), H = f I + k (x, y, z)^2
+  switch (c.kind) {
+    case SSC_COMP_MIYAMOTO_NAGAI: {
+      const double a = c.p[1], b = c.p[2], z2 = z * z;
+      const double zeta = sqrt_rn(fma(b, b, z2));
+      const double S = a + zeta;
+      const double D2 = fma(S, S, xy2);
+      const double iD3 = div_rn(1.0, D2 * sqrt_rn(D2));
+      const double dz = div_rn(z * S, zeta);
+      const double m = -3.0 * gm * div_rn(iD3, D2), d = gm * iD3;
+      const double w = div_rn(S * b * b, zeta * (zeta * zeta)) + div_rn(z2, zeta * zeta);
+      o[0] = mul_rn(gm * x, iD3);
+      o[1] = mul_rn(gm * y, iD3);
+      o[2] = mul_rn(gm * dz, iD3);
+      o[3] = fma(m * x, x, d);
+      o[4] = mul_rn(m * x, y);
+      o[5] = mul_rn(m * x, dz);
+      o[6] = fma(m * y, y, d);
+      o[7] = mul_rn(m * y, dz);
+      o[8] = dot2(gm * w, iD3, m * dz, dz);
+      return;
+    }
+    case SSC_COMP_NFW: {
+      const double rs = c.p[1];
+      const double r = sqrt_rn(fma(z, z, xy2));
+      const double L = log1p(div_rn(r, rs));
+      const double rp = r + rs, r2 = r * r;
+      const double d1 = gm * (div_rn(L, r2) - div_rn(1.0, r * rp));
+      const double d2 = gm * (div_rn(1.0, r2 * rp) - div_rn(2.0 * L, r * r2) +
+                              div_rn(fma(2.0, r, rs), r2 * rp * rp));
+      f = div_rn(d1, r);
+      k = div_rn(d2 - f, r2);
+      break;
+    }
+    case SSC_COMP_HERNQUIST: {
+      const double r = sqrt_rn(fma(z, z, xy2) + c.p[2]);
+      const double rc = r + c.p[1], rc2 = rc * rc;
+      f = div_rn(div_rn(gm, rc2), r);
+      k = div_rn(div_rn(-2.0 * gm, rc * rc2) - f, r * r);
+      break;
+    }
+    case SSC_COMP_PLUMMER: {
+      const double rs = c.p[1];
+      const double s2 = fma(rs, rs, fma(z, z, xy2));
+      f = gm * div_rn(1.0, s2 * sqrt_rn(s2));
+      k = div_rn(-3.0 * f, s2);
+      break;
+    }
+    default:
+      break;
+  }
+  o[0] = mul_rn(f, x);
+  o[1] = mul_rn(f, y);
+  o[2] = mul_rn(f, z);
+  o[3] = fma(k * x, x, f);
+  o[4] = mul_rn(k * x, y);
+  o[5] = mul_rn(k * x, z);
+  o[6] = fma(k * y, y, f);
+  o[7] = mul_rn(k * y, z);
+  o[8] = fma(k * z, z, f);
+}
+
+// WIDE: groups of several waves (L > 64).
+template <int SK, int RAD, int G, bool WIDE>
 __global__ __launch_bounds__(PD_BLOCK) __attribute__((amdgpu_waves_per_eu(G == 1 ? 2 : 1,
                                                                           G == 1 ? 2 : 1)))
 void perturb_dopri5_kernel(
@@ -203,11 +306,9 @@ void perturb_dopri5_kernel(
     double* __restrict__ dys, int32_t* __restrict__ stats) {
   extern __shared__ __align__(16) char lds_raw[];
   __shared__ double part_sh[2][PD_WAVES];
-  __shared__ __align__(16) CompQuad hg_sh[2][PD_WAVES / 2][SSC_MAX_COMPONENTS];  // wide groups
+  __shared__ double hg_sh[WIDE ? 2 : 1][PD_WAVES / 2][SSC_MAX_COMPONENTS][PARTS];
   constexpr int DD = RAD ? 12 : 6;
   constexpr bool HQ = SK == SSC_SRC_LINE_HERNQUIST;
-  if (threadIdx.x < 2 * (PD_WAVES / 2) * SSC_MAX_COMPONENTS)
-    (&hg_sh[0][0][0])[threadIdx.x] = CompQuad{0.0, 0.0, 0.0, 0.0};
   SourceLDS<SK> lds;
   lds.init(pert, lds_raw);  // barrier inside
 
@@ -217,10 +318,9 @@ void perturb_dopri5_kernel(
   const int gi = threadIdx.x / L, lane = threadIdx.x - gi * L;
   const int64_t i = (int64_t)blockIdx.x * ppb + gi;
   const bool valid = i < n;
-  const bool wide = L > 64;                          // several waves per particle
-  const int WL = wide ? 64 : L;                      // lanes of the group in one wave
-  const int nw = wide ? L >> 6 : 1;
-  const int wi = __builtin_amdgcn_readfirstlane(wide ? lane >> 6 : 0);  // wave of the group
+  const int WL = WIDE ? 64 : L;                      // lanes of the group in one wave
+  const int nw = WIDE ? L >> 6 : 1;
+  const int wi = __builtin_amdgcn_readfirstlane(WIDE ? lane >> 6 : 0);  // wave of the group
   const int wl = lane & (WL - 1);
   const int bc = wl < 6 ? wl : -1;                   // carried base component
   const bool bw = lane < 6;                          // the copy that counts and is written
@@ -279,7 +379,7 @@ void perturb_dopri5_kernel(
           continue;
         }
         const double x0 = y[q][c], v0 = y[q][3 + c];
-        o[c] = quartic(x0, yn[q][c], dir * h * v0, dir * h * yn[q][3 + c],
+        o[c] = quartic(x0, yn[q][c], dir * h, v0, yn[q][3 + c],
                        pos_sum<9>(x0, v0, kv[q][c], h, dir), s);
         o[3 + c] = dense_at(v0, kv[q][c], yn[q][3 + c], h, s);
       }
@@ -305,7 +405,13 @@ void perturb_dopri5_kernel(
   bool live = valid && tau0 < tau1;
   int hb = 0, pb = 0;
   const int nc = hp.n_components;
-  const ssc_component mine = hp.c[wi < nc ? wi : 0];  // this wave's host component (wide groups)
+  // this wave's host components (wide groups): neighbours in the list, so that two waves part disk
+  // + bulge and halo, whose log1p outlasts the others together
+  // this wave's host components (wide groups), neighbours in the list: two waves then part disk and
+  // bulge from the halo, whose log1p outlasts both (halo and disk on one wave: 4.0 against 3.6 ms
+  // for 500 particles x 64 Hernquist subhalos with the radius block, 800 Myr)
+  const int per = (nc + nw - 1) / nw, c_lo = wi * per, c_hi = c_lo + per < nc ? c_lo + per : nc;
+  const ssc_component mine = hp.c[c_lo < nc ? c_lo : 0];
 
   // Stage S at tau_s = tau + c_S h.  A wave whose particles have all finished only keeps the
   // barriers of a wide block; lanes of finished particles of a live wave compute unused values
@@ -318,46 +424,48 @@ void perturb_dopri5_kernel(
     double xv[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) xv[c] = part_bcast(bval, c, WL);
-    double g[3] = {0.0, 0.0, 0.0}, H[9];
+    double P[PARTS];  // the components' parts, added in component order
 #pragma unroll
-    for (int r = 0; r < 9; ++r) H[r] = 0.0;
-    if (wide) {
-      if (wi < nc) {
-        const CompQuad cq = comp_quad(mine, xv[0], xv[1], xv[2]);
-        if (wl == 0) hg_sh[hb][gi][wi] = cq;
-      }
-      for (int c = wi + nw; c < nc; c += nw) {  // a host of more components than waves
-        const CompQuad cq = comp_quad(hp.c[c], xv[0], xv[1], xv[2]);
-        if (wl == 0) hg_sh[hb][gi][c] = cq;
+    for (int r = 0; r < PARTS; ++r) P[r] = 0.0;
+    if constexpr (WIDE) {
+      ssc_component k = mine;
+      for (int c = c_lo; c < c_hi;) {
+        double o[PARTS];
+        host_part(k, xv[0], xv[1], xv[2], o);
+        if (wl == 0)
+#pragma unroll
+          for (int r = 0; r < PARTS; ++r) hg_sh[hb][gi][c][r] = o[r];
+        ++c;
+        if (c < c_hi) k = hp.c[c];
       }
       __syncthreads();
-      // the first three slots in one batch of reads (empty ones hold zeros; a loop with one LDS
-      // round trip per component: 8.8 against 8.2 us a step)
-      CompQuad cq[3];
+      for (int c = 0; c < nc; ++c)
 #pragma unroll
-      for (int c = 0; c < 3; ++c) cq[c] = hg_sh[hb][gi][c];
-#pragma unroll
-      for (int c = 0; c < 3; ++c) quad_add(cq[c], xv[0], xv[1], g, H);
-      for (int c = 3; c < nc; ++c) quad_add(hg_sh[hb][gi][c], xv[0], xv[1], g, H);
+        for (int r = 0; r < PARTS; ++r) P[r] += hg_sh[hb][gi][c][r];
       hb ^= 1;
     } else {
-      for (int c = 0; c < nc; ++c)
-        quad_add(comp_quad(hp.c[c], xv[0], xv[1], xv[2]), xv[0], xv[1], g, H);
+      for (int c = 0; c < nc; ++c) {
+        double o[PARTS];
+        host_part(hp.c[c], xv[0], xv[1], xv[2], o);
+#pragma unroll
+        for (int r = 0; r < PARTS; ++r) P[r] += o[r];
+      }
     }
-    H[3] = H[1]; H[6] = H[2]; H[7] = H[5];
+    const double g[3] = {P[0], P[1], P[2]};
+    const double H[9] = {P[3], P[4], P[5], P[4], P[6], P[7], P[5], P[7], P[8]};
     if (bc >= 0) {
       const double gb = bc == 3 ? g[0] : (bc == 4 ? g[1] : g[2]);
       const double vb = bc == 0 ? xv[3] : (bc == 1 ? xv[4] : xv[5]);
       bk[O] = bc < 3 ? dir * vb : -dir * gb;
     }
-    const double t = dir * (tau + stage_c<S>() * h);
+    const double t = dir * fma(stage_c<S>(), h, tau);
 #pragma unroll
     for (int q = 0; q < G; ++q) {
       double yt[6];
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         yt[c] = pos_sum<S>(y[q][c], y[q][3 + c], kv[q][c], h, dir);
-        yt[3 + c] = stage_in<S>(y[q][3 + c], kv[q][c], h);
+        yt[3 + c] = stage_in<S, true>(y[q][3 + c], kv[q][c], h);
       }
       if (S == 6)
 #pragma unroll
@@ -369,7 +477,7 @@ void perturb_dopri5_kernel(
       if (HQ) {      // qs = a
         const double r2 = fma(ex, ex, fma(ey, ey, ez * ez));
         const double ir = rsq(r2);
-        const double ia = recip(fma(r2, ir, qs));
+        const double ia = div_rn(1.0, fma(r2, ir, qs));
         f = gm * ir * ia * ia;
         fr = -2.0 * f * ia;
       } else {  // qs = a^2
@@ -380,10 +488,11 @@ void perturb_dopri5_kernel(
       // an inactive source contributes nothing whatever its position
       const double ff = vh[q] && act ? (voff[q] ? fr : f) : 0.0;
       const bool on = vh[q] && act;
-      const double fx = on ? ff * ex : 0.0, fy = on ? ff * ey : 0.0, fz = on ? ff * ez : 0.0;
-      const double hx = H[0] * yt[0] + H[1] * yt[1] + H[2] * yt[2];
-      const double hy = H[3] * yt[0] + H[4] * yt[1] + H[5] * yt[2];
-      const double hz = H[6] * yt[0] + H[7] * yt[1] + H[8] * yt[2];
+      const double fx = on ? mul_rn(ff, ex) : 0.0, fy = on ? mul_rn(ff, ey) : 0.0,
+                   fz = on ? mul_rn(ff, ez) : 0.0;
+      const double hx = fma(H[2], yt[2], dot2(H[0], yt[0], H[1], yt[1]));
+      const double hy = fma(H[5], yt[2], dot2(H[3], yt[0], H[4], yt[1]));
+      const double hz = fma(H[8], yt[2], dot2(H[6], yt[0], H[7], yt[1]));
       kv[q][0][O] = -dir * (fx + hx);
       kv[q][1][O] = -dir * (fy + hy);
       kv[q][2][O] = -dir * (fz + hz);
@@ -449,7 +558,7 @@ void perturb_dopri5_kernel(
       }
       const double d2 = sqrt(reduce(s2) / ntot) / h0;
       const double md = fmax(d1, d2);
-      const double h1 = md <= 1e-15 ? fmax(1e-6, h0 * 1e-3) : pow(0.01 / md, 0.2);
+      const double h1 = md <= 1e-15 ? fmax(1e-6, h0 * 1e-3) : fifth_root(0.01 / md);
       dt0 = fmin(100.0 * h0, h1);
     }
     // the first step is clamped to [dtmin, dtmax] like every later one (a first step raised
@@ -467,8 +576,8 @@ void perturb_dopri5_kernel(
   // of several waves share its barriers; with one group per block every wave forms the same
   // `live`.
   auto more = [&]() -> bool {
-    if (L == PD_BLOCK) return __builtin_amdgcn_readfirstlane(live ? 1 : 0) != 0;
-    if (wide) return __syncthreads_or(live ? 1 : 0) != 0;
+    if (WIDE && L == PD_BLOCK) return __builtin_amdgcn_readfirstlane(live ? 1 : 0) != 0;
+    if (WIDE) return __syncthreads_or(live ? 1 : 0) != 0;
     return __any(live ? 1 : 0) != 0;
   };
   while (more()) {
@@ -481,23 +590,28 @@ void perturb_dopri5_kernel(
     stage(std::integral_constant<int, 6>{}, tprev, h);
     double ss = 0.0;
     if (live) {
-      if (bw) ss = err_of(by, bk, byn, h, ctl);
+      if (bw) {
+        const double u = err_of(by, bk, byn, h, ctl);
+        ss = u * u;
+      }
 #pragma unroll
       for (int q = 0; q < G; ++q)
         if (vh[q])
 #pragma unroll
           for (int c = 0; c < 3; ++c) {
-            ss += err_of(y[q][3 + c], kv[q][c], yn[q][3 + c], h, ctl);
+            const double uv = err_of(y[q][3 + c], kv[q][c], yn[q][3 + c], h, ctl);
+            ss = fma(uv, uv, ss);
             const double ex = dir * h * (h * qsum<8, 5>(kv[q][c]));
             const double u =
-                ex * recip(ctl.atol + ctl.rtol * fmax(fabs(y[q][c]), fabs(yn[q][c])));
+                div_rn(ex, fma(ctl.rtol, fmax(fabs(y[q][c]), fabs(yn[q][c])), ctl.atol));
             ss = fma(u, u, ss);
           }
     }
     const double e = sqrt(reduce(ss) / ntot);
     if (live) {
       const bool keep = (e < 1.0) || at_dtmin;
-      const double factor = fmin(fmax(step_factor(e), keep ? 1.0 : 0.2), 10.0);
+      double factor = 0.9 * fifth_root(1.0 / e);
+      factor = fmin(fmax(factor, keep ? 1.0 : 0.2), 10.0);
       double dtn = h * factor;
       if (ctl.dtmax > 0.0 && dtn > ctl.dtmax) dtn = ctl.dtmax;
       if (ctl.dtmin > 0.0) {
@@ -576,7 +690,7 @@ void perturb_dopri5_kernel(
   }
 }
 
-template <int SK, int RAD, int G>
+template <int SK, int RAD, int G, bool WIDE>
 int launch_pd(const ssc_host_potential& hp, const ssc_sources& pert, const double* w0,
               const double* dw0, const double* t_start, int64_t n, int L, double t0, double t1,
               const double* ts, int nts, const Dp5Ctl& ctl, double* w_out, double* dw_out,
@@ -584,7 +698,7 @@ int launch_pd(const ssc_host_potential& hp, const ssc_sources& pert, const doubl
   const size_t lds = SourceLDS<SK>::bytes(pert);
   if (lds > 120 * 1024) return fail(SSC_E_LIMIT, "ssc_perturb_dopri5: source table exceeds LDS");
   if (lds > 60 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)perturb_dopri5_kernel<SK, RAD, G>,
+    hipError_t e = hipFuncSetAttribute((const void*)perturb_dopri5_kernel<SK, RAD, G, WIDE>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess)
       return fail(SSC_E_HIP, std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
@@ -592,7 +706,7 @@ int launch_pd(const ssc_host_potential& hp, const ssc_sources& pert, const doubl
   const int ppb = PD_BLOCK / L;
   const int64_t blocks = (n + ppb - 1) / ppb;
   if (blocks > (int64_t)INT_MAX) return fail(SSC_E_LIMIT, "ssc_perturb_dopri5: too many orbits");
-  hipLaunchKernelGGL((perturb_dopri5_kernel<SK, RAD, G>), dim3((unsigned)blocks), dim3(PD_BLOCK),
+  hipLaunchKernelGGL((perturb_dopri5_kernel<SK, RAD, G, WIDE>), dim3((unsigned)blocks), dim3(PD_BLOCK),
                      lds, st, hp, pert, w0, dw0, t_start, n, pert.n, L, t0, t1, ts, nts, ctl,
                      w_out, dw_out, ys, dys, stats);
   return check_launch("ssc_perturb_dopri5");
@@ -608,13 +722,16 @@ int dispatch_g(const ssc_host_potential& hp, const ssc_sources& s, const double*
   const int per = (nvec + G - 1) / G;
   int L = PD_MIN_L;
   while (L < per) L <<= 1;
+  if (G == 1 && L > 64)
+    return launch_pd<SK, RAD, 1, true>(hp, s, w0, dw0, t_start, n, L, t0, t1, ts, nts, ctl, w_out,
+                                       dw_out, ys, dys, stats, st);
   if (G == 1)
-    return launch_pd<SK, RAD, 1>(hp, s, w0, dw0, t_start, n, L, t0, t1, ts, nts, ctl, w_out,
+    return launch_pd<SK, RAD, 1, false>(hp, s, w0, dw0, t_start, n, L, t0, t1, ts, nts, ctl, w_out,
                                  dw_out, ys, dys, stats, st);
   if (G == 2)
-    return launch_pd<SK, RAD, 2>(hp, s, w0, dw0, t_start, n, L, t0, t1, ts, nts, ctl, w_out,
+    return launch_pd<SK, RAD, 2, true>(hp, s, w0, dw0, t_start, n, L, t0, t1, ts, nts, ctl, w_out,
                                  dw_out, ys, dys, stats, st);
-  return launch_pd<SK, RAD, 4>(hp, s, w0, dw0, t_start, n, L, t0, t1, ts, nts, ctl, w_out,
+  return launch_pd<SK, RAD, 4, true>(hp, s, w0, dw0, t_start, n, L, t0, t1, ts, nts, ctl, w_out,
                                dw_out, ys, dys, stats, st);
 }
 
