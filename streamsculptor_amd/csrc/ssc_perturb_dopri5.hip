@@ -123,13 +123,12 @@ __device__ __forceinline__ double stage_c() {
   return 0.0;
 }
 
-// err / (atol + rtol max(|y|, |yn|)) of a component with stored slopes.
+// err / (atol + rtol max(|y|, |yn|)), none where a tolerance is infinite, of a component with stored slopes.
 __device__ __forceinline__ double err_of(double y, const double (&k)[7], double yn, double h,
                                          const Dp5Ctl& ctl) {
   const double err =
       h * fma(E7, k[6], fma(E6, k[5], fma(E5, k[4], fma(E4, k[3], dot2(E1, k[0], E3, k[2])))));
-  const double u = div_rn(err, fma(ctl.rtol, fmax(fabs(y), fabs(yn)), ctl.atol));
-  return u;
+  return div_patched(err, fma(ctl.rtol, fmax(fabs(y), fabs(yn)), ctl.atol));
 }
 
 // Quartic through y (s = 0), yn (s = 1), slopes F0 = h f0 and F7 = h f7, and the midpoint
@@ -603,7 +602,7 @@ void perturb_dopri5_kernel(
             ss = fma(uv, uv, ss);
             const double ex = dir * h * (h * qsum<8, 5>(kv[q][c]));
             const double u =
-                div_rn(ex, fma(ctl.rtol, fmax(fabs(y[q][c]), fabs(yn[q][c])), ctl.atol));
+                div_patched(ex, fma(ctl.rtol, fmax(fabs(y[q][c]), fabs(yn[q][c])), ctl.atol));
             ss = fma(u, u, ss);
           }
     }
