@@ -254,7 +254,7 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
     side = _side_stream(dev)
     w = _lib.f64(prog_w0).reshape(1, 6)
     spray = _side_stream(dev, 1)
-    state, keep = None, []  # keep: read on another stream than its own
+    state, keep = None, []  # keep: read on the third stream, for which the current one waits
     try:
         for c in range(len(cuts) - 1):
             a, b = cuts[c], cuts[c + 1]
@@ -270,7 +270,10 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
                 table = release_pot._release_seeds(ys[:, 0, :], idx_all[a:b], gms_all[a:b],
                                                    seed_num, nseed, kval_arr, at=at)
                 new = table.view(-1, 6).index_select(0, pick_all[a * per_step:b * per_step])
-            keep.append((ys, new))
+            # read on the second stream, for which neither the third nor another caller's current
+            # stream waits: its memory is not handed out before those reads are done
+            new.record_stream(side)
+            keep.append(ys)
             side.wait_stream(spray)
             with torch.cuda.stream(side):
                 w_in = new if state is None else torch.cat([state, new], 0)
