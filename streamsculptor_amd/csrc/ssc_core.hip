@@ -99,7 +99,9 @@ __device__ __forceinline__ void eval_pair(const SrcGeo& s, double gm, double x, 
   if constexpr (HQ) {  // s.rs2 holds a: f = G m / (r (r + a)^2), k = -f (3 r + a) / (r^2 (r + a))
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
     const double ir = rsq(r2);
-    const double ia = recip(fma(r2, ir, s.rs2));
+    // at the centre, and where r^2 overflows, ir is NaN but the potential is not
+    const double r = r2 > 0.0 && r2 < __builtin_inf() ? r2 * ir : r2;
+    const double ia = div_patched(1.0, r + s.rs2);
     const double d1 = gm * ia * ia;
     f = d1 * ir;
     k = -(ir * ir) * fma(2.0 * d1, ia, f);
