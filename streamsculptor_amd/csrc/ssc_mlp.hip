@@ -551,9 +551,9 @@ namespace {
 using namespace mlp;
 
 struct Workspace {
-  float *Z1, *Z2, *Z3, *dZ3, *dZ2, *dZ1, *dY, *ytmp, *loss_part;
+  float *Z1, *Z2, *Z3, *dZ3, *dZ2, *dZ1, *dY, *loss_part;
   float *pW4, *pW3, *pW2, *pb4, *pb3, *pb2, *pl1;  // partials of the gradient sums
-  uint16_t *A1, *A2, *A3, *A1t, *A2t, *A3t, *dZb, *dZ3t, *dZ2t, *dYb, *dYt;
+  uint16_t *A1, *A2, *A3, *A1t, *A2t, *A3t, *dZ3b, *dZ2b, *dZ3t, *dZ2t, *dYb, *dYt;
   uint16_t *W2b, *W3b, *W4b, *W2t, *W3t;
   int64_t ldt;  // row pitch of the transposed arrays: the batch rounded up to 8
   int64_t bytes;
@@ -579,16 +579,21 @@ Workspace carve(void* base, int64_t nb) {
   auto b16 = [&](int64_t n) { return (uint16_t*)take(n * 2); };
   const int64_t nz = splitk_for(nb), nc = chunks_of(nb);
   w.ldt = (nb + 7) / 8 * 8;
-  w.Z1 = f32(nb * H); w.Z2 = f32(nb * H); w.Z3 = f32(nb * H);
-  w.dZ3 = f32(nb * H); w.dZ2 = f32(nb * H); w.dZ1 = w.dZ3;  // dZ3 is done with before dZ1
-  w.dY = f32(nb * OUT); w.ytmp = f32(nb * OUT);
+  // The backward pass takes no room of its own for a point: a layer's gradient replaces its
+  // pre-activations element by element, and its BF16 copies take arrays that the launches before
+  // have read for the last time (6.2 KB a point; 10.3 with arrays of their own).
+  w.Z1 = f32(nb * H); w.Z2 = f32(nb * H);
+  w.Z3 = f32(std::max(nb * H, nz * H * H));
+  w.dZ3 = w.Z3; w.dZ2 = w.Z2; w.dZ1 = w.Z1;
+  w.dY = f32(nb * OUT);
   w.loss_part = f32((nb + GT - 1) / GT);
-  w.pW4 = f32(nz * OUT * H); w.pW3 = f32(nz * H * H); w.pW2 = f32(nz * H * H);
+  w.pW4 = f32(nz * OUT * H); w.pW3 = f32(nz * H * H);
+  w.pW2 = w.Z3;  // formed by the third launch; dZ3 is read by the first two
   w.pb4 = f32(nc * OUT); w.pb3 = f32(nc * H); w.pb2 = f32(nc * H); w.pl1 = f32(nc * H * (IN + 1));
-  w.A1 = b16(nb * H); w.A2 = b16(nb * H); w.A3 = b16(nb * H);
+  w.A1 = b16(w.ldt * H); w.A2 = b16(nb * H); w.A3 = b16(nb * H);
   w.A1t = b16(w.ldt * H); w.A2t = b16(w.ldt * H); w.A3t = b16(w.ldt * H);
-  w.dZb = b16(2 * nb * H);  // two layers in turn: one is read while the next is written
-  w.dZ3t = b16(w.ldt * H); w.dZ2t = b16(w.ldt * H);
+  w.dZ3b = w.A3; w.dZ3t = w.A1;   // A3 and A1 are read by the forward pass only,
+  w.dZ2b = w.A2; w.dZ2t = w.A3t;  // A2 too, A3t by the first backward launch
   w.dYb = b16(nb * OUT); w.dYt = b16(w.ldt * OUT);
   w.W2b = b16(H * H); w.W3b = b16(H * H); w.W4b = b16(OUT * H);
   w.W2t = b16(H * H); w.W3t = b16(H * H);
@@ -687,25 +692,24 @@ void forward(const float* p, const float* x, int64_t nb, float* y, Workspace& w,
 void backward(const float* x, int64_t nb, float* g, Workspace& w, float* loss, hipStream_t st) {
   const int nz = (int)splitk_for(nb), n = (int)nb;
   const int nc = (int)chunks_of(nb);
-  uint16_t* dZb[2] = {w.dZb, w.dZb + nb * H};
   // each launch: the gradient of one layer's weights and biases, and the next layer down
   Product w4 = make_product({w.dYt, w.ldt, 1, OUT}, {w.A3t, w.ldt, 1, H}, n, nz, EPI_PART);
   w4.out = w.pW4;
   Product d3 = make_product({w.dYb, OUT, 1, n}, {w.W4b, 1, H, H}, OUT, 1, EPI_DACT);
-  d3.Z = w.Z3; d3.out = w.dZ3; d3.out16 = dZb[0]; d3.out16t = w.dZ3t; d3.ldt = w.ldt;
+  d3.Z = w.Z3; d3.out = w.dZ3; d3.out16 = w.dZ3b; d3.out16t = w.dZ3t; d3.ldt = w.ldt;
   const ColSum b4{w.dY, w.pb4, nb, OUT};
   launch_backward(b4, d3, w4, st);
 
   Product w3 = make_product({w.dZ3t, w.ldt, 1, H}, {w.A2t, w.ldt, 1, H}, n, nz, EPI_PART);
   w3.out = w.pW3;
-  Product d2 = make_product({dZb[0], H, 1, n}, {w.W3t, H, 1, H}, H, 1, EPI_DACT);
-  d2.Z = w.Z2; d2.out = w.dZ2; d2.out16 = dZb[1]; d2.out16t = w.dZ2t; d2.ldt = w.ldt;
+  Product d2 = make_product({w.dZ3b, H, 1, n}, {w.W3t, H, 1, H}, H, 1, EPI_DACT);
+  d2.Z = w.Z2; d2.out = w.dZ2; d2.out16 = w.dZ2b; d2.out16t = w.dZ2t; d2.ldt = w.ldt;
   const ColSum b3{w.dZ3, w.pb3, nb, H};
   launch_backward(b3, d2, w3, st);
 
   Product w2 = make_product({w.dZ2t, w.ldt, 1, H}, {w.A1t, w.ldt, 1, H}, n, nz, EPI_PART);
   w2.out = w.pW2;
-  Product d1 = make_product({dZb[1], H, 1, n}, {w.W2t, H, 1, H}, H, 1, EPI_DACT);
+  Product d1 = make_product({w.dZ2b, H, 1, n}, {w.W2t, H, 1, H}, H, 1, EPI_DACT);
   d1.Z = w.Z1; d1.out = w.dZ1;
   const ColSum b2{w.dZ2, w.pb2, nb, H};
   launch_backward(b2, d1, w2, st);
@@ -801,8 +805,9 @@ int ssc_mlp_backward(const float* params, const float* x, const float* dy, int64
   if (workspace_bytes < ws_bytes(batch)) return fail(SSC_E_ARG, "ssc_mlp_backward: workspace too small");
   hipStream_t st = (hipStream_t)stream;
   Workspace w = carve(workspace, batch);
-  // recompute the forward into the workspace; dy takes the place of the loss gradient
-  forward(params, x, batch, w.ytmp, w, true, nullptr, st);
+  // recompute the forward into the workspace; dy takes the place of the loss gradient (and of the
+  // outputs, which are not asked for)
+  forward(params, x, batch, w.dY, w, true, nullptr, st);
   hipLaunchKernelGGL(seed_kernel, dim3(nblk(batch * OUT)), dim3(256), 0, st, dy, batch, w.dY, w.dYb,
                      w.dYt, w.ldt);
   backward(x, batch, grads, w, nullptr, st);
