@@ -254,7 +254,9 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
     side = _side_stream(dev)
     w = _lib.f64(prog_w0).reshape(1, 6)
     spray = _side_stream(dev, 1)
-    state, keep = None, []  # keep: read on the third stream, for which the current one waits
+    # keep: memory of the current stream that the other two use; it waits for both, as neither
+    # does for the other or for another caller's current stream
+    state, keep = None, []
     try:
         for c in range(len(cuts) - 1):
             a, b = cuts[c], cuts[c + 1]
@@ -263,17 +265,16 @@ def spray_stream(prog_pot, release_pot, ts, prog_w0, Msat, seed_num, per_step, d
             save, start = views[2 * c:2 * c + 2]
             pn = (g1 if b < T else int(kidx[T - 1])) - g0
             w, ys = prog_pot._leapfrog(w, t0 + g0 * dt, dt, pn, save_idx=save)
+            new = torch.empty((b - a) * per_step, 6, dtype=torch.float64, device=dev)
+            keep.append((ys, new))
             spray.wait_stream(main)
             with torch.cuda.stream(spray):
                 at = (sd, None if t_all is None else t_all[a:b],
                       None if step_all is None else step_all[a:b], src)
                 table = release_pot._release_seeds(ys[:, 0, :], idx_all[a:b], gms_all[a:b],
                                                    seed_num, nseed, kval_arr, at=at)
-                new = table.view(-1, 6).index_select(0, pick_all[a * per_step:b * per_step])
-            # read on the second stream, for which neither the third nor another caller's current
-            # stream waits: its memory is not handed out before those reads are done
-            new.record_stream(side)
-            keep.append(ys)
+                torch.index_select(table.view(-1, 6), 0, pick_all[a * per_step:b * per_step],
+                                   out=new)
             side.wait_stream(spray)
             with torch.cuda.stream(side):
                 w_in = new if state is None else torch.cat([state, new], 0)
