@@ -235,11 +235,13 @@ int ssc_release_seeds(const ssc_host_potential* host, const ssc_sources* src, co
  *   w_out[n][6], dw_out[n][m][D] at grid index nsteps (must not alias w0, dw0 when a
  *                   workspace is given)
  *   workspace       NULL, or device memory of workspace_bytes (ssc_perturb_workspace_bytes
- *                   gives a size of at most 4 GiB): the base orbits are then advanced once per
- *                   particle through segments of grid rows, recording position and host Hessian
- *                   per row for the responses; without it every lane that holds responses of a
- *                   particle recomputes them (about twice the arithmetic; the source forces
- *                   are summed in another order, so results agree to the last bits). */
+ *                   gives the size worth having: 72 bytes a particle and row for a quarter of
+ *                   the grid, at least 128 rows, at most 4 GiB; one row is the least): the base
+ *                   orbits are then advanced once per particle through segments of grid rows,
+ *                   recording position and host Hessian per row for the responses; without it
+ *                   every lane that holds responses of a particle recomputes them (about twice
+ *                   the arithmetic; the source forces are summed in another order, so results
+ *                   agree to the last bits). */
 int64_t ssc_perturb_workspace_bytes(int64_t n, int32_t nsteps);
 int ssc_perturb_leapfrog(const ssc_host_potential* host, const ssc_sources* pert,
                          const double* w0, const double* dw0, const int32_t* start_step,

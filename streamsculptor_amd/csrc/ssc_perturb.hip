@@ -18,7 +18,8 @@
 // through a segment and records, at every row a particle is kicked at, its position and the host
 // Hessian; response_rows then advances the responses through the segment from those records.
 // One launch carries the base rows of segment s + 1 beside the responses of segment s: the first
-// waits for memory (72 B a particle and row), the second for FP64 issue.  Without a workspace
+// waits for memory (72 B a particle and row), the second for FP64 issue (a grid of fewer than two
+// segments of 64 rows has one, its responses after its base rows).  Without a workspace
 // perturb_kernel has each of the L lanes recompute the base orbit and the host Hessian (2.2x the
 // arithmetic of the split form, measured by counters).
 // Velocities are carried at half steps so that forces are consumed as soon as they are formed.
@@ -473,11 +474,20 @@ static bool split_few(int64_t n, int m, bool radius) {
   return radius || n * L < (int64_t)2 * 1024 * 64;
 }
 
-// Rows per segment that fit in workspace_bytes (0 when not even one does).
+// Rows of records to keep where there is room: two segments of an eighth of the grid each, so that
+// all but an eighth of the base rows are formed beside responses, or all rows of a grid of fewer
+// than two segments of 64.  Segments of an eighth and one of all rows (ms): 8,000 particles x 64
+// sources, 4,000 steps 3.94 and 5.91 (0.6 and 2.3 GB), 1,000 x 7, 500 steps 0.51 and 0.68, 40,000 x
+// 64, 1,000 steps 2.42 and 2.55; with fewer than 64 rows a segment the two parts' blocks no
+// longer last each other out: 500,000 x 4, 100 steps 1.24 (13 rows) and 0.91.
+static int64_t perturb_rows_wanted(int nsteps) {
+  const int64_t r = std::max<int64_t>(64, ((int64_t)nsteps + 8) / 8);
+  return 2 * r > nsteps ? (int64_t)nsteps + 1 : 2 * r;
+}
+
+// Rows of records that fit in workspace_bytes (0 when not even one does), no more than wanted.
 static int64_t perturb_segment_rows(int64_t n, int nsteps, int64_t workspace_bytes) {
-  const int64_t per_row = n * PR_REC * 8;
-  const int64_t e = per_row > 0 ? workspace_bytes / per_row : 0;
-  return e < (int64_t)nsteps + 1 ? e : (int64_t)nsteps + 1;
+  return std::min(workspace_bytes / (n * PR_REC * 8), perturb_rows_wanted(nsteps));
 }
 
 // Segments take turns in the two halves of a workspace that holds at least two rows but not all.
@@ -564,10 +574,10 @@ using namespace ssc;
 extern "C" int64_t ssc_perturb_workspace_bytes(int64_t n, int32_t nsteps) {
   if (n <= 0 || nsteps < 0) return 0;
   const int64_t per_row = n * PR_REC * 8;
-  int64_t e = ((int64_t)1 << 32) / per_row;  // two segments of rows of at most 2 GiB each
-  if (e < 1) e = 1;
-  if (e > (int64_t)nsteps + 1) e = (int64_t)nsteps + 1;
-  return e * per_row;
+  // two segments of at most 2 GiB each (1 GiB each: 200,000 particles x 16 sources, 2,000 steps
+  // 9.3 ms for 8.7, a million x 8, 500 steps 13.8 for 10.9)
+  const int64_t e = std::min(((int64_t)1 << 32) / per_row, perturb_rows_wanted(nsteps));
+  return (e < 1 ? 1 : e) * per_row;
 }
 
 extern "C" int ssc_perturb_leapfrog(const ssc_host_potential* host, const ssc_sources* pert,

@@ -127,7 +127,8 @@ def perturb_leapfrog(base, src, w0, dw0, start, t0, dt, nsteps, with_radius, spl
     """Run ssc_perturb_leapfrog: base rows w0 (n, 6), responses dw0 (n, m, 6|12) or None.
     split: advance the base orbits once per particle through segments of rows kept in a
     workspace (otherwise every lane of a particle recomputes them); segment_rows: rows of
-    records in the workspace (default: the library's choice, at most 4 GiB)."""
+    records in the workspace (default: the library's choice, a quarter of the grid and at least
+    128 rows, at most 4 GiB)."""
     h = base._host_only()
     w0 = _lib.f64(w0).reshape(-1, 6).contiguous()
     n = w0.shape[0]
