@@ -709,11 +709,15 @@ static int set_lds(const void* fn, size_t lds) {
 // Launch shape: one wave per orbit while every orbit has a SIMD of its own (512 clumps: 1,000
 // orbits 1.81 us a step against 2.87 with 16 lanes an orbit, 2,000 orbits 4.39 against 2.96; one
 // orbit in 20 tracked subhalos saved at every step 0.85 against 1.12, in 4 clumps 0.74 unsaved
-// against 0.70: from 8 sources on); two particles per lane for batches that fill the chip several times
-// over, unless the pairing costs a round of waves (512 clumps: 1e6 orbits 326 us against 331,
-// 4e5 169 against 153); group_lanes otherwise.  Without sources: for up to 65536 orbits in a
-// host of no known signature, host components over waves; one particle per lane otherwise (with
-// straight-line host code for the known hosts, which is faster still).
+// against 0.70: from 8 sources on), and up to two to a SIMD for orbits that start all along the
+// grid among many sources, half of whose waves wait for nobody's earlier start (1,300 orbits, 100
+// rows: 256 clumps 0.113 ms against 0.166 with 16 lanes an orbit, 512 clumps 0.136 against 0.242;
+// 2,500 among 512 0.195 against 0.243, but among 1,024 0.451 against 0.393); two particles per
+// lane for batches that fill the chip several times over, unless the pairing costs a round of
+// waves (512 clumps: 1e6 orbits 326 us against 331, 4e5 169 against 153); group_lanes otherwise.
+// Without sources: for up to 65536 orbits in a host of no known signature, host components over
+// waves; one particle per lane otherwise (with straight-line host code for the known hosts, which
+// is faster still).
 template <int SK, int HS>
 static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src, const double* w0,
                            const int32_t* start, int64_t n, double t0, double dt, int nsteps,
@@ -721,7 +725,8 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                            hipStream_t st) {
   const size_t lds = SourceLDS<SK>::bytes(src);
   const bool dense = nsave > nsteps / 2;  // see SaveRows
-  if (SK != SSC_SRC_NONE && src.n >= 8 && n <= 1024) {
+  const int64_t waves = !ragged || src.n < 128 ? 1024 : (src.n >= 256 && src.n <= 512 ? 2560 : 2048);
+  if (SK != SSC_SRC_NONE && src.n >= 8 && n <= waves) {
     auto kernel = dense ? leapfrog_wave_kernel<SK, HS, true> : leapfrog_wave_kernel<SK, HS, false>;
     int rc = set_lds((const void*)kernel, lds);
     if (rc) return rc;
