@@ -91,7 +91,7 @@ __device__ __forceinline__ void adj_apply(const ssc_host_potential& hp, const So
       }
     };
     int j = rl;
-    for (; j + 3 * G < lds.n; j += 4 * G) terms(std::integral_constant<int, 4>{}, j);
+    for (; j - rl + 4 * G <= lds.n; j += 4 * G) terms(std::integral_constant<int, 4>{}, j);
     for (; j < lds.n; j += G) terms(std::integral_constant<int, 1>{}, j);
 #pragma unroll
     for (int c = 0; c < 3; ++c) hw[c] += group_sum<G>(sw[c]);

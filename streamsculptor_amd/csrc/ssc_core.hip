@@ -508,7 +508,7 @@ __device__ __forceinline__ void leapfrog_group(
 }
 
 // The first n_whole orbits (whole rounds of waves) take one lane each, the rest G lanes.
-template <int SK, int G, int HS>
+template <int SK, int G, int HS, bool WHOLE>
 __global__ __launch_bounds__(LF_BLOCK) void leapfrog_group_kernel(
     ssc_host_potential hp, ssc_sources src, const double* __restrict__ w0,
     const int32_t* __restrict__ start, int64_t n_whole, int64_t n, double t0, double dt, int nsteps,
@@ -517,7 +517,7 @@ __global__ __launch_bounds__(LF_BLOCK) void leapfrog_group_kernel(
   extern __shared__ __align__(16) char lds_raw[];
   __shared__ int kmin_sh;
   const int64_t first = (int64_t)blockIdx.x * LF_BLOCK;
-  if (first < n_whole)
+  if (WHOLE && first < n_whole)
     leapfrog_group<SK, 1, HS>(hp, src, w0, start, first + threadIdx.x, n, t0, dt, nsteps, w_out,
                               save_idx, nsave, ys, lds_raw, kmin_sh);
   else
@@ -706,18 +706,28 @@ static int set_lds(const void* fn, size_t lds) {
   return SSC_OK;
 }
 
-// Launch shape: one wave per orbit while every orbit has a SIMD of its own (512 clumps: 1,000
-// orbits 1.81 us a step against 2.87 with 16 lanes an orbit, 2,000 orbits 4.39 against 2.96; one
-// orbit in 20 tracked subhalos saved at every step 0.85 against 1.12, in 4 clumps 0.74 unsaved
-// against 0.70: from 8 sources on), and up to two to a SIMD for orbits that start all along the
-// grid among many sources, half of whose waves wait for nobody's earlier start (1,300 orbits, 100
-// rows: 256 clumps 0.113 ms against 0.166 with 16 lanes an orbit, 512 clumps 0.136 against 0.242;
-// 2,500 among 512 0.195 against 0.243, but among 1,024 0.451 against 0.393); two particles per
-// lane for batches that fill the chip several times over, unless the pairing costs a round of
-// waves (512 clumps: 1e6 orbits 326 us against 331, 4e5 169 against 153); group_lanes otherwise.
-// Without sources: for up to 65536 orbits in a host of no known signature, host components over
-// waves; one particle per lane otherwise (with straight-line host code for the known hosts, which
-// is faster still).
+// Most orbits that take a wave each.  Every orbit has a SIMD of its own (512 clumps: 1,000 orbits
+// 1.81 us a step against 2.87 with 16 lanes an orbit, 2,000 orbits 4.39 against 2.96; one orbit in 20
+// tracked subhalos saved at every step 0.85 against 1.12, in 4 clumps 0.74 unsaved against 0.70: from
+// 8 sources on).  Up to two or so to a SIMD for orbits that start all along the grid among many
+// sources, half of whose waves wait for nobody's earlier start (1,300 orbits, 100 rows: 256 clumps
+// 0.113 ms against 0.166 with 16 lanes an orbit, 512 clumps 0.136 against 0.242; 2,500 among 512
+// 0.195 against 0.243, but among 1,024 0.451 against 0.393; 1,300 among 64 0.105 against 0.110).  Twice
+// as many with straight-line sources, whose chains leave a SIMD idle (60 rows: 1,500 orbits, 200
+// Hernquist subhalos 0.134 ms against 0.204, ragged 3,000 0.137 against 0.197).
+static int64_t wave_orbits(int nsrc, bool ragged, bool line) {
+  if (line) return (nsrc < 64 ? 1024 : 2048) * (ragged ? 2 : 1);
+  if (!ragged || nsrc < 64) return 1024;
+  return nsrc >= 256 && nsrc <= 512 ? 2560 : std::min(2048, 768 + 10 * nsrc);
+}
+
+// Launch shape: a wave per orbit (see wave_orbits); two particles per lane for batches that fill
+// the chip several times over, unless the pairing costs a round of waves (512 clumps: 1e6 orbits
+// 326 us against 331, 4e5 169 against 153), which pays all the same where two particles share the
+// place of a straight-line source (200 Hernquist subhalos, 8e5 orbits, 60 rows 10.5 ms against
+// 11.6); group_lanes otherwise.  Without sources: for up to
+// 65536 orbits in a host of no known signature, host components over waves; one particle per lane
+// otherwise (with straight-line host code for the known hosts, which is faster still).
 template <int SK, int HS>
 static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src, const double* w0,
                            const int32_t* start, int64_t n, double t0, double dt, int nsteps,
@@ -725,7 +735,8 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
                            hipStream_t st) {
   const size_t lds = SourceLDS<SK>::bytes(src);
   const bool dense = nsave > nsteps / 2;  // see SaveRows
-  const int64_t waves = !ragged || src.n < 128 ? 1024 : (src.n >= 256 && src.n <= 512 ? 2560 : 2048);
+  constexpr bool LINE = SK == SSC_SRC_LINE || SK == SSC_SRC_LINE_HERNQUIST;
+  const int64_t waves = wave_orbits(src.n, ragged, LINE);
   if (SK != SSC_SRC_NONE && src.n >= 8 && n <= waves) {
     auto kernel = dense ? leapfrog_wave_kernel<SK, HS, true> : leapfrog_wave_kernel<SK, HS, false>;
     int rc = set_lds((const void*)kernel, lds);
@@ -735,7 +746,7 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
     return check_launch("ssc_leapfrog");
   }
   if (SK != SSC_SRC_NONE && src.n >= 16 && n >= 393216 &&
-      2 * ((n + 131071) / 131072) <= (n + 65535) / 65536) {
+      (LINE || 2 * ((n + 131071) / 131072) <= (n + 65535) / 65536)) {
     int rc = set_lds((const void*)leapfrog_kernel<SK, 2, HS, false>, lds);
     if (rc) return rc;
     const int64_t blocks = (n + 2 * LF_BLOCK - 1) / (2 * LF_BLOCK);
@@ -751,15 +762,18 @@ static int launch_leapfrog(const ssc_host_potential& hp, const ssc_sources& src,
     return check_launch("ssc_leapfrog");
   }
   int64_t n_whole = 0;
-  const int g = SK == SSC_SRC_NONE ? 1 : group_lanes(n, src.n, ragged, &n_whole);
+  const int g = SK == SSC_SRC_NONE ? 1
+                : LINE             ? group_lanes_line(n, src.n, ragged, &n_whole)
+                                   : group_lanes(n, src.n, ragged, &n_whole);
 #define SSC_GROUP(GV)                                                                              \
   if (g == GV) {                                                                                   \
-    int rc = set_lds((const void*)leapfrog_group_kernel<SK, GV, HS>, lds);                         \
+    auto kernel = n_whole ? leapfrog_group_kernel<SK, GV, HS, true>                                \
+                          : leapfrog_group_kernel<SK, GV, HS, false>;                              \
+    int rc = set_lds((const void*)kernel, lds);                                                    \
     if (rc) return rc;                                                                             \
     const int64_t blocks = n_whole / LF_BLOCK + (n - n_whole + LF_BLOCK / GV - 1) / (LF_BLOCK / GV); \
-    hipLaunchKernelGGL((leapfrog_group_kernel<SK, GV, HS>), dim3((unsigned)blocks),                \
-                       dim3(LF_BLOCK), lds, st, hp, src, w0, start, n_whole, n, t0, dt, nsteps,    \
-                       w_out, save_idx, nsave, ys);                                                \
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(LF_BLOCK), lds, st, hp, src, w0, start, \
+                       n_whole, n, t0, dt, nsteps, w_out, save_idx, nsave, ys);                    \
     return check_launch("ssc_leapfrog");                                                           \
   }
   SSC_GROUP(2)

@@ -145,7 +145,7 @@ inline int group_lanes(int64_t n, int nsrc, bool ragged, int64_t* n_whole = null
     const double waves = ragged ? std::max(1.0, n * g / 131072.0)
                                 : (double)((n * g + 65535) / 65536);
     const double cost = (4.0 * waves + 1.0) * wave(lg);
-    if (lg == 0 || cost <= least) { least = cost; best = (int)g; }
+    if (lg == 0 || cost < least) { least = cost; best = (int)g; }
   }
   if (!n_whole || ragged) return best;
   *n_whole = 0;
@@ -155,6 +155,36 @@ inline int group_lanes(int64_t n, int nsrc, bool ragged, int64_t* n_whole = null
   for (int lg = 1; lg <= 4; ++lg) {
     const int64_t g = 1 << lg, waves = (rest * g + 65535) / 65536;
     const double cost = (4.0 * rounds + 1.0) * wave(0) + 4.0 * waves * wave(lg);
+    if (cost < least) { least = cost; best = (int)g; *n_whole = rounds * 65536; }
+  }
+  return best;
+}
+
+// The same for straight-line sources, each of which is first looked up by its window and placed at
+// the time: a source takes about 2.5 times as long and its chain leaves a SIMD idle, so that time
+// does not grow up to about 2.5 waves per SIMD (2 of the halved ones of ragged starts); a wave by
+// itself takes as long.  60 steps (ms), three waves per SIMD wanted / the rule above / this one: 30
+// Plummer subhalos, 20,000 orbits 0.157 / 0.187 / 0.149, 40,000 0.202 / 0.304 / 0.202, ragged
+// starts of 130,000 0.210 / 0.298 / 0.20; 200 Hernquist subhalos, 12,000 orbits 0.337 / 0.646 /
+// 0.33, ragged 30,000 0.369 / 0.629 / 0.38.
+inline int group_lanes_line(int64_t n, int nsrc, bool ragged, int64_t* n_whole) {
+  auto wave = [&](int lg) { return (nsrc + (1 << lg) - 1) / (1 << lg) + 1.6 + 1.2 * lg; };
+  *n_whole = 0;
+  if (nsrc < 16 && n >= 32768) return 1;  // a few sources: the exchanges outweigh the shorter sums
+  int best = 1;
+  double least = 0.0;
+  for (int lg = 0; lg <= 4; ++lg) {
+    const int64_t g = 1 << lg;
+    const double cost = wave(lg) * (ragged ? std::max(2.0, n * g / 131072.0)
+                                           : std::max(2.5, (double)((n * g + 65535) / 65536)));
+    if (lg == 0 || cost < least) { least = cost; best = (int)g; }
+  }
+  const int64_t rounds = n / 65536, rest = n - rounds * 65536;
+  if (ragged || rounds == 0 || rest == 0) return best;
+  least *= 0.95;
+  for (int lg = 1; lg <= 4; ++lg) {
+    const int64_t g = 1 << lg, waves = (rest * g + 65535) / 65536;
+    const double cost = std::max(2.5 * wave(0), rounds * wave(0) + waves * wave(lg));
     if (cost < least) { least = cost; best = (int)g; *n_whole = rounds * 65536; }
   }
   return best;

@@ -9,6 +9,7 @@
 #pragma once
 
 #include <climits>
+#include <type_traits>
 
 #include "ssc_device.h"
 
@@ -75,26 +76,33 @@ struct SourceLDS<SSC_SRC_STATIC> {
   template <int P>
   __device__ void add_grad(int, double, const double* x, const double* y, const double* z,
                            double* gx, double* gy, double* gz, int j0, int js) const {
-    auto term = [&](const SrcGeo& g, const SrcK& c) {
+    auto terms = [&](auto count, int j) {
+      constexpr int U = decltype(count)::value;
+      SrcGeo g[U];
+      SrcK c[U];
 #pragma unroll
-      for (int p = 0; p < P; ++p)
-        plummer_grad_k(x[p] - g.x, y[p] - g.y, z[p] - g.z, g.rs2, c.c1, c.c2, gx[p], gy[p], gz[p]);
-    };
-    // four sources at a time, in order (see TrackLDS); two particles a lane interleave by
-    // themselves (1e6 particles of a stream, 512 clumps: 140.9 ms so, 137.6 one at a time)
-    int j = j0;
-    for (; P == 1 && j + 3 * js < n; j += 4 * js) {
-      SrcGeo g[4];
-      SrcK c[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < U; ++u) {
         g[u] = geo[j + u * js];
         c[u] = kc[j + u * js];
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) term(g[u], c[u]);
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+          plummer_grad_k(x[p] - g[u].x, y[p] - g[u].y, z[p] - g[u].z, g[u].rs2, c[u].c1, c[u].c2,
+                         gx[p], gy[p], gz[p]);
+    };
+    // four sources at a time, in order (see TrackLDS); two particles a lane interleave by
+    // themselves (1e6 particles of a stream, 512 clumps: 140.9 ms so, 137.6 one at a time)
+    int j = j0;
+    if (P == 1) {
+      for (; j - j0 + 4 * js <= n; j += 4 * js) terms(std::integral_constant<int, 4>{}, j);
+      if (j - j0 + 2 * js <= n) {
+        terms(std::integral_constant<int, 2>{}, j);
+        j += 2 * js;
+      }
     }
-    for (; j < n; j += js) term(geo[j], kc[j]);
+    for (; j < n; j += js) terms(std::integral_constant<int, 1>{}, j);
   }
   __device__ bool get(int, double, int j, double& sx, double& sy, double& sz, double& gm,
                       double& q) const {
@@ -186,31 +194,38 @@ struct TrackLDS {
   __device__ void add_grad(int k, double, const double* x, const double* y, const double* z,
                            double* gx, double* gy, double* gz, int j0, int js) const {
     const SrcGeo* row = rec + (k - kb) * n;
-    auto term = [&](const SrcGeo& g, const SrcK& c, int j) {
+    auto terms = [&](auto count, int j) {
+      constexpr int U = decltype(count)::value;
+      SrcGeo g[U];
+      SrcK c[U];
 #pragma unroll
-      for (int p = 0; p < P; ++p) {
-        if (HQ)
-          hernquist_grad(x[p] - g.x, y[p] - g.y, z[p] - g.z, gmv[j], g.rs2, gx[p], gy[p], gz[p]);
-        else
-          plummer_grad_k(x[p] - g.x, y[p] - g.y, z[p] - g.z, g.rs2, c.c1, c.c2, gx[p], gy[p],
-                         gz[p]);
-      }
-    };
-    // four sources at a time, in order: their reads are in flight together and their chains
-    // interleave (one source per iteration waited for its LDS reads and its 15-instruction chain)
-    int j = j0;
-    for (; j + 3 * js < n; j += 4 * js) {
-      SrcGeo g[4];
-      SrcK c[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < U; ++u) {
         g[u] = row[j + u * js];
         c[u] = kc[j + u * js];
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) term(g[u], c[u], j + u * js);
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          if (HQ)
+            hernquist_grad(x[p] - g[u].x, y[p] - g[u].y, z[p] - g[u].z, gmv[j + u * js], g[u].rs2,
+                           gx[p], gy[p], gz[p]);
+          else
+            plummer_grad_k(x[p] - g[u].x, y[p] - g[u].y, z[p] - g[u].z, g[u].rs2, c[u].c1, c[u].c2,
+                           gx[p], gy[p], gz[p]);
+        }
+    };
+    // four sources at a time, then two, in order: their reads are in flight together and their chains
+    // interleave (one source per iteration waited for its LDS reads and its 15-instruction chain).
+    // All lanes of an orbit (j0 = 0 ... js - 1) take the same blocks: with blocks for the lanes that
+    // have one more source, a wave per orbit went through both loops (200 tracked subhalos 10 %).
+    int j = j0;
+    for (; j - j0 + 4 * js <= n; j += 4 * js) terms(std::integral_constant<int, 4>{}, j);
+    if (j - j0 + 2 * js <= n) {
+      terms(std::integral_constant<int, 2>{}, j);
+      j += 2 * js;
     }
-    for (; j < n; j += js) term(row[j], kc[j], j);
+    for (; j < n; j += js) terms(std::integral_constant<int, 1>{}, j);
   }
   __device__ bool get(int k, double, int j, double& sx, double& sy, double& sz, double& gm,
                       double& q) const {
