@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "ssc_device.h"
 
@@ -113,15 +114,29 @@ __device__ void release_sources(const ssc_sources& src, const double* __restrict
   const bool outside = (src.kind == SSC_SRC_TRACK || src.kind == SSC_SRC_TRACK_HERNQUIST) &&
                        (step < 0 || step >= src.n_track);
   double phi = 0.0, g[3] = {}, H[9] = {};
-  for (int j = outside ? src.n : lane; j < src.n; j += LANES) {
-    double sx, sy, sz;
-    if (!source_position(src, j, step, t, sx, sy, sz)) continue;
-    const double rs = src.rs[j];
-    if (src.kind == SSC_SRC_LINE_HERNQUIST || src.kind == SSC_SRC_TRACK_HERNQUIST)
-      hernquist_full(w[0] - sx, w[1] - sy, w[2] - sz, src.gm[j], rs, phi, g, H);
-    else
-      plummer_full(w[0] - sx, w[1] - sy, w[2] - sz, src.gm[j], rs * rs, phi, g, H);
-  }
+  const double x = w[0], y = w[1], z = w[2];
+  auto add = [&](auto kind) {  // a loop for each kind: no branch on it at every source
+    constexpr int K = decltype(kind)::value;
+    ssc_sources s = src;
+    s.kind = K;
+#pragma unroll 4
+    for (int j = lane; j < s.n; j += LANES) {
+      double sx, sy, sz;
+      if (!source_position(s, j, step, t, sx, sy, sz)) continue;
+      const double rs = s.rs[j];
+      if (K == SSC_SRC_LINE_HERNQUIST || K == SSC_SRC_TRACK_HERNQUIST)
+        hernquist_full(x - sx, y - sy, z - sz, s.gm[j], rs, phi, g, H);
+      else
+        plummer_full(x - sx, y - sy, z - sz, s.gm[j], rs * rs, phi, g, H);
+    }
+  };
+  if (!outside) switch (src.kind) {
+      case SSC_SRC_STATIC: add(std::integral_constant<int, SSC_SRC_STATIC>{}); break;
+      case SSC_SRC_TRACK: add(std::integral_constant<int, SSC_SRC_TRACK>{}); break;
+      case SSC_SRC_LINE: add(std::integral_constant<int, SSC_SRC_LINE>{}); break;
+      case SSC_SRC_LINE_HERNQUIST: add(std::integral_constant<int, SSC_SRC_LINE_HERNQUIST>{}); break;
+      default: add(std::integral_constant<int, SSC_SRC_TRACK_HERNQUIST>{}); break;
+    }
   constexpr int at[6] = {0, 1, 2, 4, 5, 8};
 #pragma unroll
   for (int k = 0; k < 6; ++k) S[k] = outside ? __builtin_nan("") : group_sum<LANES>(H[at[k]]);
@@ -170,30 +185,39 @@ __device__ void release_frame(const ssc_host_potential& hp, const double* __rest
   }
 }
 
-// One of the two released rows' four vectors of frame f, release index ridx and seed, by four
-// consecutive lanes: lane q of them draws Gaussian multiplier q (key PRNGKey(ridx * r_q), main.py:
-// 220-228,263-266) and gets the others' by shuffles, then forms the close position, far position,
-// close velocity or far velocity (trailing arm = far, leading arm = close; main.py:269-278).
+// The released rows' four vectors of frame f and its Gaussian multipliers, component a: close
+// position, far position, close velocity, far velocity (trailing arm = far, leading arm = close;
+// main.py:263-278).  The sums are the FMAs written here, whatever is inlined around them.
+struct ReleaseScale {
+  double kr, kvphi, kz, kvz;
+  __device__ ReleaseScale(const KVals& kv, const double* z)
+      : kr(fma(z[0], kv.k[4], kv.k[0])), kvphi(kr * fma(z[1], kv.k[5], kv.k[1])),
+        kz(fma(z[2], kv.k[6], kv.k[2])), kvz(fma(z[3], kv.k[7], kv.k[3])) {}
+  __device__ void vectors(const ReleaseFrame& f, int a, double* o) const {
+    const double pr = kr * f.rh[a], pz = f.zh[a] * kz;
+    const double vp = kvphi * f.relv, vz = kvz * f.relv;
+    o[0] = fma(-pz, f.rt, fma(-pr, f.rt, f.x[a]));
+    o[1] = fma(pz, f.rt, fma(pr, f.rt, f.x[a]));
+    o[2] = fma(-vz, f.zh[a], fma(-vp, f.ph[a], f.v[a]));
+    o[3] = fma(vz, f.zh[a], fma(vp, f.ph[a], f.v[a]));
+  }
+};
+
+// One of the four vectors of frame f, release index ridx and seed, by four consecutive lanes: lane q
+// of them draws Gaussian multiplier q (key PRNGKey(ridx * r_q), main.py:220-228) and gets the
+// others' by shuffles, then forms vector q.
 __device__ void release_vector(const ReleaseFrame& f, int64_t ridx, int64_t seed, const KVals& kv,
                                int q, double* o) {
-  // products and sums in the roundings written here, whatever is inlined around them
-#pragma clang fp contract(off)
   const double z = prng_normal(ridx * randint1000(seed, q));
   double zr[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) zr[k] = __shfl(z, k, 4);
-  const double kr = fma(zr[0], kv.k[4], kv.k[0]);
-  const double kvphi = kr * fma(zr[1], kv.k[5], kv.k[1]);
-  const double kz = fma(zr[2], kv.k[6], kv.k[2]);
-  const double kvz = fma(zr[3], kv.k[7], kv.k[3]);
+  const ReleaseScale c(kv, zr);
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    const double pr = kr * f.rh[a], pz = f.zh[a] * kz;
-    const double ptr = fma(pz, f.rt, fma(pr, f.rt, f.x[a]));
-    const double vtr = f.v[a] + kvphi * f.relv * f.ph[a] + kvz * f.relv * f.zh[a];
-    const double pld = fma(-pz, f.rt, fma(-pr, f.rt, f.x[a]));
-    const double vld = f.v[a] - kvphi * f.relv * f.ph[a] - kvz * f.relv * f.zh[a];
-    o[a] = q == 0 ? pld : (q == 1 ? ptr : (q == 2 ? vld : vtr));
+    double v[4];
+    c.vectors(f, a, v);
+    o[a] = q == 0 ? v[0] : (q == 1 ? v[1] : (q == 2 ? v[2] : v[3]));
   }
 }
 
@@ -252,6 +276,37 @@ __global__ __launch_bounds__(256) void release_kernel(
   }
 }
 
+// One seed of many releases: a lane each, which fills the chip, so that what the lanes of
+// release_kernel do over again or exchange is only more work (1e6 releases: host 0.18 ms against
+// 0.41, 64 clumps 0.54 against 1.59, 512 clumps 1.42 against 2.54; 50,000: 39 us against 48, 93
+// against 130).  The rows are release_kernel's in the host alone; sources are added up in order.
+constexpr int RELEASE_MANY = 32768;
+template <bool SRC>
+__global__ __launch_bounds__(256) void release_many_kernel(
+    ssc_host_potential hp, ssc_sources src, const double* __restrict__ prog_w,
+    const int32_t* __restrict__ rel_idx, const double* __restrict__ t_rel,
+    const int32_t* __restrict__ step_rel, const double* __restrict__ g_msat, int nrel,
+    int64_t seed, KVals kv, ReleaseOut out) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= nrel) return;
+  double S[6];
+  if (SRC) release_sources<1>(src, prog_w, t_rel, step_rel, i, 0, S);
+  ReleaseFrame f;
+  release_frame(hp, prog_w, g_msat, i, SRC ? S : nullptr, f);
+  const int64_t ridx = rel_idx ? (int64_t)rel_idx[i] : i;
+  double z[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) z[k] = prng_normal(ridx * randint1000(seed, k));
+  const ReleaseScale c(kv, z);
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    double v[4];
+    c.vectors(f, a, v);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out.v[q][i * out.row + a] = v[q];
+  }
+}
+
 static void launch_release(const ssc_host_potential& hp, const ssc_sources& src,
                            const double* prog_w, const int32_t* rel_idx, const double* t_rel,
                            const int32_t* step_rel, const double* g_msat, int nrel, int64_t seed0,
@@ -263,6 +318,12 @@ static void launch_release(const ssc_host_potential& hp, const ssc_sources& src,
     hipLaunchKernelGGL(kernel, dim3((unsigned)bx, (unsigned)by), dim3(256), 0, st, hp, src,
                        prog_w, rel_idx, t_rel, step_rel, g_msat, nrel, seed0, nseed, kv, out);
   };
+  if (nseed == 1 && nrel >= RELEASE_MANY) {
+    auto kernel = src.kind == SSC_SRC_NONE ? release_many_kernel<false> : release_many_kernel<true>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(((int64_t)nrel + 255) / 256)), dim3(256), 0, st, hp,
+                       src, prog_w, rel_idx, t_rel, step_rel, g_msat, nrel, seed0, kv, out);
+    return;
+  }
   // The lanes depend on the source table alone, so that a release's rows are the same bits
   // whatever else its launch holds.
   if (src.kind == SSC_SRC_NONE) go(release_kernel<1>, release_block(1));
