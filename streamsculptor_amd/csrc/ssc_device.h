@@ -165,8 +165,9 @@ inline int group_lanes(int64_t n, int nsrc, bool ragged, int64_t* n_whole = null
 
 // The same for straight-line sources, each of which is first looked up by its window and placed at
 // the time: a source takes about 2.5 times as long and its chain leaves a SIMD idle, so that time
-// does not grow up to about 2.5 waves per SIMD (2 of the halved ones of ragged starts); a wave by
-// itself takes as long.  60 steps (ms), three waves per SIMD wanted / the rule above / this one: 30
+// does not grow up to about 2.5 waves per SIMD (2 of the halved ones of ragged starts), then by 0.8
+// of a wave's time for each one more, and from 5 on in proportion; a wave by itself takes as long
+// as 2.5.  60 steps (ms), three waves per SIMD wanted / the rule above / this one: 30
 // Plummer subhalos, 20,000 orbits 0.157 / 0.187 / 0.149, 40,000 0.202 / 0.304 / 0.202, ragged
 // starts of 130,000 0.210 / 0.298 / 0.20; 200 Hernquist subhalos, 12,000 orbits 0.337 / 0.646 /
 // 0.33, ragged 30,000 0.369 / 0.629 / 0.38.
@@ -178,8 +179,10 @@ inline int group_lanes_line(int64_t n, int nsrc, bool ragged, int64_t* n_whole) 
   double least = 0.0;
   for (int lg = 0; lg <= 4; ++lg) {
     const int64_t g = 1 << lg;
-    const double cost = wave(lg) * (ragged ? std::max(2.0, n * g / 131072.0)
-                                           : std::max(2.5, (double)((n * g + 65535) / 65536)));
+    const double waves = ragged ? n * g / 131072.0 : (double)((n * g + 65535) / 65536);
+    const double cost =
+        wave(lg) * (ragged ? std::max(2.0, waves)
+                           : std::max({2.5, 2.5 + 0.8 * (waves - 2.5), 0.9 * waves}));
     if (lg == 0 || cost < least) { least = cost; best = (int)g; }
   }
   const int64_t rounds = n / 65536, rest = n - rounds * 65536;
