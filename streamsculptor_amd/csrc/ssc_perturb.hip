@@ -234,8 +234,12 @@ __global__ void pt_zero_kernel(double* __restrict__ p, int64_t n) {
 
 // Base orbits in place in w (initialised to w0), rows [ka, kb]: one particle per lane.  A wave's
 // 64 records of a row go through LDS, so that they leave as nine stores of 512 consecutive bytes
-// (80,000 orbits x 4,000 rows 6.3 ms by itself; 7.6 ms written by their own lanes 72 B apart).
+// (80,000 orbits x 4,000 rows 6.3 ms by itself; 7.6 ms written by their own lanes 72 B apart), while
+// there are enough waves for that to be a matter of bandwidth: below 32,768 orbits a row's way
+// through LDS is a part of its chain, and the lanes write their own (60 rows, 50 orbits x 64 sources
+// 0.087 ms against 0.104, 20,000 x 64 0.165 against 0.171).
 constexpr int BASE_LDS = PT_BLOCK * PR_REC * 8;
+constexpr int64_t BASE_DIRECT = 32768;
 
 template <int HS>
 __device__ __forceinline__ void base_rows(const ssc_host_potential& hp, int block, char* lds_raw,
@@ -270,19 +274,27 @@ __device__ __forceinline__ void base_rows(const ssc_host_potential& hp, int bloc
     for (int q = 0; q < 9; ++q) H[q] = 0.0;
     host_quads<HS>(hp, x, y, z, g, H);
     // records of particles that have not started are written and never read
-    double* b = buf + lane * PR_REC;
-    b[0] = x; b[1] = y; b[2] = z;
-    b[3] = H[0]; b[4] = H[1]; b[5] = H[2]; b[6] = H[4]; b[7] = H[5]; b[8] = H[8];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    double* r = rows + ((int64_t)(k - ka) * n + i0) * PR_REC;
+    if (n < BASE_DIRECT) {
+      if (i < n) {
+        double* r = rows + ((int64_t)(k - ka) * n + i) * PR_REC;
+        r[0] = x; r[1] = y; r[2] = z;
+        r[3] = H[0]; r[4] = H[1]; r[5] = H[2]; r[6] = H[4]; r[7] = H[5]; r[8] = H[8];
+      }
+    } else {
+      double* b = buf + lane * PR_REC;
+      b[0] = x; b[1] = y; b[2] = z;
+      b[3] = H[0]; b[4] = H[1]; b[5] = H[2]; b[6] = H[4]; b[7] = H[5]; b[8] = H[8];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      double* r = rows + ((int64_t)(k - ka) * n + i0) * PR_REC;
 #pragma unroll
-    for (int e = 0; e < PR_REC; ++e) {
-      const int o = 64 * e + lane;
-      if (o < tail) r[o] = buf[o];
+      for (int e = 0; e < PR_REC; ++e) {
+        const int o = 64 * e + lane;
+        if (o < tail) r[o] = buf[o];
+      }
+      __builtin_amdgcn_wave_barrier();
     }
-    __builtin_amdgcn_wave_barrier();
     if (on) {
       const double c = (k == s || k == nsteps) ? h : dt;
       vx -= c * g[0]; vy -= c * g[1]; vz -= c * g[2];
