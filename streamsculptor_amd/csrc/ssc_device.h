@@ -256,8 +256,9 @@ __device__ __forceinline__ double group_sum(double v) {
 // (rsq, recip) where the library would expand an IEEE square root or division, and
 // log1p_nonneg -- about one unit in the last place each, and half the instructions of a host
 // force (241 -> 115 per step of the one-lane leapfrog with MN + Hernquist + NFW).  The
-// adaptive kernels keep the IEEE forms (LEAN = false): their step sequences follow the last
-// bits of every force, and parity with the reference's step sequence is stated there.
+// adaptive kernels keep the bits of the IEEE forms (LEAN = false; responses: host_part there): their
+// step sequences follow the last bits of every force, and parity with the reference's step
+// sequence is stated there.
 template <bool LEAN = true>
 __device__ __forceinline__ void parts_mn(const ssc_component& c, double x, double y, double z,
                                          double& f, double& zm) {
@@ -383,11 +384,10 @@ inline int host_signature(const ssc_host_potential& hp) {
 }
 
 // The fixed-step kernels take the LEAN host forms except with STATIC sources (the clumpy
-// halo): there the 512-term source sum is nearly all of a step, so the host forms' cost does
-// not matter, and the IEEE forms keep the plain orbits -- and with them the surrogate's
-// training positions and its measured error -- as they were measured (that error moves with
-// the last bits of the training data: one training seed went from 2.8 to 19.4 pc when the
-// plain orbits changed only there).
+// halo): there the 512-term source sum is nearly all of a step, so shorter host forms bring
+// nothing, while the surrogate's training positions, and with them its measured error, move with
+// the last bits of these orbits (three training seeds: 6.6, 2.8 and 3.1 pc, 5.2, 3.6 and 3.9 with
+// the source sum in another order, and one of them 19.4 with the LEAN forms).
 constexpr bool lean_host(int SK) { return SK != SSC_SRC_STATIC; }
 
 template <int HS, bool LEAN = true>

@@ -2,9 +2,9 @@
 // and adjoint, BF16 MFMA network forward and input-VJP).
 //
 // Forward: the surrogate leapfrog kernel with checkpoint rows (x, v, a) every E grid steps.
-// Backward, segment by segment from the last: a block of 8 waves (two per SIMD, 256 registers
-// each) takes 128 particles, each in the four lanes p + 16 g of its wave like the forward.  Starting from the segment's end checkpoint it
-// walks the leapfrog backwards -- the map is explicitly invertible:
+// Backward, segment by segment from the last: a block of 4 waves (one per SIMD, up to 512
+// registers each) takes 64 particles, each in the four lanes p + 16 g of its wave like the
+// forward.  Starting from the segment's end checkpoint it walks the leapfrog backwards -- the map is explicitly invertible:
 //   vh = v_{k+1} - h a_{k+1};  x_k = x_{k+1} - dt vh;  v_k = vh - h a(x_k)
 // -- so positions are reconstructed in registers instead of being stored, and at every row
 // applies the same adjoint recursion as the plain adjoint kernel:
