@@ -25,10 +25,10 @@
 // bit for bit, which is why divisions, square roots, log1p and pow are the library's or equal to
 // them: shorter forms would take another 40 % off a step.  What bounds a step is instruction
 // latency -- the wave with the halo's log1p, 130 instructions in a chain, at every stage -- with
-// two waves a SIMD in 256 registers.  One particle with 256 response vectors: 16.4 -> 13.5 us a
+// two waves a SIMD in 256 registers.  One particle with 256 response vectors: 16.4 -> 12.9 us a
 // step; 1,000 of them, their responses to 128 Hernquist subhalos with the radius block over
-// 1,500 Myr on average at rtol = atol = 1e-8: 29 -> 24.5 ms; 20,000 particles with 3 vectors
-// over 800 Myr 12.7 -> 8.8 ms.
+// 1,500 Myr on average at rtol = atol = 1e-8: 29 -> 23.6 ms; 20,000 particles with 3 vectors
+// over 800 Myr 12.7 -> 8.6 ms.
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -404,8 +404,6 @@ void perturb_dopri5_kernel(
   bool live = valid && tau0 < tau1;
   int hb = 0, pb = 0;
   const int nc = hp.n_components;
-  // this wave's host components (wide groups): neighbours in the list, so that two waves part disk
-  // + bulge and halo, whose log1p outlasts the others together
   // this wave's host components (wide groups), neighbours in the list: two waves then part disk and
   // bulge from the halo, whose log1p outlasts both (halo and disk on one wave: 4.0 against 3.6 ms
   // for 500 particles x 64 Hernquist subhalos with the radius block, 800 Myr)
