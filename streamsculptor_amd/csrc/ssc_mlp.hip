@@ -27,16 +27,17 @@ namespace mlp {
 // Training kernels.  A minibatch's matrix products are small (8192 x 256 x 256: 1 GFLOP, 12 MB),
 // so an iteration is bound by launches, load latency and how many blocks each launch has.  One
 // launch therefore carries every job whose inputs are ready (ProductJobs, FinishJobs: products,
-// column sums and reductions side by side, a block range each); a product's epilogue applies the activation or
-// its derivative; and a product's tile loads its whole K range (up to TK) into LDS with every
-// load in flight at once.  Operands are kept K-contiguous for all products: activations and
+// column sums and reductions side by side, a block range each); a product's epilogue applies the
+// activation or its derivative; and a product's tile loads its whole K range (up to TK) into LDS
+// with every load in flight at once.  Operands are kept K-contiguous for all products: activations and
 // their gradients are written in both orders by the epilogue that forms them.  Every sum that a
 // gradient goes through keeps its order (K ascending in steps of 16 within a tile, the split-K
 // chunks, the column sums), so a training run gives the same network bit for bit; the loss, which
 // nothing but the caller reads, is added up by tiles of 64 points, and its last bit is not that of
 // sums over 256.  An iteration of 8,192 points (loss, gradients, Adam): 31 launches and 281 us with
-// a kernel per step and a 32-wide K stage, 11 launches and 127 us now; of it 21 us per backward launch (its 20 MB would take 5), 12 us per
-// forward product, 14 us the first layer's gradient (chains of 128 additions, the order's price).
+// a kernel per step and a 32-wide K stage, 11 launches and 127 us now; of it 21 us per backward
+// launch (its 20 MB would take 5), 12 us per forward product, 14 us the first layer's gradient
+// (chains of 128 additions, the order's price).
 //
 // A product: C(m, n) = sum_k A(m, k) B(n, k), A(m, k) = a[m * sa + k * ka] and B likewise, in
 // 64 x 64 tiles by four waves of 32 x 32; K split into chunks of kchunk.
